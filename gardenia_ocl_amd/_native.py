@@ -117,6 +117,15 @@ class DeviceCsr(ctypes.Structure):
                 ("degree", ctypes.c_void_p)]
 
 
+class CsrJob(ctypes.Structure):
+    _fields_ = [("m", ctypes.c_int32), ("nnz", ctypes.c_int64), ("records", ctypes.c_int64),
+                ("keys", ctypes.c_void_p), ("weights", ctypes.c_void_p),
+                ("base", ctypes.c_void_p), ("symmetrize", ctypes.c_int32),
+                ("transpose", ctypes.c_int32), ("sorted", ctypes.c_int32),
+                ("remove_selfloops", ctypes.c_int32), ("remove_redundents", ctypes.c_int32),
+                ("mirror_selfloops", ctypes.c_int32)]
+
+
 class PprPlanConfig(ctypes.Structure):
     _fields_ = [("relabel", ctypes.c_int), ("k_chunk", ctypes.c_int),
                 ("column_stop", ctypes.c_int), ("compact", ctypes.c_int),
@@ -187,6 +196,10 @@ SIGNATURES = {
                              _P]),
     "gd_csr_from_edges_device": (_i, [_i, _i64, _P, _P, _P, _i, _i, _i, _i, _i, _i, _P,
                                       ctypes.POINTER(DeviceCsr)]),
+    "gd_csr_workspace": (_i, [_i, _i64, _i, _i, _i, ctypes.POINTER(ctypes.c_size_t)]),
+    "gd_csr_sort_edges": (_i, [_i, _i64, _P, _P, _P, _i, _i, _i, _i, _i, _i, _P, ctypes.c_size_t,
+                               _P, ctypes.POINTER(CsrJob)]),
+    "gd_csr_finish": (_i, [ctypes.POINTER(CsrJob), _P, _P, _P, _P, _P]),
     "gd_device_csr_copy": (_i, [ctypes.POINTER(DeviceCsr), _P, _P, _P, _P, _P]),
     "gd_device_csr_free": (_i, [ctypes.POINTER(DeviceCsr)]),
     "gd_pr_verify": (_i, [_i, _i64, _P, _P, _P, _P, ctypes.c_float, _P, _F64P]),

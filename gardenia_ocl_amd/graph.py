@@ -117,24 +117,33 @@ def csr_from_edges_device(m: int, src, dst, wt=None, *, symmetrize=False, transp
     n = int(src.shape[0])
     if int(dst.shape[0]) != n or (wt is not None and int(wt.shape[0]) != n):
         raise ValueError("src, dst (and wt) must have the same length")
-    st = stream if stream is not None else torch.cuda.current_stream()
+    cur = torch.cuda.current_stream()
+    st = stream if stream is not None else cur
     sp = ctypes.c_void_p(st.cuda_stream)
-    c = N.DeviceCsr()
-    N.call("gd_csr_from_edges_device", m, n, src.data_ptr(), dst.data_ptr(),
+    dev = src.device
+    size = ctypes.c_size_t()
+    N.call("gd_csr_workspace", m, n, int(wt is not None), int(symmetrize), int(sorted),
+           ctypes.byref(size))
+    # Scratch and results come from torch's caching allocator: repeated builds
+    # reuse the memory.  The scratch belongs to the build's stream; the
+    # results to the caller's, which the build's stream waits for, since the
+    # allocator may hand out memory that work queued there still reads.
+    with torch.cuda.stream(st):
+        ws = torch.empty(max(1, size.value), dtype=torch.uint8, device=dev)
+    job = N.CsrJob()
+    N.call("gd_csr_sort_edges", m, n, src.data_ptr(), dst.data_ptr(),
            None if wt is None else wt.data_ptr(), int(symmetrize), int(transpose), int(sorted),
-           int(remove_selfloops), int(remove_redundents), int(mirror_selfloops), sp, ctypes.byref(c))
-    try:
-        dev = src.device
-        out = {"row_offsets": torch.empty(m + 1, dtype=torch.int32, device=dev),
-               "column_indices": torch.empty(c.nnz, dtype=torch.int32, device=dev),
-               "weight": torch.empty(c.nnz, dtype=torch.float32, device=dev),
-               "degree": torch.empty(m, dtype=torch.int32, device=dev)}
-        N.call("gd_device_csr_copy", ctypes.byref(c), out["row_offsets"].data_ptr(),
-               out["column_indices"].data_ptr(), out["weight"].data_ptr(),
-               out["degree"].data_ptr(), sp)
-        st.synchronize()
-    finally:
-        N.lib().gd_device_csr_free(ctypes.byref(c))
+           int(remove_selfloops), int(remove_redundents), int(mirror_selfloops), ws.data_ptr(),
+           ws.numel(), sp, ctypes.byref(job))
+    out = {"row_offsets": torch.empty(m + 1, dtype=torch.int32, device=dev),
+           "column_indices": torch.empty(job.nnz, dtype=torch.int32, device=dev),
+           "weight": torch.empty(job.nnz, dtype=torch.float32, device=dev),
+           "degree": torch.empty(m, dtype=torch.int32, device=dev)}
+    if st != cur:
+        st.wait_stream(cur)
+    N.call("gd_csr_finish", ctypes.byref(job), out["row_offsets"].data_ptr(),
+           out["column_indices"].data_ptr(), out["weight"].data_ptr(), out["degree"].data_ptr(), sp)
+    st.synchronize()
     return out
 
 

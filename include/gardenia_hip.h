@@ -15,6 +15,7 @@
 #ifndef GARDENIA_HIP_H_
 #define GARDENIA_HIP_H_
 
+#include <stddef.h>
 #include <stdint.h>
 
 #include "gardenia_graph.h"
@@ -169,6 +170,31 @@ int gd_csr_from_edges_device(int m, int64_t n, const int32_t *d_src, const int32
                              const float *d_weight, int symmetrize, int transpose, int sorted,
                              int remove_selfloops, int remove_redundents, int mirror_selfloops,
                              void *stream, gd_device_csr *out);
+/* The same build in memory of the caller's, for programs that build graphs
+ * repeatedly: gd_csr_workspace gives the scratch bytes, gd_csr_sort_edges
+ * sorts the records there and sets job->nnz (synchronises stream), and
+ * gd_csr_finish writes the CSR into arrays of m+1, nnz, nnz and m entries
+ * (d_weight may be NULL) on stream.  The workspace (256-byte aligned) must
+ * stay as it is between the two calls and until the second one's work has
+ * run. */
+typedef struct gd_csr_job {
+  int32_t m;
+  int64_t nnz; /* edges of the CSR */
+  /* the library's: where the sorted records lie, and the flags */
+  int64_t records;
+  void *keys, *weights, *base;
+  int32_t symmetrize, transpose, sorted, remove_selfloops, remove_redundents, mirror_selfloops;
+} gd_csr_job;
+
+int gd_csr_workspace(int m, int64_t n, int have_weight, int symmetrize, int sorted,
+                     size_t *bytes);
+int gd_csr_sort_edges(int m, int64_t n, const int32_t *d_src, const int32_t *d_dst,
+                      const float *d_weight, int symmetrize, int transpose, int sorted,
+                      int remove_selfloops, int remove_redundents, int mirror_selfloops,
+                      void *d_workspace, size_t workspace_bytes, void *stream, gd_csr_job *job);
+int gd_csr_finish(const gd_csr_job *job, int32_t *d_row_offsets, int32_t *d_column_indices,
+                  float *d_weight, int32_t *d_degree, void *stream);
+
 /* Device-to-device copies into caller arrays (any may be NULL), on stream. */
 int gd_device_csr_copy(const gd_device_csr *c, int32_t *d_row_offsets, int32_t *d_column_indices,
                        float *d_weight, int32_t *d_degree, void *stream);
