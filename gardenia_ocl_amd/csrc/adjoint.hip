@@ -40,6 +40,8 @@ struct WGather {
   const float* __restrict__ w;  // per-edge weight, in the order of the pulled CSR
   const float* __restrict__ c;  // gathered vector
   __device__ __forceinline__ float value(int e, int u) const { return w[e] * c[u]; }
+  __device__ __forceinline__ const float* source() const { return c; }
+  __device__ __forceinline__ void from(const float* v) { c = v; }
 };
 
 // forward: x_v = base + d * sum_u a_uv c_u,  c_v = x_v / s_v

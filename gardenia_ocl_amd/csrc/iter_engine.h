@@ -25,6 +25,10 @@ struct wide_tiles : std::false_type {};
 template <class P>
 struct wide_tiles<P, std::void_t<decltype(P::kWideTiles)>> : std::bool_constant<P::kWideTiles> {};
 
+// Windowed gathers above this many sources: 4 MB of them, one XCD's L2, which
+// serves a smaller vector's gathers by itself.
+constexpr int kWindowMin = 1 << 20;
+
 struct IterEngine {
   int m = 0;
   int64_t nnz = 0;
@@ -36,6 +40,10 @@ struct IterEngine {
   bool persistent = true;
   int exact_len = 0;         // > 0: rows longer than this are whole-row exact hub tiles
   bool sort_tiles = false;   // gather each tile's edges in source order (tile_sort.h)
+  // Windowed gather (window_gather.h) where the gathered vector exceeds an
+  // XCD's L2; sorted tiles and exact hubs only.
+  bool windows = false;
+  WindowGather win;
   int32_t* col_owned = nullptr;  // the caller's private copy of col: sorted in place
   int pull_grid = 0;
   const int32_t* off = nullptr;
@@ -128,9 +136,14 @@ struct IterEngine {
         if (rc) return rc;
         dst = col_sorted.as<int32_t>();
       }
-      // exact hub rows are kept in edge order
+      // exact hub rows are kept in edge order, or sorted in staging blocks
+      const int64_t segs = (int64_t)sched.tiles.size() + nnz / kScanChunk + sched.n_slots;
+      const bool win_on = windows && exact_len > 0 && stage_hubs != 0 && !persistent && m > kWindowMin &&
+                          window_gather_fits(m, nnz, segs);
+      std::vector<int2> seg;
       rc = build_tile_sort(sched, block * ipt, col, dst, pos.as<uint16_t>(), stream,
-                           exact_len > 0);
+                           exact_len > 0, win_on ? kScanChunk : 0, &seg);
+      if (!rc && win_on) rc = build_window_gather(m, nnz, seg, dst, stream, &win);
       if (rc) return rc;
       col = dst;
     }
@@ -151,7 +164,7 @@ struct IterEngine {
       int64_t hub_edges = 0;
       for (const Tile& t : hubs) hub_edges += t.w - t.z;
       const int64_t longest = hubs[0].w - hubs[0].z;
-      const bool want = stage_hubs == 1 ||
+      const bool want = stage_hubs == 1 || win.on() ||
                         (stage_hubs < 0 && longest * 500 > (int64_t)nnz - hub_edges);
       std::vector<int32_t> soff(n_hub_tiles, -1);
       std::vector<int4> blocks;
@@ -238,7 +251,8 @@ struct IterEngine {
                     n_tiles > 0 ? pull_grid : 0, off, col, e_max, pos.as<uint16_t>(),
                     hub_part.as<float>(), err_part.as<double>(), state.as<IterState>(),
                     fused ? parts : 0, errors.as<double>(),
-                    staged ? hub_soff.as<int32_t>() : nullptr, stage.as<float>()};
+                    staged ? hub_soff.as<int32_t>() : nullptr, stage.as<float>(),
+                    win.on() ? win.stage.as<float>() : nullptr};
   }
 
   // exact hubs finish their rows in the pull launch: no hub epilogues here
@@ -278,9 +292,16 @@ struct IterEngine {
     // staged hubs: their values are gathered first, by the whole GPU, before
     // the fork (the row tiles would otherwise fill the CUs first and hold the
     // hub rows back until they drain)
-    if (staged)
-      hipLaunchKernelGGL((hub_stage_kernel<P, NT>), dim3(n_stage_blocks), dim3(kBlock), 0, stream,
-                         a, it, stage_blocks.as<int4>(), stage.as<float>());
+    if (win.on())
+      hipLaunchKernelGGL(window_expand_kernel<P>, dim3(win.n_pieces), dim3(kExpandBlock), 0, stream,
+                         a, it, win.n_src, win.pieces.as<int4>(), win.sid.as<uint16_t>(),
+                         win.stage.as<float>());
+    if (staged && win.on())
+      hipLaunchKernelGGL((hub_stage_kernel<P, NT, true>), dim3(n_stage_blocks), dim3(kBlock), 0,
+                         stream, a, it, stage_blocks.as<int4>(), stage.as<float>());
+    else if (staged)
+      hipLaunchKernelGGL((hub_stage_kernel<P, NT, false>), dim3(n_stage_blocks), dim3(kBlock), 0,
+                         stream, a, it, stage_blocks.as<int4>(), stage.as<float>());
     hipStream_t ts = stream;
     if (fork) {
       (void)hipEventRecord(fork_ev, stream);

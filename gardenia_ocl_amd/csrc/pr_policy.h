@@ -13,6 +13,8 @@ namespace gd {
 struct PrGather {
   const float* __restrict__ contrib;
   __device__ __forceinline__ float value(int /*e*/, int u) const { return contrib[u]; }
+  __device__ __forceinline__ const float* source() const { return contrib; }
+  __device__ __forceinline__ void from(const float* v) { contrib = v; }
 };
 
 // NT: 0 plain, 1 streamed arrays non-temporal, 2 also the new contrib

@@ -32,6 +32,7 @@
 
 #include "gd_common.h"
 #include "pull_engine.h"
+#include "window_gather.h"
 
 namespace gd {
 
@@ -66,7 +67,20 @@ struct IterArgs {
   // at stage[hub_soff[h]...]; nullptr when the plan does not stage
   const int32_t* __restrict__ hub_soff;
   const float* __restrict__ stage;
+  // windowed plans: the values expanded by window_expand_kernel; `col` holds
+  // each edge's slot in it (nullptr: `col` holds sources)
+  const float* __restrict__ slots;
 };
+
+// The gather of policy P: from the iteration's source vector, or from the
+// expanded slots of a windowed plan.
+template <class P, int NT>
+__device__ __forceinline__ auto iter_gather(const typename P::Args& a, const IterArgs& it,
+                                            int odd) {
+  auto g = P::template gather<NT>(a, odd);
+  if (it.slots) g.from(it.slots);
+  return g;
+}
 
 // Values of a staged hub row: the row's first edge e0 is stage[0].
 struct StagedGather {
@@ -141,7 +155,7 @@ __device__ __forceinline__ void tile_body(const typename P::Args& a, const IterA
   const int odd = it.st->iter & 1;
   __shared__ double s_err[NB / kWave];
   const Tile t = it.tiles[b];
-  const auto g = P::template gather<NT>(a, odd);
+  const auto g = iter_gather<P, NT>(a, it, odd);
   double err = 0.0;
   if (t.y >= 0) {
     const auto e = P::template epilogue<NT>(a, odd);
@@ -166,7 +180,8 @@ __global__ __launch_bounds__(NB) void pull_tile_kernel(const typename P::Args a,
                                                        const IterArgs it) {
   if (it.st->done) return;
   __shared__ RowTileLds<IPT, NB> lds;
-  tile_body<P, IPT, NT, SORTED, NB>(a, it, blockIdx.x, lds);
+  const int b = it.slots ? xcd_run_block(blockIdx.x, gridDim.x) : (int)blockIdx.x;
+  tile_body<P, IPT, NT, SORTED, NB>(a, it, b, lds);
 }
 
 // Persistent, software-pipelined form: workgroup b walks tiles b, b+G, ...;
@@ -270,26 +285,50 @@ __device__ __forceinline__ void hub_body(const typename P::Args& a, const IterAr
 // exact_hub_kernel (same stream): the hub kernel then scans values read
 // coalesced from L2 instead of waiting on each chunk's random gathers, so a
 // long row's workgroup is bound by its scan.  Workgroup b gathers block b:
-// x = first edge, y = edges (<= kScanChunk), z = offset in stage.
-template <class P, int NT>
+// x = first edge, y = edges (<= kScanChunk), z = offset in stage.  PERM
+// (windowed plans): a block's edges are sorted by source; the values go back
+// to edge order through LDS.
+template <class P, int NT, bool PERM>
 __global__ __launch_bounds__(kBlock) void hub_stage_kernel(const typename P::Args a,
                                                            const IterArgs it,
                                                            const int4* __restrict__ blocks,
                                                            float* __restrict__ stage) {
   if (it.st->done) return;
-  const int4 b = blocks[blockIdx.x];
-  const auto g = P::template gather<NT>(a, it.st->iter & 1);
-  int idx[kScanPT];
+  const int4 b = blocks[PERM ? xcd_run_block(blockIdx.x, gridDim.x) : (int)blockIdx.x];
+  const auto g = iter_gather<P, NT>(a, it, it.st->iter & 1);
+  int idx[kScanPT], p[kScanPT];
   float v[kScanPT];
 #pragma unroll
   for (int j = 0; j < kScanPT; j++)
     idx[j] = ld_stream<(NT > 0)>(it.col + b.x + min((int)threadIdx.x + j * kBlock, b.y - 1));
+  if constexpr (PERM) load_positions<kScanPT, (NT > 0)>(it.pos, b.x, b.y, p);
 #pragma unroll
   for (int j = 0; j < kScanPT; j++)
-    v[j] = g.value(b.x + min((int)threadIdx.x + j * kBlock, b.y - 1), idx[j]);
+    v[j] = g.value(b.x + (PERM ? p[j] : min((int)threadIdx.x + j * kBlock, b.y - 1)), idx[j]);
+  if constexpr (PERM) {
+    __shared__ float s_v[kScanChunk];
+#pragma unroll
+    for (int j = 0; j < kScanPT; j++)
+      if ((int)threadIdx.x + j * kBlock < b.y) s_v[p[j]] = v[j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kScanPT; j++) v[j] = s_v[min((int)threadIdx.x + j * kBlock, b.y - 1)];
+  }
 #pragma unroll
   for (int j = 0; j < kScanPT; j++)
     if ((int)threadIdx.x + j * kBlock < b.y) stage[b.z + threadIdx.x + j * kBlock] = v[j];
+}
+
+// Pass 1 of a windowed gather (window_gather.h): one piece of a window's
+// slots per workgroup.
+template <class P>
+__global__ __launch_bounds__(kExpandBlock) void window_expand_kernel(
+    const typename P::Args a, const IterArgs it, int n_src, const int4* __restrict__ pieces,
+    const uint16_t* __restrict__ sid, float* __restrict__ slots) {
+  if (it.st->done) return;
+  __shared__ float win[kWinSize];
+  const auto g = P::template gather<0>(a, it.st->iter & 1);
+  window_expand(g.source(), n_src, pieces[blockIdx.x], sid, slots, win);
 }
 
 // Held to 3 waves per SIMD (<= 168 VGPRs): the hub workgroups share the CUs

@@ -13,6 +13,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <vector>
+
 #include "gd_common.h"
 
 namespace gd {
@@ -26,9 +28,12 @@ constexpr int kSortMax = 16384;  // longest sorted segment (one workgroup's LDS 
 // offset in the segment.  col and col_sorted may be the same array.
 // exact_hubs (a schedule built with exact_len > 0, whose hub tiles are whole
 // rows): hub rows stay in edge order (col_sorted = col and pos = offset
-// there).
+// there) unless hub_chunk > 0: then they are sorted in chunks of hub_chunk
+// edges, too.  segs (may be NULL) receives the sorted segments (x: first edge,
+// y: edges; < 0 where they stay in edge order), row tiles first.
 int build_tile_sort(const Schedule& s, int chunk, const int32_t* d_col, int32_t* d_col_sorted,
-                    uint16_t* d_pos, hipStream_t stream, bool exact_hubs = false);
+                    uint16_t* d_pos, hipStream_t stream, bool exact_hubs = false,
+                    int hub_chunk = 0, std::vector<int2>* segs = nullptr);
 
 }  // namespace gd
 

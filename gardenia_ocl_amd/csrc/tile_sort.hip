@@ -59,16 +59,18 @@ __global__ __launch_bounds__(BS) void segment_sort_kernel(const int2* __restrict
 }  // namespace
 
 int build_tile_sort(const Schedule& s, int chunk, const int32_t* d_col, int32_t* d_col_sorted,
-                    uint16_t* d_pos, hipStream_t stream, bool exact_hubs) {
-  if (chunk <= 0 || chunk > kSortMax) {
+                    uint16_t* d_pos, hipStream_t stream, bool exact_hubs, int hub_chunk,
+                    std::vector<int2>* segs_out) {
+  if (chunk <= 0 || chunk > kSortMax || hub_chunk < 0 || hub_chunk > kSortMax) {
     set_error("build_tile_sort: chunk must be in [1, 16384]");
     return GD_ERR_INVALID;
   }
   std::vector<int2> segs;
   segs.reserve(s.tiles.size() + 16);
-  for (const Tile& t : s.tiles) {
-    const bool keep = exact_hubs && t.y < 0;  // whole-row exact hubs stay in edge order
-    const int seg = chunk;
+  auto cut = [&](const Tile& t) {
+    // whole-row exact hubs stay in edge order or have chunks of their own
+    const bool hub = exact_hubs && t.y < 0, keep = hub && hub_chunk == 0;
+    const int seg = hub && hub_chunk > 0 ? hub_chunk : chunk;
     for (int32_t e = t.z; e < t.w; e += seg) {
       const int32_t n = std::min(seg, t.w - e);
       if (n > kSortMax) {
@@ -77,7 +79,14 @@ int build_tile_sort(const Schedule& s, int chunk, const int32_t* d_col, int32_t*
       }
       segs.push_back(make_int2(e, keep ? -n : n));
     }
-  }
+    return GD_OK;
+  };
+  for (int hubs = 0; hubs < 2; hubs++)  // row tiles first
+    for (const Tile& t : s.tiles)
+      if ((t.y < 0) == (hubs == 1)) {
+        const int rc = cut(t);
+        if (rc) return rc;
+      }
   if (segs.empty()) return GD_OK;
   DeviceBuffer d_segs;
   int rc = d_segs.alloc(sizeof(int2) * segs.size());
@@ -86,10 +95,11 @@ int build_tile_sort(const Schedule& s, int chunk, const int32_t* d_col, int32_t*
                             hipMemcpyHostToDevice, stream));
   static_assert(1024 * kSortIPT == kSortMax, "the widest sort covers kSortMax edges");
   const dim3 grid((unsigned)segs.size());
-  if (chunk > 8192)
+  const int widest = std::max(chunk, hub_chunk);
+  if (widest > 8192)
     hipLaunchKernelGGL(segment_sort_kernel<1024>, grid, dim3(1024), 0, stream, d_segs.as<int2>(),
                        d_col, d_col_sorted, d_pos);
-  else if (chunk > 4096)
+  else if (widest > 4096)
     hipLaunchKernelGGL(segment_sort_kernel<512>, grid, dim3(512), 0, stream, d_segs.as<int2>(),
                        d_col, d_col_sorted, d_pos);
   else
@@ -97,6 +107,7 @@ int build_tile_sort(const Schedule& s, int chunk, const int32_t* d_col, int32_t*
                        d_col, d_col_sorted, d_pos);
   GD_HIP_TRY(hipGetLastError());
   GD_HIP_TRY(hipStreamSynchronize(stream));  // d_segs is freed on return
+  if (segs_out) *segs_out = std::move(segs);
   return GD_OK;
 }
 

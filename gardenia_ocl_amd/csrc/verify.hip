@@ -31,6 +31,8 @@ namespace {
 struct VerifyGather {
   const float* __restrict__ contrib;
   __device__ __forceinline__ float value(int /*e*/, int u) const { return contrib[u]; }
+  __device__ __forceinline__ const float* source() const { return contrib; }
+  __device__ __forceinline__ void from(const float* v) { contrib = v; }
 };
 
 struct VerifyEpilogue {
