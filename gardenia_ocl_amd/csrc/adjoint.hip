@@ -52,6 +52,7 @@ struct WprEpilogue {
   const float* __restrict__ s;
   float base;
   float damp;
+  static constexpr bool kWaveRows = true;  // edge weights and scores are not negative in earnest
   struct Pre {
     float old;
     float s;

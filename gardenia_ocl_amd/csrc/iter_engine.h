@@ -176,7 +176,7 @@ struct IterEngine {
         for (int o = 0; o < ne; o += kScanChunk)
           blocks.push_back(make_int4(hubs[h].z + o, std::min(kScanChunk, ne - o),
                                      (int)(staged + o), 0));
-        staged += ne;
+        staged += (ne + 3) & ~3;  // rows start 16-byte aligned
       }
       n_stage_blocks = (int)blocks.size();
       if (n_stage_blocks) {

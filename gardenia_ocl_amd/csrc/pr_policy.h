@@ -26,6 +26,7 @@ struct PrEpilogue {
   float base;
   float damp;
   int seed;
+  static constexpr bool kWaveRows = true;  // scores are never negative
   struct Pre {
     float old;
     int deg;

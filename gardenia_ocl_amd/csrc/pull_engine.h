@@ -21,6 +21,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "gd_common.h"
 
 namespace gd {
@@ -148,6 +150,350 @@ __device__ __forceinline__ float seq_sum(float s, const float* __restrict__ v, i
   return s;
 }
 
+// ---------------------------------------------------------------------------
+// Sequential-order sums of long rows in parallel.
+//
+// wave_exact_seg / exact_row_sum return s0 + v[0] + v[1] + ... + v[n-1]
+// rounded exactly as the sequential FP32 loop `s = s0; for (i) s += v[i];`
+// rounds it (the reference's per-row loop, src/pr/omp_base.cc:34-37):
+//   While the running sum s > 0 lies in one binade [B, 2B) and no term is
+//   negative, a step s + v advances s by a whole number of ulps that depends
+//   on v and, through ties (round to even), on the parity of s alone.  So a
+//   lane adds its terms in FP32 twice, from B and from B + ulp; the two
+//   advances are its map of the running value (Steps), the hardware having
+//   rounded every step.  Maps compose into maps of the same form, and a
+//   prefix over the lanes' maps gives the running value after every lane's
+//   terms; where no lane's advance depends on the parity (most wavefronts of
+//   a long row) it is a prefix of integers.
+//   The running values never decrease, so the binade holds up to a lane
+//   exactly when the value after that lane is below 2B.  The first lane past
+//   it, or one with a negative term, adds its terms from the running value
+//   itself, and the prefix restarts after it in the new binade.  inf and NaN
+//   terms carry a lane past any binade.  A zero s skips to the first nonzero
+//   term; a subnormal, negative or non-finite s takes a lane's terms as they
+//   are.
+// For sums of positive terms (PageRank) the restarts are the ~log2(n) binade
+// crossings.  A pass over 16 terms a lane is 32 FP32 additions and the prefix
+// (about 0.3 us per 1024 terms); one lane's dependent chain costs about 3 ns
+// per term, and the form before this one, which rounded each term to ulps in
+// integers and checked every running value, about 1,230 vector instructions
+// a pass: the 48,023-edge hub of a 1 M-vertex RMAT graph took 67 us of a
+// staged 84-us iteration.
+// ---------------------------------------------------------------------------
+
+constexpr int kScanPT = 16;                   // terms per thread per chunk
+constexpr int kScanChunk = kBlock * kScanPT;  // 4096
+constexpr uint32_t kBinade = 1u << 23;        // ulps from a binade's start to its end
+
+// A run of steps as one map of the running value x, in ulps: x -> x + a0 for
+// even x, x + a1 for odd x.
+struct Steps {
+  uint32_t a0, a1;
+};
+
+__device__ __forceinline__ Steps compose(Steps p, Steps q) {  // p, then q
+  const uint32_t d = q.a0 ^ q.a1;  // selects without branches: q.a1 = q.a0 ^ d
+  return Steps{p.a0 + (q.a0 ^ (d & (0u - (p.a0 & 1u)))), p.a1 + (q.a1 ^ (d & (0u - (p.a1 & 1u))))};
+}
+__device__ __forceinline__ uint32_t apply(Steps p, uint32_t x) {
+  return x + (p.a0 ^ ((p.a0 ^ p.a1) & (0u - (x & 1u))));
+}
+
+// Inclusive prefixes over the 64 lanes of a wavefront: DPP row shifts inside
+// each row of 16 lanes, then row broadcasts across rows (lanes whose source
+// is outside the row read 0, the identity).
+#define GD_DPP(V, CTRL, ROWS) \
+  (uint32_t) __builtin_amdgcn_update_dpp(0, (int)(V), CTRL, ROWS, 0xf, false)
+#define GD_SCAN_STEPS(STEP)                                                              \
+  STEP(0x111, 0xf) STEP(0x112, 0xf) STEP(0x114, 0xf) STEP(0x118, 0xf) /* row_shr:1,2,4,8 */ \
+  STEP(0x142, 0xa) STEP(0x143, 0xc) /* row_bcast:15 -> rows 1, 3; row_bcast:31 -> rows 2, 3 */
+
+__device__ __forceinline__ uint32_t wave_incl_scan_add(uint32_t x) {
+#define GD_STEP(CTRL, ROWS) x += GD_DPP(x, CTRL, ROWS);
+  GD_SCAN_STEPS(GD_STEP)
+#undef GD_STEP
+  return x;
+}
+
+__device__ __forceinline__ Steps wave_incl_scan_steps(Steps x) {
+#define GD_STEP(CTRL, ROWS) x = compose(Steps{GD_DPP(x.a0, CTRL, ROWS), GD_DPP(x.a1, CTRL, ROWS)}, x);
+  GD_SCAN_STEPS(GD_STEP)
+#undef GD_STEP
+  return x;
+}
+#undef GD_SCAN_STEPS
+#undef GD_DPP
+
+// Wavefront-uniform values kept in scalar registers.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ float uniform(float v) {
+  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+__device__ __forceinline__ uint32_t read_lane(uint32_t v, int lane) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
+}
+
+// s > 0 is a normal number; its binade starts at binade(s), and it lies
+// ulps(s) >= 2^23 ulps above zero.  Inside one binade the bits of a float
+// count ulps.
+__device__ __forceinline__ bool in_binade(float s) {
+  const uint32_t b = __float_as_uint(s);
+  return b >= kBinade && b < 0x7f800000u;
+}
+__device__ __forceinline__ uint32_t binade(float s) { return __float_as_uint(s) & 0x7f800000u; }
+
+// Some term of the lane has its sign bit set.
+template <int K>
+__device__ __forceinline__ bool lane_negative(const float (&v)[K]) {
+  uint32_t b = 0u;
+#pragma unroll
+  for (int k = 0; k < K; k++) b |= __float_as_uint(v[k]);
+  return b >> 31;
+}
+
+// The inclusive prefix of the wavefront's maps in the binade that starts at
+// the float bits `base`.  Inactive lanes are identities.  `stop`: the lane is
+// negative or leaves a binade by itself; such a lane counts as a binade, so
+// lanes before the first stop see sums below 2^30.
+template <int K>
+__device__ __forceinline__ Steps wave_steps(const float (&v)[K], bool active, bool negative,
+                                            uint32_t base, bool& stop) {
+  float x0 = __uint_as_float(base), x1 = __uint_as_float(base + 1u);
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    x0 += v[k];
+    x1 += v[k];
+  }
+  Steps L{__float_as_uint(x0) - base, __float_as_uint(x1) - (base + 1u)};
+  stop = negative || L.a0 >= kBinade - 1u || L.a1 >= kBinade - 1u;
+  if (stop) L = Steps{kBinade, kBinade};
+  if (!active) L = Steps{0u, 0u};
+  stop = stop && active;
+  if (__ballot(L.a0 != L.a1)) return wave_incl_scan_steps(L);
+  const uint32_t a = wave_incl_scan_add(L.a0);
+  return Steps{a, a};
+}
+
+// s + the wavefront's terms in lane order (lane l: v[0..K-1] are terms l*K ..
+// l*K+K-1; missing terms 0), rounded as the sequential loop.  The whole
+// wavefront calls it with one s; every pass finishes a lane, so it ends.
+template <int K>
+__device__ __forceinline__ float wave_exact_seg(float s, const float (&v)[K]) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const bool negative = lane_negative<K>(v);
+  // terms of both signs: a lane at a time from the start
+  const bool mixed = __popcll(__ballot(negative)) > 4;
+  int from = 0;  // lanes before it are added
+  s = uniform(s);
+  for (;;) {
+    int f = from;
+    if (in_binade(s) && !mixed) {
+      const uint32_t base = binade(s), at = __float_as_uint(s) - base;
+      bool stop;
+      const Steps inc = wave_steps<K>(v, lane >= from, negative, base, stop);
+      const uint32_t r = apply(inc, at);
+      const uint64_t m = __ballot(stop || r >= kBinade);
+      if (!m) return __uint_as_float(base + read_lane(r, kWave - 1));
+      f = __builtin_ctzll(m);
+      if (f > 0) s = __uint_as_float(base + read_lane(r, f - 1));
+    } else if (__float_as_uint(s) == 0u) {
+      uint32_t any = 0u;
+#pragma unroll
+      for (int k = 0; k < K; k++) any |= __float_as_uint(v[k]) << 1;
+      const uint64_t m = __ballot(lane >= from && any != 0u);
+      if (!m) return s;
+      f = __builtin_ctzll(m);
+    }
+    float t = s;  // lane f's terms from s (every lane computes its own)
+#pragma unroll
+    for (int k = 0; k < K; k++) t += v[k];
+    s = __uint_as_float(read_lane(__float_as_uint(t), f));
+    from = f + 1;
+    if (from >= kWave) return s;
+  }
+}
+
+// The whole row v[b, e) of LDS (`v` 16-byte aligned) by one wavefront: the
+// first terms, where s crosses a binade every few terms, as a plain chain,
+// then 256 terms a pass, then 1024.
+constexpr int kRowHead = 64;
+
+template <int K>
+__device__ __forceinline__ void wave_terms(const float* __restrict__ v, int i, int e,
+                                           float (&t)[K]) {
+  const int at = i + (threadIdx.x & (kWave - 1)) * K;
+#pragma unroll
+  for (int k = 0; k < K; k += 4) {
+    const float4 x = *reinterpret_cast<const float4*>(v + (at + k < e ? at + k : i));
+    t[k] = at + k < e ? x.x : 0.0f;
+    t[k + 1] = at + k + 1 < e ? x.y : 0.0f;
+    t[k + 2] = at + k + 2 < e ? x.z : 0.0f;
+    t[k + 3] = at + k + 3 < e ? x.w : 0.0f;
+  }
+}
+
+__device__ __forceinline__ float wave_exact_row(float s, const float* __restrict__ v, int b, int e) {
+  int i = min(e, (b + kRowHead) & ~3);
+  s = seq_sum(s, v, b, i);
+  while (i < e && (i < b + 512 || e - i <= 512)) {
+    float t[4];
+    wave_terms<4>(v, i, e, t);
+    s = wave_exact_seg<4>(s, t);
+    i += 4 * kWave;
+  }
+  while (i < e) {
+    float t[kScanPT];
+    wave_terms<kScanPT>(v, i, e, t);
+    s = wave_exact_seg<kScanPT>(s, t);
+    i += kScanPT * kWave;
+  }
+  return s;
+}
+
+struct ExactLds {
+  Steps tot[2][kWaves];  // wave totals of the maps, by pass parity
+  int stop[2][kWaves];   // the wave has a stop of its own
+  float s[2];
+};
+
+// s + one chunk of the row, thread t's terms being its 16t .. 16t+15 (v,
+// missing terms 0).  The waves' totals in s's binade are combined in order;
+// a wave in which the binade ends (or that holds a negative term) adds its
+// terms by itself, and the waves after it go on in the new binade.  Every
+// pass finishes a wave.  `pass` counts the workgroup's passes (the parity of
+// the buffers: one barrier apart, a buffer is written again two passes later).
+__device__ __forceinline__ float exact_scan_chunk(const float (&v)[kScanPT], float s, int& pass,
+                                                  ExactLds& x) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wid = uniform((int)(threadIdx.x / kWave));
+  const bool negative = lane_negative<kScanPT>(v);
+  int fw = 0;  // waves before it are added
+  s = uniform(s);
+  while (fw < kWaves) {
+    int w = fw;
+    if (in_binade(s)) {
+      const uint32_t base = binade(s);
+      const int p = pass & 1;
+      pass++;
+      if (wid >= fw) {
+        bool stop;
+        const Steps inc = wave_steps<kScanPT>(v, true, negative, base, stop);
+        const int any = __ballot(stop) != 0;
+        if (lane == kWave - 1) {
+          x.tot[p][wid] = inc;
+          x.stop[p][wid] = any;
+        }
+      }
+      __syncthreads();
+      uint32_t at = __float_as_uint(s) - base;
+      for (; w < kWaves; w++) {
+        const uint32_t r = apply(x.tot[p][w], at);
+        if (uniform((int)(x.stop[p][w] || r >= kBinade))) break;
+        at = r;
+      }
+      s = uniform(__uint_as_float(base + at));
+    }
+    if (w < kWaves) {
+      const int p = pass & 1;
+      pass++;
+      if (wid == w) {
+        const float t = wave_exact_seg<kScanPT>(s, v);
+        if (lane == 0) x.s[p] = t;
+      }
+      __syncthreads();
+      s = uniform(x.s[p]);
+      w++;
+    }
+    fw = w;
+  }
+  return s;
+}
+
+// s0 + the gathered values of edges [e0, e0+ne) in edge order, rounded as the
+// sequential FP32 loop starting from s0 (all threads return it).  `buf`: a
+// 16-byte aligned LDS buffer of kScanChunk floats.  Chunk c is gathered as
+// thread t's terms t + 256 j (coalesced index loads), stored at their
+// position in the chunk, and scanned as thread t's terms 16t..16t+15; chunk
+// c+1's gathers and chunk c+2's index loads are in flight meanwhile.  (Every
+// scan has a barrier after all threads have read their terms, so one buffer
+// serves every chunk.)
+// STAGED: the row's values were gathered beforehand into a 16-byte aligned
+// buffer (g.s, padded to a multiple of 4): each thread loads its terms from
+// there, the next chunk's in flight, and no LDS is needed for them.
+template <bool NT, class G, bool STAGED = false>
+__device__ float exact_row_sum(const int32_t* __restrict__ col, int e_max, int e0, int ne,
+                               const G& g, float s0, float* __restrict__ buf, ExactLds& x) {
+  const int tid = threadIdx.x;
+  const int nchunks = (ne + kScanChunk - 1) / kScanChunk;
+  float s = s0;
+  int pass = 0;
+  if (nchunks == 0) return s;
+  if constexpr (STAGED) {
+    float4 nx[kScanPT / 4];
+    auto load = [&](int c) {
+      const int at = c * kScanChunk + tid * kScanPT;
+#pragma unroll
+      for (int k = 0; k < kScanPT / 4; k++)
+        nx[k] = *reinterpret_cast<const float4*>(g.s + (at + 4 * k < ne ? at + 4 * k : 0));
+    };
+    load(0);
+    for (int c = 0; c < nchunks; c++) {
+      const int at = c * kScanChunk + tid * kScanPT;
+      float v[kScanPT];
+#pragma unroll
+      for (int k = 0; k < kScanPT / 4; k++) {
+        v[4 * k] = at + 4 * k < ne ? nx[k].x : 0.0f;
+        v[4 * k + 1] = at + 4 * k + 1 < ne ? nx[k].y : 0.0f;
+        v[4 * k + 2] = at + 4 * k + 2 < ne ? nx[k].z : 0.0f;
+        v[4 * k + 3] = at + 4 * k + 3 < ne ? nx[k].w : 0.0f;
+      }
+      if (c + 1 < nchunks) load(c + 1);
+      s = exact_scan_chunk(v, s, pass, x);
+    }
+    return s;
+  } else {
+    int idx[kScanPT];
+    float vv[kScanPT];
+    auto elem = [&](int c, int j) {  // edge offset in the row, clamped into it
+      return min(c * kScanChunk + tid + j * kBlock, ne - 1);
+    };
+    auto load_idx = [&](int c) {
+#pragma unroll
+      for (int j = 0; j < kScanPT; j++)
+        idx[j] = ld_stream<NT>(col + min(e0 + elem(c, j), e_max));
+    };
+    auto gather = [&](int c) {
+#pragma unroll
+      for (int j = 0; j < kScanPT; j++) vv[j] = g.value(e0 + elem(c, j), idx[j]);
+    };
+    load_idx(0);
+    gather(0);
+    if (nchunks > 1) load_idx(1);
+    for (int c = 0; c < nchunks; c++) {
+#pragma unroll
+      for (int j = 0; j < kScanPT; j++)
+        buf[tid + j * kBlock] = c * kScanChunk + tid + j * kBlock < ne ? vv[j] : 0.0f;
+      if (c + 1 < nchunks) {
+        gather(c + 1);                         // in flight during the scan of chunk c
+        if (c + 2 < nchunks) load_idx(c + 2);  // likewise
+      }
+      __syncthreads();
+      float v[kScanPT];
+      const float4* v4 = reinterpret_cast<const float4*>(buf + tid * kScanPT);
+#pragma unroll
+      for (int k = 0; k < kScanPT / 4; k++) {
+        const float4 t = v4[k];
+        v[4 * k] = t.x;
+        v[4 * k + 1] = t.y;
+        v[4 * k + 2] = t.z;
+        v[4 * k + 3] = t.w;
+      }
+      s = exact_scan_chunk(v, s, pass, x);
+    }
+    return s;
+  }
+}
+
 // Loads the tile's edge indices col[e0 + tid + j*kBlock] (clamped into the
 // tile so all IPT loads issue back to back).  Requires ne >= 1.
 template <int IPT, bool NT, int NB = kBlock>
@@ -197,12 +543,25 @@ __device__ __forceinline__ float segment_sum(const int32_t* __restrict__ col,
   return block_sum<kWaves>(s, s_tmp);
 }
 
+// Rows of a tile longer than this are added by a wavefront (wave_exact_row)
+// where the epilogue's terms are never negative (E::kWaveRows); shorter ones
+// by their owner threads, side by side, which lasts as long as the longest.
+constexpr int kWaveRow = 512;
+
+template <class E, class = void>
+struct wave_rows : std::false_type {};
+template <class E>
+struct wave_rows<E, std::void_t<decltype(E::kWaveRows)>> : std::bool_constant<E::kWaveRows> {};
+
 // LDS of one row tile of a workgroup of NB threads.
 template <int IPT, int NB = kBlock>
 struct RowTileLds {
   alignas(16) float val[NB * IPT];           // gathered per-edge values
   int off[kRowsPerThread * NB + 1];          // row offsets, rebased to the tile on use
-  float longsum[kRowsPerThread * NB];        // wavefront sums of rows longer than kSeqRow
+  float longsum[kRowsPerThread * NB];        // sums of the rows that wavefronts add
+  // rows of more than kWaveRow edges, added by a wavefront each (wave_rows epilogues)
+  int n_long;
+  int16_t long_row[NB * IPT / kWaveRow];
 };
 
 // Registers holding the loads of one tile that do not depend on a gather:
@@ -256,16 +615,38 @@ __device__ __forceinline__ double reduce_row_tile(int r0, int nr, const E& e,
   const int tid = threadIdx.x;
   float sum[kRowsPerThread];
   bool have_long = false;
+  constexpr bool kWaves1 = SEQ_ALL && wave_rows<E>::value;
 #pragma unroll
   for (int q = 0; q < kRowsPerThread; q++) {
     const int i = tid + q * NB;
     sum[q] = 0.0f;
     if (i < nr) {
       const int b = lds.off[i], en = lds.off[i + 1];
-      if (SEQ_ALL || en - b <= kSeqRow)
+      if (kWaves1 && en - b > kWaveRow) {
+        lds.long_row[atomicAdd(&lds.n_long, 1)] = (int16_t)i;
+        lds.longsum[i] = e.init(pre[q]);
+      } else if (SEQ_ALL || en - b <= kSeqRow)
         sum[q] = seq_sum(e.init(pre[q]), lds.val, b, en);
       else
         have_long = true;
+    }
+  }
+  if constexpr (kWaves1) {
+    __syncthreads();
+    const int n = lds.n_long;
+    if (n) {
+      for (int k = uniform((int)(tid / kWave)); k < n; k += NB / kWave) {
+        const int row = uniform((int)lds.long_row[k]);
+        const float s = wave_exact_row(uniform(lds.longsum[row]), lds.val, uniform(lds.off[row]),
+                                       uniform(lds.off[row + 1]));
+        if ((tid & (kWave - 1)) == 0) lds.longsum[row] = s;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < kRowsPerThread; q++) {
+        const int i = tid + q * NB;
+        if (i < nr && lds.off[i + 1] - lds.off[i] > kWaveRow) sum[q] = lds.longsum[i];
+      }
     }
   }
   if (!SEQ_ALL && __syncthreads_or(have_long)) {
@@ -315,6 +696,7 @@ __device__ __forceinline__ void stage_row_tile(const Tile& t, const TileRegs<IPT
                                                const float (&v)[IPT], RowTileLds<IPT, NB>& lds) {
   const int tid = threadIdx.x;
   const int nr = t.y - t.x, ne = t.w - t.z;
+  if (tid == 0) lds.n_long = 0;
 #pragma unroll
   for (int q = 0; q < kOffLoads; q++)
     if (tid + q * NB <= nr) lds.off[tid + q * NB] = R.offv[q] - t.z;
@@ -345,332 +727,6 @@ __device__ __forceinline__ double row_tile(const int32_t* __restrict__ off,
   stage_row_tile<IPT, SORTED, typename E::Pre, NB>(t, R, v, lds);
   __syncthreads();
   return reduce_row_tile<IPT, E, SEQ_ALL, NB>(r0, r1 - r0, e, R.pre, lds);
-}
-
-// ---------------------------------------------------------------------------
-// Sequential-order sums of long rows by a workgroup.
-//
-// exact_row_sum returns s0 + v[0] + v[1] + ... + v[n-1] rounded exactly as
-// the sequential FP32 loop `s = s0; for (i) s += v[i];` rounds it (the
-// reference's per-row loop, src/pr/omp_base.cc:34-37), computed by the whole
-// workgroup, kScanChunk terms at a time (thread t owns terms [16t, 16t+16)):
-//   While the running sum s lies in one binade, 2^k <= |s| < 2^(k+1) with
-//   ulp u = 2^(k-23), and the exact s + v[i] stays strictly inside it, the
-//   rounded step is s + q_i*u with q_i = v[i]/u rounded to the nearest
-//   integer: s advances by an integer number of ulps.  A positive term whose
-//   fraction is exactly 1/2 (a tie) rounds s to even: that step is the map
-//   x -> (x + floor(q)) rounded up to even.  Steps are maps of the running
-//   value that compose into maps of the same form (TieMap), so one workgroup
-//   prefix over the maps gives every running value of the chunk, ties
-//   included.  s advances over every step up to the first one that leaves
-//   the binade, is a negative tie or inf / NaN; that step is one ordinary
-//   FP32 addition and the scan restarts after it in the new binade.  From
-//   s == +0 the sum jumps to the first nonzero term; from a subnormal, -0 or
-//   non-finite s it takes one ordinary addition.  For sums of positive terms
-//   (PageRank) the restarts are the ~log2(n) binade crossings, most of them
-//   in the first terms of a row, which one lane adds serially (kExactHead).
-//   The next chunk's terms are gathered into registers while a chunk is
-//   scanned, so the gathers' latency overlaps the scan.
-// A host emulation of these steps (integer and float forms of q) matched the
-// sequential loop bit for bit on rows built to hit ties, binade crossings,
-// zeros, signs, subnormals and wide ranges.
-// ---------------------------------------------------------------------------
-
-constexpr int kScanPT = 16;                   // terms per thread per chunk
-constexpr int kScanChunk = kBlock * kScanPT;  // 4096
-constexpr int kExactHead = kScanChunk;       // terms of a row added by one lane first
-constexpr int kNoBad = 0x7fffffff;
-
-// A run of steps in integer ulps as one map of the running value x:
-//   t == 0:  x -> x + a
-//   t == 1:  x -> y + (y & 1) + b,  y = x + a
-// A regular step q is (0, q, 0); a positive tie above floor f is (1, f, 0).
-// After a round-to-even step the value is even, so what follows it only
-// depends on constants: maps compose into maps of the same form (wrapping
-// 32-bit arithmetic keeps the parity).
-struct TieMap {
-  uint32_t t, a, b;
-};
-
-__device__ __forceinline__ TieMap tie_compose(const TieMap& p, const TieMap& q) {  // p, then q
-  if (!p.t) return TieMap{q.t, p.a + q.a, q.b};
-  if (!q.t) return TieMap{1u, p.a, p.b + q.a};
-  const uint32_t c = p.b + q.a;
-  return TieMap{1u, p.a, c + (c & 1u) + q.b};
-}
-
-__device__ __forceinline__ uint32_t tie_apply(const TieMap& m, uint32_t x) {
-  const uint32_t y = x + m.a;
-  return m.t ? y + (y & 1u) + m.b : y;
-}
-
-// The step of term v (sign bit `neg`) in ulps of the binade with exponent ex:
-// T = v / u exactly (a power-of-two scaling; inf when v is far above the
-// binade), rounded to the nearest integer, |q| clamped to 2^26 (such a step
-// leaves the binade anyway).  irregular: a negative tie, or T not finite.
-// The sign comes in as an integer so that no per-term comparison of v is
-// loop-invariant (hoisted lane masks would crowd the scalar registers).
-__device__ __forceinline__ TieMap step_map(float v, uint32_t neg, int ex, uint32_t& irregular) {
-  const float T = ldexpf(v, 23 - ex);
-  const float fl = floorf(T);
-  const float fr = T - fl;  // exact
-  const float qf = fminf(fmaxf(fr > 0.5f ? fl + 1.0f : fl, -0x1p26f), 0x1p26f);
-  const uint32_t half = fr == 0.5f;  // T == +-0 gives fr == 0: no tie
-  irregular = (half & neg) | (uint32_t)!isfinite(T);
-  return TieMap{half & (neg ^ 1u), (uint32_t)(int32_t)qf, 0u};
-}
-
-// Inclusive prefix of the maps over the 64 lanes of a wavefront: DPP row
-// shifts inside each row of 16 lanes, then row broadcasts across rows (lanes
-// whose source is outside the row read the identity map (0, 0, 0)).
-#define GD_MAP_SCAN_STEP(CTRL, ROWS)                                                          \
-  {                                                                                           \
-    TieMap l;                                                                                 \
-    l.t = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)inc.t, CTRL, ROWS, 0xf, false);       \
-    l.a = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)inc.a, CTRL, ROWS, 0xf, false);       \
-    l.b = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)inc.b, CTRL, ROWS, 0xf, false);       \
-    inc = tie_compose(l, inc);                                                                \
-  }
-
-__device__ __forceinline__ TieMap wave_incl_scan_map(TieMap inc) {
-  GD_MAP_SCAN_STEP(0x111, 0xf)  // row_shr:1
-  GD_MAP_SCAN_STEP(0x112, 0xf)  // row_shr:2
-  GD_MAP_SCAN_STEP(0x114, 0xf)  // row_shr:4
-  GD_MAP_SCAN_STEP(0x118, 0xf)  // row_shr:8
-  GD_MAP_SCAN_STEP(0x142, 0xa)  // row_bcast:15 -> rows 1, 3
-  GD_MAP_SCAN_STEP(0x143, 0xc)  // row_bcast:31 -> rows 2, 3
-  return inc;
-}
-#undef GD_MAP_SCAN_STEP
-
-struct ExactLds {
-  uint32_t wt[kWaves], wa[kWaves], wb[kWaves];  // wave totals of the maps
-  int wbad[kWaves];                             // wave's first irregular term
-  float s;
-};
-
-// Workgroup-uniform values kept in scalar registers: branches on them are
-// scalar branches, not exec-mask updates.
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ float uniform(float v) {
-  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
-}
-
-// First value over the workgroup of a per-thread int that increases with the
-// thread index where present (kNoBad elsewhere): ballot per wave, then waves
-// in order.  Uniform result.  The cross-lane read runs with the whole wave
-// active: inside `if (lane == 0)` the compiler may compute v in lane 0 only
-// (it is used nowhere else), and the read would return another lane's stale
-// register.
-__device__ __forceinline__ int block_first(int v, ExactLds& x) {
-  const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
-  const uint64_t m = __ballot(v != kNoBad);
-  const int first = m ? __builtin_amdgcn_readlane(v, __builtin_ctzll(m)) : kNoBad;
-  if (lane == 0) x.wbad[wid] = first;
-  __syncthreads();
-  int r = kNoBad;
-#pragma unroll
-  for (int w = kWaves - 1; w >= 0; w--) r = (x.wbad[w] != kNoBad) ? x.wbad[w] : r;
-  return uniform(r);
-}
-
-// The scan of one chunk: nc terms in LDS (`val`, thread t's terms at 16t),
-// added to s from term `start` on.  All threads return the same s.  Ends with
-// the workgroup synchronised.  A thread's terms in [start, nc) are the set
-// bits of its mask `act`; the per-term checks are branch-free selects.
-__device__ __forceinline__ float exact_scan_chunk(const float* __restrict__ val, int nc,
-                                                  int start, float s, ExactLds& x) {
-  const int tid = threadIdx.x;
-  const int lane = tid & (kWave - 1), wid = tid / kWave;
-  const int lo = tid * kScanPT;
-  float v[kScanPT];
-  {
-    const float4* v4 = reinterpret_cast<const float4*>(val + lo);
-#pragma unroll
-    for (int k = 0; k < kScanPT / 4; k++) {
-      const float4 t = v4[k];
-      v[4 * k] = t.x;
-      v[4 * k + 1] = t.y;
-      v[4 * k + 2] = t.z;
-      v[4 * k + 3] = t.w;
-    }
-  }
-  const uint32_t below_nc = (1u << min(max(nc - lo, 0), kScanPT)) - 1u;
-  uint32_t negs = 0u, nonzero = 0u;  // per-term bits, computed once
-#pragma unroll
-  for (int k = 0; k < kScanPT; k++) {
-    const uint32_t b = __float_as_uint(v[k]);
-    negs |= (b >> 31) << k;
-    nonzero |= (uint32_t)((b << 1) != 0u) << k;
-  }
-  start = uniform(start);
-  s = uniform(s);
-  while (start < nc) {
-    const uint32_t sb = __float_as_uint(s);
-    const int eb = (int)((sb >> 23) & 0xffu);
-    if (eb <= 1 || eb == 0xff) {  // zero, subnormal, [2^-126, 2^-125), inf / NaN
-      if (sb == 0u) {
-        // +0 + (+-0) == +0: jump to the first nonzero term (+0 + v == v)
-        const uint32_t cand =
-            nonzero & below_nc & ~((1u << min(max(start - lo, 0), kScanPT)) - 1u);
-        const int nz = cand ? lo + __builtin_ctz(cand) : kNoBad;
-        const int jz = block_first(nz, x);
-        if (jz == kNoBad) {
-          start = nc;
-        } else {
-          s = uniform(val[jz]);
-          start = max(jz, start) + 1;  // every pass advances: the loop ends
-        }
-        __syncthreads();  // wbad is reused
-        continue;
-      }
-      s = uniform(s + val[start]);
-      start++;
-      continue;
-    }
-    const int ex = eb - 127;
-    const int32_t P = (int32_t)(sb & 0x7fffffu) | 0x800000;
-    const uint32_t Ps = (uint32_t)((sb >> 31) ? -P : P);
-    const uint32_t act = below_nc & ~((1u << min(max(start - lo, 0), kScanPT)) - 1u);
-    // this thread's steps (identity outside act) and their composition
-    uint32_t q[kScanPT];
-    uint32_t ties = 0u, irrs = 0u;
-    TieMap L{0u, 0u, 0u};
-    if (act) {  // whole waves before a restart skip this
-#pragma unroll
-      for (int k = 0; k < kScanPT; k++) {
-        const uint32_t a = (act >> k) & 1u;  // integer masks: no lane-mask registers
-        uint32_t irr;
-        const TieMap mk = step_map(v[k], (negs >> k) & 1u, ex, irr);
-        q[k] = mk.a & (0u - a);
-        const uint32_t tk = mk.t & a;
-        ties |= tk << k;
-        irrs |= (irr & a) << k;
-        L = tie_compose(L, TieMap{tk, q[k], 0u});
-      }
-    } else {
-#pragma unroll
-      for (int k = 0; k < kScanPT; k++) q[k] = 0u;
-    }
-    // workgroup prefix of the maps: waves in order, lanes in order
-    const TieMap inc = wave_incl_scan_map(L);
-    if (lane == kWave - 1) {
-      x.wt[wid] = inc.t;
-      x.wa[wid] = inc.a;
-      x.wb[wid] = inc.b;
-    }
-    TieMap ex_lane;
-    ex_lane.t = (uint32_t)__shfl_up((int)inc.t, 1, kWave);
-    ex_lane.a = (uint32_t)__shfl_up((int)inc.a, 1, kWave);
-    ex_lane.b = (uint32_t)__shfl_up((int)inc.b, 1, kWave);
-    if (lane == 0) ex_lane = TieMap{0u, 0u, 0u};
-    __syncthreads();
-    TieMap before{0u, 0u, 0u}, total{0u, 0u, 0u};
-#pragma unroll
-    for (int w = 0; w < kWaves; w++) {
-      const TieMap wm{x.wt[w], x.wa[w], x.wb[w]};
-      if (w < wid) before = tie_compose(before, wm);
-      total = tie_compose(total, wm);
-    }
-    // running values of this thread's terms, in order, up to the first one
-    // whose step is irregular or leaves the binade: |r| in (2^23, 2^24), or
-    // |r| == 2^23 (|s| == 2^k exactly) left unchanged by a zero term or one of
-    // its own sign, whose exact sum cannot have come from below 2^k
-    uint32_t run = tie_apply(tie_compose(before, ex_lane), Ps);
-    int bad = kNoBad;
-    uint32_t run_bad = 0u, alive = 1u;
-#pragma unroll
-    for (int k = 0; k < kScanPT; k++) {
-      const uint32_t y = run + q[k];
-      const uint32_t r = y + (y & (ties >> k) & 1u);  // a tie rounds to even
-      const uint32_t ar = (uint32_t)abs((int32_t)r);
-      const uint32_t away = ((nonzero >> k) ^ 1u) | ((negs >> k) ^ (run >> 31) ^ 1u);
-      const uint32_t stay = (uint32_t)(r == run) & (uint32_t)(ar == 0x800000u) & away;
-      const uint32_t ok = ((uint32_t)(ar - 0x800001u < 0x7fffffu) | stay) & ~(irrs >> k) & 1u;
-      const uint32_t lv = (act >> k) & alive;
-      const uint32_t fail = lv & (ok ^ 1u);
-      run_bad = fail ? run : run_bad;
-      bad = fail ? lo + k : bad;
-      alive &= fail ^ 1u;
-      run = (lv & ok) ? r : run;
-    }
-    const int jb = block_first(bad, x);
-    if (jb == kNoBad) {
-      // exact: an integer below 2^24 in magnitude times a power of two
-      s = uniform(ldexpf((float)(int32_t)tie_apply(total, Ps), ex - 23));
-      start = nc;
-      __syncthreads();  // wt/wa/wb and wbad are reused
-    } else {
-      if (bad == jb) x.s = ldexpf((float)(int32_t)run_bad, ex - 23) + val[jb];  // FP32 step
-      __syncthreads();
-      s = uniform(x.s);
-      start = max(jb, start) + 1;
-      __syncthreads();
-    }
-  }
-  return s;
-}
-
-// s0 + the gathered values of edges [e0, e0+ne) in edge order, rounded as the
-// sequential FP32 loop starting from s0 (all threads return it).  `buf0`,
-// `buf1`: two 16-byte aligned LDS buffers of kScanChunk floats.  Chunk c is
-// gathered as thread t's terms t + 256 j (coalesced index loads), stored at
-// their position in the chunk, and scanned as thread t's terms 16t..16t+15;
-// chunk c+1's gathers and chunk c+2's index loads are in flight meanwhile.
-// The first kExactHead terms are one lane's chain (lane_seq_sum): there the
-// running sum crosses binades every few terms, and each crossing would cost
-// the scan a restart.  STAGED: the row's values were gathered beforehand into
-// a buffer (`g` reads it by edge, the column index is not loaded).
-template <bool NT, class G, bool STAGED = false>
-__device__ float exact_row_sum(const int32_t* __restrict__ col, int e_max, int e0, int ne,
-                               const G& g, float s0, float* __restrict__ buf0,
-                               float* __restrict__ buf1, ExactLds& x) {
-  const int tid = threadIdx.x;
-  const int nchunks = (ne + kScanChunk - 1) / kScanChunk;
-  int idx[kScanPT];
-  float vv[kScanPT];
-  auto elem = [&](int c, int j) {  // edge offset in the row, clamped into it
-    return min(c * kScanChunk + tid + j * kBlock, ne - 1);
-  };
-  auto load_idx = [&](int c) {
-#pragma unroll
-    for (int j = 0; j < kScanPT; j++)
-      idx[j] = STAGED ? 0 : ld_stream<NT>(col + min(e0 + elem(c, j), e_max));
-  };
-  auto gather = [&](int c) {
-#pragma unroll
-    for (int j = 0; j < kScanPT; j++) vv[j] = g.value(e0 + elem(c, j), idx[j]);
-  };
-  float s = s0;
-  if (nchunks == 0) return s;
-  load_idx(0);
-  gather(0);
-  if (nchunks > 1) load_idx(1);
-  for (int c = 0; c < nchunks; c++) {
-    float* cur = (c & 1) ? buf1 : buf0;
-    const int nc = min(kScanChunk, ne - c * kScanChunk);
-#pragma unroll
-    for (int j = 0; j < kScanPT; j++)
-      if (tid + j * kBlock < nc) cur[tid + j * kBlock] = vv[j];
-    if (c + 1 < nchunks) {
-      gather(c + 1);                         // in flight during the scan of chunk c
-      if (c + 2 < nchunks) load_idx(c + 2);  // likewise
-    }
-    __syncthreads();
-    int start = 0;
-    if (c == 0) {
-      // the first terms, where s crosses a binade every few steps: one lane's
-      // pipelined chain, in order
-      const int nh = min(nc, kExactHead);
-      if (tid == 0) x.s = lane_seq_sum<8>(s, cur, nh);
-      __syncthreads();
-      s = x.s;
-      start = nh;
-      __syncthreads();
-    }
-    s = exact_scan_chunk(cur, nc, start, s, x);
-  }
-  return s;
 }
 
 // ---------------------------------------------------------------------------

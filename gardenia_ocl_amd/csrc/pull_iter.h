@@ -247,7 +247,7 @@ __global__ __launch_bounds__(kBlock) void pull_persistent_kernel(const typename 
 // edge order.  hub_body: exact hub h of the iteration (the caller checked
 // st->done).
 struct HubLds {
-  alignas(16) float buf[2 * kScanChunk];  // two chunks of the row, double-buffered
+  alignas(16) float buf[kScanChunk];  // one chunk of the row
   ExactLds xs;
 };
 
@@ -256,7 +256,6 @@ __device__ __forceinline__ void hub_body(const typename P::Args& a, const IterAr
                                          HubLds& lds) {
   const int odd = it.st->iter & 1;
   __shared__ double s_err[kWaves];
-  float* const buf = lds.buf;
   ExactLds& xs = lds.xs;
   const Tile t = it.hub_tiles[h];
   const auto g = P::template gather<NT>(a, odd);
@@ -266,11 +265,10 @@ __device__ __forceinline__ void hub_body(const typename P::Args& a, const IterAr
   float sum;
   if constexpr (STAGED)
     sum = exact_row_sum<(NT > 0), StagedGather, true>(
-        it.col, it.e_max, t.z, ne, StagedGather{it.stage + it.hub_soff[h], t.z}, e.init(pre), buf,
-        buf + kScanChunk, xs);
+        it.col, it.e_max, t.z, ne, StagedGather{it.stage + it.hub_soff[h], t.z}, e.init(pre),
+        nullptr, xs);
   else
-    sum = exact_row_sum<(NT > 0)>(it.col, it.e_max, t.z, ne, g, e.init(pre), buf,
-                                  buf + kScanChunk, xs);
+    sum = exact_row_sum<(NT > 0)>(it.col, it.e_max, t.z, ne, g, e.init(pre), lds.buf, xs);
   double err = 0.0;
   if (threadIdx.x == 0) err = e.finish(t.x, sum, pre);
   const double tot = block_sum<kWaves>(err, s_err);

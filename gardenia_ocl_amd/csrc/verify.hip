@@ -39,6 +39,7 @@ struct VerifyEpilogue {
   const float* __restrict__ scores;
   float base;
   float damp;
+  static constexpr bool kWaveRows = true;
   struct Pre {
     float old;
   };
