@@ -7,12 +7,17 @@
 // bit-identical to solving each graph alone), its own base score (1-d)/m_g,
 // its own iteration counter / parity / convergence flag.  One pull launch
 // covers the tiles of every graph (tiles of converged graphs exit at once;
-// rows of > 2048 edges are whole-row tiles summed in the reference's order),
+// rows of > 4096 edges are whole-row tiles summed in the reference's order),
 // then one finalize workgroup per graph adds its tiles' L1 partials in a fixed
-// order and updates that graph's state -- no cross-workgroup synchronisation.  A chunk of iterations (pull + finalize
-// launches with identical arguments) is captured once into a hipGraph and
-// replayed until every graph has converged; small graphs are launch-bound, so
-// this is where the time goes.
+// order and updates that graph's state -- no cross-workgroup synchronisation.
+// A chunk of iterations (pull + finalize launches with identical arguments) is
+// captured once into a hipGraph and replayed until every graph has converged.
+//
+// What bounds it: the L2 requests of the gathers.  Every graph's contrib fits
+// an XCD's L2, so a tile's edges are gathered in source order (tile_sort.h;
+// lanes share lines) and the kernel holds 94 registers and 24.6 KB of LDS:
+// 64 RMAT graphs of 2^12 to 2^18 vertices, 62 M edges, tol 1e-4: 4.00 ms; in
+// edge order and with one lane's chain for the hub rows 5.23 ms.
 
 #include <hip/hip_runtime.h>
 
@@ -25,6 +30,7 @@
 #include "gd_common.h"
 #include "pr_policy.h"
 #include "pull_engine.h"
+#include "tile_sort.h"
 
 namespace gd {
 namespace {
@@ -46,6 +52,7 @@ struct MgArgs {
   const int32_t* __restrict__ off;
   const int32_t* __restrict__ col;
   int e_max;
+  const uint16_t* __restrict__ pos;  // each edge's offset in its tile (tile_sort.h)
   const int32_t* __restrict__ outdeg;
   float* __restrict__ scores;
   float* __restrict__ c0;
@@ -66,23 +73,25 @@ __global__ __launch_bounds__(kBlock) void mg_pull_kernel(const MgArgs a) {
   const int g = a.tile_graph[blockIdx.x];
   if (a.gs[g].done) return;
   const int odd = a.gs[g].iter & 1;
-  // a row tile's LDS, or a hub row's two chunk buffers + the broadcast sum
-  static_assert(sizeof(RowTileLds<kMgIPT>) >= (2 * kHubChunk + 1) * sizeof(float), "LDS union");
-  __shared__ __align__(16) unsigned char smem[sizeof(RowTileLds<kMgIPT>)];
-  RowTileLds<kMgIPT>& lds = *reinterpret_cast<RowTileLds<kMgIPT>*>(smem);
+  __shared__ union {
+    RowTileLds<kMgIPT> tile;
+    struct {
+      alignas(16) float buf[kScanChunk];
+      ExactLds xs;
+    } hub;
+  } lds;
   __shared__ double s_err[kWaves];
   const Tile t = a.tiles[blockIdx.x];
   const PrGather gat{odd ? a.c1 : a.c0};
   double err = 0.0;
   const PrEpilogue<0> e{a.scores, odd ? a.c0 : a.c1, a.outdeg, a.gs[g].base, a.damp, -1};
   if (t.y >= 0) {
-    err = row_tile<kMgIPT, false, false, decltype(gat), decltype(e), true>(
-        a.off, a.col, nullptr, a.e_max, t.x, t.y, t.z, t.w - t.z, gat, e, lds);
+    err = row_tile<kMgIPT, false, true, decltype(gat), decltype(e), true>(
+        a.off, a.col, a.pos, a.e_max, t.x, t.y, t.z, t.w - t.z, gat, e, lds.tile);
   } else {  // whole hub row in the reference's order, as the single-graph plan
     const auto pre = e.pre(t.x);
-    float* const buf = reinterpret_cast<float*>(smem);
-    const float sum = hub_chain_sum<8, false>(a.col, nullptr, a.e_max, t.z, t.w - t.z, gat,
-                                              e.init(pre), buf, buf + kHubChunk, buf + 2 * kHubChunk);
+    const float sum = exact_row_sum<false>(a.col, a.e_max, t.z, t.w - t.z, gat, e.init(pre),
+                                           lds.hub.buf, lds.hub.xs);
     if (threadIdx.x == 0) err = e.finish(t.x, sum, pre);
   }
   const double tot = block_sum<kWaves>(err, s_err);
@@ -162,7 +171,7 @@ struct gd_multi_pr_plan {
   hipStream_t user_stream = nullptr;
   hipStream_t stream = nullptr;  // private stream (graph capture needs a non-null one)
   std::vector<int32_t> m, vbase;
-  DeviceBuffer off, col, deg, scores, c0, c1, tiles, tile_graph, hub_row, hub_slot, hub_nseg,
+  DeviceBuffer off, col, pos, deg, scores, c0, c1, tiles, tile_graph, hub_row, hub_slot, hub_nseg,
       hub_part, err_part, gs, errors, d_vbase, d_user_ptrs;
   int n_tiles = 0;
   int e_max = 0;
@@ -218,6 +227,7 @@ int gd_multi_pr_plan_create(int n_graphs, const int32_t* m, const int64_t* nnz,
   GD_HIP_TRY(hipStreamSynchronize(p->user_stream));
   int rc = p->off.alloc(4 * ((size_t)tm + 1));
   if (!rc) rc = p->col.alloc(4 * (size_t)std::max<int64_t>(te, 1));
+  if (!rc) rc = p->pos.alloc(2 * (size_t)std::max<int64_t>(te, 1));
   if (!rc) rc = p->deg.alloc(4 * (size_t)tm);
   if (!rc) rc = p->scores.alloc(4 * (size_t)tm);
   if (!rc) rc = p->c0.alloc(4 * (size_t)tm);
@@ -273,6 +283,13 @@ int gd_multi_pr_plan_create(int n_graphs, const int32_t* m, const int64_t* nnz,
   p->e_max = (int)std::max<int64_t>(te - 1, 0);
   if (te == 0) GD_HIP_TRY(hipMemsetAsync(p->col.ptr, 0, 4, p->stream));
   p->h_state = gs;
+  if (te > 0) {  // each tile's edges in source order, as the single-graph plan
+    Schedule all;
+    all.tiles = tiles;
+    rc = build_tile_sort(all, kBlock * kMgIPT, p->col.as<int32_t>(), p->col.as<int32_t>(),
+                         p->pos.as<uint16_t>(), p->stream, true);
+    if (rc) return fail(rc);
+  }
   const int nh = (int)hub_row.size();
   rc = p->tiles.alloc(sizeof(Tile) * p->n_tiles);
   if (!rc) rc = p->tile_graph.alloc(4 * (size_t)p->n_tiles);
@@ -337,7 +354,7 @@ int gd_multi_pr_run(gd_multi_pr_plan* p, float* const* d_scores, const gd_pr_opt
   GD_HIP_TRY(hipMemcpyAsync(p->d_user_ptrs.ptr, d_scores, sizeof(float*) * G,
                             hipMemcpyHostToDevice, p->stream));
   const MgArgs a{p->tiles.as<Tile>(), p->tile_graph.as<int32_t>(), p->off.as<int32_t>(),
-                 p->col.as<int32_t>(), p->e_max, p->deg.as<int32_t>(), p->scores.as<float>(),
+                 p->col.as<int32_t>(), p->e_max, p->pos.as<uint16_t>(), p->deg.as<int32_t>(), p->scores.as<float>(),
                  p->c0.as<float>(), p->c1.as<float>(), p->hub_part.as<float>(),
                  p->err_part.as<double>(), p->gs.as<GraphState>(), p->hub_row.as<int32_t>(),
                  p->hub_slot.as<int32_t>(), p->hub_nseg.as<int32_t>(), p->errors.as<double>(),
