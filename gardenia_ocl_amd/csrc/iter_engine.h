@@ -277,31 +277,33 @@ struct IterEngine {
 
   template <class P, int IPT, int NT, bool SORTED>
   void launch_pull_s(const typename P::Args& a, const IterArgs& it) {
-    // Exact hubs go first, on the plan's stream, so that their workgroups
-    // (longest row first) are placed before the row tiles fill the CUs; the
-    // row tiles fork onto the side stream (after the same prior work) and
-    // join back.
-    if (fused) {  // small iteration: one launch (hubs first, then row tiles)
-      hipLaunchKernelGGL((pull_small_kernel<P, IPT, NT, SORTED>),
-                         dim3(n_hub_tiles + (n_tiles > 0 ? pull_grid : 0)), dim3(kBlock), 0,
-                         stream, a, it);
-      return;
-    }
-    const bool fork = n_hub_tiles > 0 && n_tiles > 0;
     const bool staged = P::kExactHubs && n_hub_tiles > 0 && it.hub_soff;
-    // staged hubs: their values are gathered first, by the whole GPU, before
-    // the fork (the row tiles would otherwise fill the CUs first and hold the
-    // hub rows back until they drain)
     if (win.on())
       hipLaunchKernelGGL(window_expand_kernel<P>, dim3(win.n_pieces), dim3(kExpandBlock), 0, stream,
                          a, it, win.n_src, win.pieces.as<int4>(), win.sid.as<uint16_t>(),
                          win.stage.as<float>());
+    // staged hubs: their values are gathered first, by the whole GPU
     if (staged && win.on())
       hipLaunchKernelGGL((hub_stage_kernel<P, NT, true>), dim3(n_stage_blocks), dim3(kBlock), 0,
                          stream, a, it, stage_blocks.as<int4>(), stage.as<float>());
     else if (staged)
       hipLaunchKernelGGL((hub_stage_kernel<P, NT, false>), dim3(n_stage_blocks), dim3(kBlock), 0,
                          stream, a, it, stage_blocks.as<int4>(), stage.as<float>());
+    if (!persistent && block == kBlock) {  // one launch: hubs first, then row tiles
+      const dim3 grid(n_hub_tiles + n_tiles);
+      if (staged)
+        hipLaunchKernelGGL((pull_kernel<P, IPT, NT, SORTED, P::kExactHubs>), grid, dim3(kBlock), 0,
+                           stream, a, it);
+      else if (grid.x > 0)
+        hipLaunchKernelGGL((pull_kernel<P, IPT, NT, SORTED, false>), grid, dim3(kBlock), 0, stream,
+                           a, it);
+      return;
+    }
+    // Exact hubs go first, on the plan's stream, so that their workgroups
+    // (longest row first) are placed before the row tiles fill the CUs; the
+    // row tiles fork onto the side stream (after the same prior work) and
+    // join back.
+    const bool fork = n_hub_tiles > 0 && n_tiles > 0;
     hipStream_t ts = stream;
     if (fork) {
       (void)hipEventRecord(fork_ev, stream);
@@ -323,11 +325,8 @@ struct IterEngine {
       if (persistent)
         hipLaunchKernelGGL((pull_persistent_kernel<P, IPT, NT, SORTED>), dim3(pull_grid),
                            dim3(kBlock), 0, ts, a, it);
-      else if (wide_tiles<P>::value && block > kBlock)
-        launch_wide<P, IPT, NT, SORTED>(a, it, ts);
       else
-        hipLaunchKernelGGL((pull_tile_kernel<P, IPT, NT, SORTED>), dim3(n_tiles), dim3(kBlock), 0,
-                           ts, a, it);
+        launch_wide<P, IPT, NT, SORTED>(a, it, ts);
     }
     if (fork) {
       (void)hipEventRecord(join_ev, side);

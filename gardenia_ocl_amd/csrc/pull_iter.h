@@ -175,7 +175,8 @@ __device__ __forceinline__ void tile_body(const typename P::Args& a, const IterA
   }
 }
 
-template <class P, int IPT, int NT, bool SORTED, int NB = kBlock>
+// Row tiles of wider workgroups.
+template <class P, int IPT, int NT, bool SORTED, int NB>
 __global__ __launch_bounds__(NB) void pull_tile_kernel(const typename P::Args a,
                                                        const IterArgs it) {
   if (it.st->done) return;
@@ -329,26 +330,27 @@ __global__ __launch_bounds__(kExpandBlock) void window_expand_kernel(
   window_expand(g.source(), n_src, pieces[blockIdx.x], sid, slots, win);
 }
 
-// Held to 3 waves per SIMD (<= 168 VGPRs): the hub workgroups share the CUs
-// with the row tiles running beside them.  The gathering form spills three
-// registers once per 4096-edge chunk, outside the scan's loops; the staged
-// form spills none.
+// A launch of its own, beside the row tiles' on another stream, where those
+// run on wider workgroups or a persistent grid.
 template <class P, int IPT, int NT, bool SORTED, bool STAGED>
-__global__ __launch_bounds__(kBlock, 3) void exact_hub_kernel(const typename P::Args a,
+__global__ __launch_bounds__(kBlock) void exact_hub_kernel(const typename P::Args a,
                                                               const IterArgs it) {
   if (it.st->done) return;
   __shared__ HubLds lds;
   hub_body<P, IPT, NT, SORTED, STAGED>(a, it, blockIdx.x, lds);
 }
 
-// Small iterations (it.fuse_parts > 0) in one launch: workgroups [0,
-// n_hub_tiles) take the exact hubs (longest first), the rest the row tiles,
-// and the last workgroup to finish closes the iteration (fused_finish) --
-// one kernel per iteration, no fork, join or finalize.
-// The two bodies share one LDS allocation.
-template <class P, int IPT, int NT, bool SORTED>
-__global__ __launch_bounds__(kBlock, 3) void pull_small_kernel(const typename P::Args a,
-                                                               const IterArgs it) {
+// Exact hubs and row tiles of 256-thread workgroups in one launch:
+// workgroups [0, n_hub_tiles) take the exact hubs (longest first), so they
+// are placed before the tiles fill the CUs, the rest the row tiles.  The two
+// bodies share one LDS allocation, and the hub body needs fewer registers
+// than the tile's (72 and 94), so it costs the tiles nothing; two launches on
+// two streams cost about 20 us of fork and join per iteration (1 M vertices:
+// 78 to 60 us).  In small iterations (it.fuse_parts > 0) the last workgroup
+// to finish closes the iteration (fused_finish): no finalize launch either.
+template <class P, int IPT, int NT, bool SORTED, bool STAGED>
+__global__ __launch_bounds__(kBlock) void pull_kernel(const typename P::Args a,
+                                                      const IterArgs it) {
   if (it.st->done) return;
   __shared__ union {
     RowTileLds<IPT> tile;
@@ -356,11 +358,12 @@ __global__ __launch_bounds__(kBlock, 3) void pull_small_kernel(const typename P:
   } lds;
   if constexpr (P::kExactHubs) {
     if ((int)blockIdx.x < it.n_hub_tiles) {
-      hub_body<P, IPT, NT, SORTED>(a, it, blockIdx.x, lds.hub);
+      hub_body<P, IPT, NT, SORTED, STAGED>(a, it, blockIdx.x, lds.hub);
       return;
     }
   }
-  tile_body<P, IPT, NT, SORTED>(a, it, blockIdx.x - it.n_hub_tiles, lds.tile);
+  const int b = blockIdx.x - it.n_hub_tiles;
+  tile_body<P, IPT, NT, SORTED>(a, it, it.slots ? xcd_run_block(b, it.n_tiles) : b, lds.tile);
 }
 
 // Hub-row epilogues (segment partials summed in segment order) and the L1
