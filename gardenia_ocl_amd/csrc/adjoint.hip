@@ -39,7 +39,10 @@ namespace gd {
 struct WGather {
   const float* __restrict__ w;  // per-edge weight, in the order of the pulled CSR
   const float* __restrict__ c;  // gathered vector
+  static constexpr bool kScaled = true;
   __device__ __forceinline__ float value(int e, int u) const { return w[e] * c[u]; }
+  __device__ __forceinline__ float raw(int u) const { return c[u]; }
+  __device__ __forceinline__ float factor(int e) const { return w[e]; }
   __device__ __forceinline__ const float* source() const { return c; }
   __device__ __forceinline__ void from(const float* v) { c = v; }
 };
@@ -138,16 +141,51 @@ struct AdjPolicy {
 
 // ---------------------------------------------------------------- small kernels
 
-// s_u = sum of the CSC row u (one wavefront per row, fixed order).
+// s_u = sum of the CSC row u: lane-strided partial sums and the wavefront's
+// butterfly, a fixed order.  Bound by latency, not bytes: most rows are short,
+// so a wavefront takes 4 rows at a time, those of at most 16 entries by 16
+// lanes each (the butterfly's first two steps would only add zeros), and a
+// long row keeps 32 loads in flight.  RMAT-20: 500 us with a wavefront per
+// row and one load at a time, 115 us.
+__device__ __forceinline__ float long_row_sum(const float* __restrict__ val, int k, int e) {
+  float s = 0.0f;
+  for (; k + 31 * 64 < e; k += 32 * 64) {
+    float v[32];
+#pragma unroll
+    for (int q = 0; q < 32; q++) v[q] = val[k + q * 64];
+#pragma unroll
+    for (int q = 0; q < 32; q++) s += v[q];
+  }
+  for (; k + 3 * 64 < e; k += 4 * 64) {
+    const float v0 = val[k], v1 = val[k + 64], v2 = val[k + 128], v3 = val[k + 192];
+    s += v0;
+    s += v1;
+    s += v2;
+    s += v3;
+  }
+  for (; k < e; k += 64) s += val[k];
+  return wave_sum(s);
+}
+
 __global__ __launch_bounds__(256) void row_sums_kernel(int n, const int32_t* __restrict__ off,
                                                        const float* __restrict__ val,
                                                        float* __restrict__ out) {
-  const int lane = threadIdx.x & 63;
-  for (int r = blockIdx.x * 4 + threadIdx.x / 64; r < n; r += gridDim.x * 4) {
-    float s = 0.0f;
-    for (int k = off[r] + lane; k < off[r + 1]; k += 64) s += val[k];
-    s = wave_sum(s);
-    if (lane == 0) out[r] = s;
+  const int lane = threadIdx.x & 63, sub = lane / 16;
+  for (int r0 = 4 * (blockIdx.x * 4 + threadIdx.x / 64); r0 < n; r0 += 16 * gridDim.x) {
+    const int r = min(r0 + sub, n - 1);
+    const int b = off[r], len = off[r + 1] - b;
+    float s = (len <= 16 && lane % 16 < len) ? val[b + lane % 16] : 0.0f;
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (len <= 16 && lane % 16 == 0 && r0 + sub < n) out[r] = s;
+    uint64_t more = __ballot(len > 16 && lane % 16 == 0 && r0 + sub < n);
+    while (more) {
+      const int l = __builtin_ctzll(more);
+      more &= more - 1;
+      const int lb = __builtin_amdgcn_readlane(b, l), ln = __builtin_amdgcn_readlane(len, l);
+      const float t = long_row_sum(val, lb + lane, lb + ln);
+      if (lane == 0) out[r0 + l / 16] = t;
+    }
   }
 }
 
@@ -286,7 +324,7 @@ namespace {
 int wpr_refresh_weights(gd_wpr_plan* p) {
   int rc = transpose_values(p->tr, p->nnz, p->a, p->at.as<float>(), p->stream);
   if (rc) return rc;
-  hipLaunchKernelGGL(row_sums_kernel, dim3(grid_n(p->m / 4 + 1)), dim3(256), 0, p->stream, p->m,
+  hipLaunchKernelGGL(row_sums_kernel, dim3(grid_n((int64_t)p->m * 16)), dim3(256), 0, p->stream, p->m,
                      p->tr.off.as<int32_t>(), p->at.as<float>(), p->s.as<float>());
   GD_HIP_TRY(hipGetLastError());
   return GD_OK;
@@ -334,9 +372,11 @@ int gd_wpr_plan_create(int m, int64_t nnz, const int32_t* d_off, const int32_t* 
   }
   // The forward sums every row in edge order (bit-exact), so it takes the
   // plain PageRank plan's tiles: 4096 edges, gathered in source order, hub
-  // rows above 4096 edges.  The adjoint tree-sums its longer rows: sorting or
-  // resizing its tiles changes that rounding, and at RMAT-20, tol 1e-7, took
-  // 145 iterations instead of 128 at the same time per iteration.
+  // rows above 4096 edges.  The adjoint tree-sums its longer rows: resizing
+  // its tiles changes that rounding, and at RMAT-20, tol 1e-7, took 145
+  // iterations instead of 128.
+  p->adj.sort_tiles = p->adj.windows = true;
+  p->fwd.windows = true;
   p->fwd.ipt = 16;
   p->fwd.sort_tiles = true;
   p->fwd.exact_len = 4096;  // hub rows in edge order, as the plain PageRank plan

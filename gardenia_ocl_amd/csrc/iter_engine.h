@@ -41,7 +41,7 @@ struct IterEngine {
   int exact_len = 0;         // > 0: rows longer than this are whole-row exact hub tiles
   bool sort_tiles = false;   // gather each tile's edges in source order (tile_sort.h)
   // Windowed gather (window_gather.h) where the gathered vector exceeds an
-  // XCD's L2; sorted tiles and exact hubs only.
+  // XCD's L2; sorted tiles only.
   bool windows = false;
   WindowGather win;
   int32_t* col_owned = nullptr;  // the caller's private copy of col: sorted in place
@@ -138,7 +138,7 @@ struct IterEngine {
       }
       // exact hub rows are kept in edge order, or sorted in staging blocks
       const int64_t segs = (int64_t)sched.tiles.size() + nnz / kScanChunk + sched.n_slots;
-      const bool win_on = windows && exact_len > 0 && stage_hubs != 0 && !persistent && m > kWindowMin &&
+      const bool win_on = windows && stage_hubs != 0 && !persistent && m > kWindowMin &&
                           window_gather_fits(m, nnz, segs);
       std::vector<int2> seg;
       rc = build_tile_sort(sched, block * ipt, col, dst, pos.as<uint16_t>(), stream,

@@ -127,26 +127,50 @@ __device__ __forceinline__ float lane_seq_sum(float s, const float* __restrict__
   return s;
 }
 
-// Sequential sum s + v[b] + ... + v[e-1] from LDS (`v` 16-byte aligned) by
-// the calling lane, in order with FP32 rounding.  More than kChainRow terms:
-// scalar adds up to a 16-byte boundary, then float4 reads 32 terms ahead of
-// the dependent adds (lane_seq_sum); fewer: 4 reads in flight.
-constexpr int kChainRow = 32;
-
+// Sequential sum s + v[b] + ... + v[e-1] from LDS (`v` 16-byte aligned, the
+// granule of 4 that holds e - 1 readable) by the calling lane, in order with
+// FP32 rounding.  All reads are whole granules issued ahead of the adds that
+// need them: the row's first granule, blocks of 4 granules double-buffered,
+// then up to 4 granules; terms outside the row are replaced by -0.0, which
+// added to any s gives s.  Reading the ends of a row term by term made each of
+// up to 34 terms wait for its own LDS read: the sums took 4-7 us of a row
+// tile's 11-16 us.
 __device__ __forceinline__ float seq_sum(float s, const float* __restrict__ v, int b, int e) {
-  int k = b;
-  if (e - b > kChainRow) {
-    for (; k & 3; k++) s += v[k];
-    return lane_seq_sum<8>(s, v + k, e - k);
+  if (b >= e) return s;
+  const float4* __restrict__ v4 = reinterpret_cast<const float4*>(v);
+  const int g1 = (e + 3) >> 2, m0 = (b >> 2) + 1;
+  const int nb = max((e >> 2) - m0, 0) >> 2;
+  const int t0 = m0 + 4 * nb;
+  const float4 h = v4[m0 - 1];
+  float4 A[4], B[4];
+  auto load = [&](float4(&R)[4], int g) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) R[k] = v4[min(g + k, g1 - 1)];
+  };
+  load(A, m0);  // the first block, or the last granules
+  auto masked = [&](const float4& x, int i) {  // the granule at term i
+    const unsigned n = (unsigned)(e - b), o = (unsigned)(i - b);
+    s += o < n ? x.x : -0.0f;
+    s += o + 1u < n ? x.y : -0.0f;
+    s += o + 2u < n ? x.z : -0.0f;
+    s += o + 3u < n ? x.w : -0.0f;
+  };
+  masked(h, 4 * (m0 - 1));
+  for (int k = 0; k < nb; k++) {
+    load(B, m0 + 4 * (k + 1));
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      s += A[q].x;
+      s += A[q].y;
+      s += A[q].z;
+      s += A[q].w;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) A[q] = B[q];
   }
-  for (; k + 4 <= e; k += 4) {
-    const float a0 = v[k], a1 = v[k + 1], a2 = v[k + 2], a3 = v[k + 3];
-    s += a0;
-    s += a1;
-    s += a2;
-    s += a3;
-  }
-  for (; k < e; k++) s += v[k];
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    if (t0 + q < g1) masked(A[q], 4 * (t0 + q));
   return s;
 }
 
@@ -517,30 +541,74 @@ __device__ __forceinline__ void load_positions(const uint16_t* __restrict__ pos,
     p[j] = (int)ld_stream<NT>(pos + e0 + min((int)threadIdx.x + j * NB, last));
 }
 
+// Gathers of the form factor(e) * raw(u) (G::kScaled): in a sorted tile the
+// factors, stored in CSR order, are loaded in that order and applied once the
+// gathered values are back at their CSR positions in LDS (scale_tile).
+template <class G, class = void>
+struct scaled_gather : std::false_type {};
+template <class G>
+struct scaled_gather<G, std::void_t<decltype(G::kScaled)>> : std::bool_constant<G::kScaled> {};
+
 template <int IPT, bool SORTED, class G, int NB = kBlock>
 __device__ __forceinline__ void gather_values(const G& g, int e0, int ne, const int (&idx)[IPT],
                                               const int (&p)[IPT], float (&v)[IPT]) {
   const int last = ne - 1;
 #pragma unroll
+  for (int j = 0; j < IPT; j++) {
+    if constexpr (SORTED && scaled_gather<G>::value)
+      v[j] = g.raw(idx[j]);
+    else
+      v[j] = g.value(e0 + (SORTED ? p[j] : min((int)threadIdx.x + j * NB, last)), idx[j]);
+  }
+}
+
+// factor(e) of this thread's edges e0 + tid + j*NB (clamped), in CSR order.
+template <int IPT, class G, int NB = kBlock>
+__device__ __forceinline__ void load_factors(const G& g, int e0, int ne, float (&f)[IPT]) {
+#pragma unroll
+  for (int j = 0; j < IPT; j++) f[j] = g.factor(e0 + min((int)threadIdx.x + j * NB, ne - 1));
+}
+
+// val[i] *= factor of edge i, between two barriers.
+template <int IPT, int NB = kBlock>
+__device__ __forceinline__ void scale_tile(float* val, int ne, const float (&f)[IPT]) {
+  __syncthreads();
+#pragma unroll
   for (int j = 0; j < IPT; j++)
-    v[j] = g.value(e0 + (SORTED ? p[j] : min((int)threadIdx.x + j * NB, last)), idx[j]);
+    if ((int)threadIdx.x + j * NB < ne) val[threadIdx.x + j * NB] *= f[j];
 }
 
 // Sum of the gathered values of a hub segment [e0, e0+ne), ne >= 1: per-thread
 // partial in j order, wave butterfly, then waves in order.  Valid in thread 0.
+// A sorted segment's values go back to their CSR positions through `val`
+// (kBlock*IPT floats of LDS) first, so the sum is the same bits.
 template <int IPT, bool NT, bool SORTED, class G>
 __device__ __forceinline__ float segment_sum(const int32_t* __restrict__ col,
                                              const uint16_t* __restrict__ pos, int e0, int ne,
-                                             const G& g, float* s_tmp) {
+                                             const G& g, float* val) {
   int idx[IPT], p[IPT];
   float v[IPT];
   load_indices<IPT, NT>(col, e0, ne, idx);
   if constexpr (SORTED) load_positions<IPT, NT>(pos, e0, ne, p);
   gather_values<IPT, SORTED>(g, e0, ne, idx, p, v);
+  if constexpr (SORTED) {
+    float f[IPT];
+    if constexpr (scaled_gather<G>::value) load_factors<IPT>(g, e0, ne, f);
+#pragma unroll
+    for (int j = 0; j < IPT; j++)
+      if ((int)threadIdx.x + j * kBlock < ne) val[p[j]] = v[j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < IPT; j++) {
+      v[j] = val[min((int)threadIdx.x + j * kBlock, ne - 1)];
+      if constexpr (scaled_gather<G>::value) v[j] *= f[j];
+    }
+    __syncthreads();  // val is reused by the block sum
+  }
   float s = 0.0f;
 #pragma unroll
   for (int j = 0; j < IPT; j++) s += ((int)threadIdx.x + j * kBlock < ne) ? v[j] : 0.0f;
-  return block_sum<kWaves>(s, s_tmp);
+  return block_sum<kWaves>(s, val);
 }
 
 // Rows of a tile longer than this are added by a wavefront (wave_exact_row)
@@ -724,7 +792,14 @@ __device__ __forceinline__ double row_tile(const int32_t* __restrict__ off,
   issue_tile_loads<IPT, NT, SORTED, E, NB>(t, off, col, pos, e_max, e, R);
   float v[IPT];
   if (ne > 0) gather_values<IPT, SORTED, G, NB>(g, e0, ne, R.idx, R.pos, v);
-  stage_row_tile<IPT, SORTED, typename E::Pre, NB>(t, R, v, lds);
+  if constexpr (SORTED && scaled_gather<G>::value) {
+    float f[IPT];
+    if (ne > 0) load_factors<IPT, G, NB>(g, e0, ne, f);
+    stage_row_tile<IPT, SORTED, typename E::Pre, NB>(t, R, v, lds);
+    scale_tile<IPT, NB>(lds.val, ne, f);
+  } else {
+    stage_row_tile<IPT, SORTED, typename E::Pre, NB>(t, R, v, lds);
+  }
   __syncthreads();
   return reduce_row_tile<IPT, E, SEQ_ALL, NB>(r0, r1 - r0, e, R.pre, lds);
 }

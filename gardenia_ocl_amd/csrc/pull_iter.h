@@ -220,6 +220,11 @@ __global__ __launch_bounds__(kBlock) void pull_persistent_kernel(const typename 
       issue_tile_loads<IPT, (NT > 0), SORTED>(nxt, it.off, it.col, it.pos, it.e_max, e, Rn);
       if (cur.y >= 0) {
         stage_row_tile<IPT, SORTED>(cur, R, v, lds);
+        if constexpr (SORTED && scaled_gather<decltype(g)>::value) {
+          float f[IPT];
+          if (ne > 0) load_factors<IPT>(g, cur.z, ne, f);
+          scale_tile<IPT>(lds.val, ne, f);
+        }
         __syncthreads();
         err += reduce_row_tile<IPT, decltype(e), P::kSeqAll>(cur.x, cur.y - cur.x, e, R.pre, lds);
       } else if constexpr (!P::kExactHubs) {
@@ -301,17 +306,20 @@ __global__ __launch_bounds__(kBlock) void hub_stage_kernel(const typename P::Arg
   for (int j = 0; j < kScanPT; j++)
     idx[j] = ld_stream<(NT > 0)>(it.col + b.x + min((int)threadIdx.x + j * kBlock, b.y - 1));
   if constexpr (PERM) load_positions<kScanPT, (NT > 0)>(it.pos, b.x, b.y, p);
-#pragma unroll
-  for (int j = 0; j < kScanPT; j++)
-    v[j] = g.value(b.x + (PERM ? p[j] : min((int)threadIdx.x + j * kBlock, b.y - 1)), idx[j]);
+  gather_values<kScanPT, PERM>(g, b.x, b.y, idx, p, v);
   if constexpr (PERM) {
     __shared__ float s_v[kScanChunk];
+    float f[kScanPT];
+    if constexpr (scaled_gather<decltype(g)>::value) load_factors<kScanPT>(g, b.x, b.y, f);
 #pragma unroll
     for (int j = 0; j < kScanPT; j++)
       if ((int)threadIdx.x + j * kBlock < b.y) s_v[p[j]] = v[j];
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < kScanPT; j++) v[j] = s_v[min((int)threadIdx.x + j * kBlock, b.y - 1)];
+    for (int j = 0; j < kScanPT; j++) {
+      v[j] = s_v[min((int)threadIdx.x + j * kBlock, b.y - 1)];
+      if constexpr (scaled_gather<decltype(g)>::value) v[j] *= f[j];
+    }
   }
 #pragma unroll
   for (int j = 0; j < kScanPT; j++)
