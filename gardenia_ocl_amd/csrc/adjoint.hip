@@ -29,7 +29,6 @@
 #include "gd_common.h"
 #include "iter_engine.h"
 #include "pull_engine.h"
-#include "spmv_internal.h"
 #include "transpose.h"
 
 namespace gd {
@@ -214,6 +213,8 @@ __global__ void pack_cq_kernel(int n, const float* __restrict__ x, const float* 
   }
 }
 
+constexpr int kBwdTile = kBlock * 8;  // edges of a tile of the SpMV backward's plan
+
 // Row tiles of at most this many edges label their edges' rows in LDS first.
 constexpr int kMapEdges = 4096;
 
@@ -225,14 +226,63 @@ constexpr int kMapEdges = 4096;
 // tiles binary-search every edge.  A launch with gridDim.y > 1 splits each
 // one-row (hub) tile's edges over gridDim.y workgroups; row tiles need
 // gridDim.y == 1.
-template <class F>
+//
+// WIN (windowed gather of the operand that the column selects): col holds
+// slots, sorted within each tile, with their offsets there in pos.  The
+// tile's values (f.slots) go to their CSR positions in LDS first, and f is
+// called with the value instead of the column.
+template <class F, bool WIN = false>
 __global__ __launch_bounds__(kBlock) void edge_map_kernel(const Tile* __restrict__ tiles,
                                                           const int32_t* __restrict__ off,
-                                                          const int32_t* __restrict__ col, F f) {
+                                                          const int32_t* __restrict__ col, F f,
+                                                          const uint16_t* __restrict__ pos = nullptr) {
+  constexpr int kEdges = WIN ? kBwdTile : kMapEdges;
   __shared__ int s_off[kTileRows + 1];
-  __shared__ uint16_t s_row[kMapEdges];
+  __shared__ uint16_t s_row[kEdges];
   static_assert(kTileRows <= 65536, "row table holds 16-bit tile rows");
-  const Tile t = tiles[blockIdx.x];
+  const Tile t = tiles[WIN ? xcd_run_block(blockIdx.x, gridDim.x) : (int)blockIdx.x];
+  if constexpr (WIN) {  // tiles of at most kBwdTile edges, hub segments too
+    __shared__ float s_val[kBwdTile];
+    constexpr int kU = kBwdTile / kBlock;
+    const int n = t.w - t.z;
+    int slot[kU], p[kU];
+    float v[kU];
+#pragma unroll
+    for (int j = 0; j < kU; j++) {
+      const int e = t.z + min((int)threadIdx.x + j * kBlock, max(n - 1, 0));
+      slot[j] = n > 0 ? col[e] : 0;
+      p[j] = n > 0 ? pos[e] : 0;
+    }
+#pragma unroll
+    for (int j = 0; j < kU; j++) v[j] = f.slots[slot[j]];
+#pragma unroll
+    for (int j = 0; j < kU; j++)
+      if ((int)threadIdx.x + j * kBlock < n) s_val[p[j]] = v[j];
+    const int nr = t.y >= 0 ? t.y - t.x : 0;
+    for (int i = threadIdx.x; i <= nr; i += kBlock) s_off[i] = off[t.x + i];
+    __syncthreads();
+    if (t.y >= 0) {
+      const int per = (n + kBlock - 1) / kBlock;
+      const int e0 = t.z + threadIdx.x * per, e1 = min(e0 + per, t.w);
+      if (e0 < e1) {
+        int lo = 0, hi = nr;
+        while (hi - lo > 1) {
+          const int mid = (lo + hi) >> 1;
+          if (s_off[mid] <= e0) lo = mid; else hi = mid;
+        }
+        int next = s_off[lo + 1];
+        for (int e = e0; e < e1; e++) {
+          while (next <= e) next = s_off[++lo + 1];
+          s_row[e - t.z] = (uint16_t)lo;
+        }
+      }
+      __syncthreads();
+    }
+    for (int i = threadIdx.x; i < n; i += kBlock)
+      f(t.z + i, t.y >= 0 ? t.x + s_row[i] : t.x, s_val[i]);
+    return;
+  }
+  if constexpr (!WIN) {
   if (t.y >= 0) {
     const int nr = t.y - t.x;
     for (int i = threadIdx.x; i <= nr; i += kBlock) s_off[i] = off[t.x + i];
@@ -269,6 +319,7 @@ __global__ __launch_bounds__(kBlock) void edge_map_kernel(const Tile* __restrict
     for (int e = t.z + blockIdx.y * kBlock + threadIdx.x; e < t.w; e += kBlock * gridDim.y)
       f(e, t.x, col[e]);
   }
+  }
 }
 
 struct WprGradOp {
@@ -289,14 +340,20 @@ struct SpmvDaOp {
   __device__ __forceinline__ void operator()(int k, int r, int c) const { dA[k] = g[r] * x[c]; }
 };
 
-// the same product with x[c] read from its slice-major copy: Xs[inv[k]] = x[c]
-struct SpmvDaSlicedOp {
-  const float* __restrict__ xs;
-  const int32_t* __restrict__ inv;
+// the same product with x[c] from its slot
+struct SpmvDaSlotOp {
+  const float* __restrict__ slots;
   const float* __restrict__ g;
   float* __restrict__ dA;
-  __device__ __forceinline__ void operator()(int k, int r, int) const { dA[k] = g[r] * xs[inv[k]]; }
+  __device__ __forceinline__ void operator()(int k, int r, float xc) const { dA[k] = g[r] * xc; }
 };
+
+__global__ __launch_bounds__(kExpandBlock) void bwd_expand_kernel(
+    const float* __restrict__ x, int cols, const int4* __restrict__ pieces,
+    const uint16_t* __restrict__ sid, float* __restrict__ slots) {
+  __shared__ float win[kWinSize];
+  window_expand(x, cols, pieces[blockIdx.x], sid, slots, win);
+}
 
 static int grid_n(int64_t n) { return (int)std::min<int64_t>((n + 255) / 256, 16384); }
 
@@ -469,7 +526,7 @@ int gd_wpr_backward(gd_wpr_plan* p, const float* d_x, const float* d_w, float* d
     // every edge once: the forward's row tiles, then its whole-row hub tiles
     if (p->fwd.n_tiles)
       hipLaunchKernelGGL(edge_map_kernel<WprGradOp>, dim3(p->fwd.n_tiles), dim3(kBlock), 0,
-                         p->stream, p->fwd.tiles.as<Tile>(), p->off, p->col, op);
+                         p->stream, p->fwd.tiles.as<Tile>(), p->off, p->col, op, nullptr);
     if (p->fwd.n_hub_tiles) {
       // one workgroup per 8 edges per thread of the longest hub
       const int split = std::min<int64_t>(
@@ -477,7 +534,7 @@ int gd_wpr_backward(gd_wpr_plan* p, const float* d_x, const float* d_w, float* d
                                        (kBlock * 8)));
       hipLaunchKernelGGL(edge_map_kernel<WprGradOp>, dim3(p->fwd.n_hub_tiles, split),
                          dim3(kBlock), 0, p->stream, p->fwd.hub_tiles.as<Tile>(), p->off, p->col,
-                         op);
+                         op, nullptr);
     }
     GD_HIP_TRY(hipGetLastError());
   }
@@ -504,53 +561,27 @@ struct gd_spmv_bwd_plan {
   DeviceBuffer tiles;
   int n_tiles = 0;
   gd_spmv_plan* tplan = nullptr;  // SpMV over the CSC: dx = A^T g
-  // tplan in the column-sliced mode: its slice-major value copy is filled from
-  // A's values by vperm (two passes through buckets) instead of `at`
-  bool sliced = false;
-  BucketedPermutation vperm;  // A's values (CSR order) -> the CSC plan's slice-major copy
-  // x larger than one XCD's L2 and A's rows sorted: x gathered in A's
-  // column-sliced order (fplan; slice s on XCD s, so the gathers hit L2), then
-  // dA over A's tiles reads x[c] from that copy (inv[k] = slice-major position
-  // of entry k: eight sequential streams, one per slice).  The copy lives in
-  // fplan's slice-major value array, which fplan itself never reads (it is
-  // never run as an SpMV).
-  gd_spmv_plan* fplan = nullptr;
-  DeviceBuffer inv;
+  // g larger than one XCD's L2: A's values go into CSC order through buckets
+  // (vperm), in two passes whose scattered accesses stay in L2
+  bool bucketed = false;
+  BucketedPermutation vperm;
+  // x larger than one XCD's L2: dA reads x through windows (window_gather.h)
+  WindowGather win;
+  DeviceBuffer slot, pos;
   ~gd_spmv_bwd_plan() {
     gd_spmv_plan_destroy(tplan);
-    gd_spmv_plan_destroy(fplan);
   }
 };
 
 namespace gd {
 namespace {
 
-// keys[k] = s * nb + (col[k] >> cshift) for the CSR entry k of row r, where
-// s = min(r / width, 7) is the column slice of the CSC plan holding the entry:
-// a bucket is one slice's entries in a range of 2^cshift columns of A.
-__global__ void bucket_keys_kernel(int rows, const int32_t* __restrict__ off,
-                                   const int32_t* __restrict__ col, int width, int cshift, int nb,
+// keys[k] = bucket of CSR entry k: its column's range of 2^cshift columns
+__global__ void bucket_keys_kernel(int64_t nnz, const int32_t* __restrict__ col, int cshift,
                                    int32_t* __restrict__ keys) {
-  const int lane = threadIdx.x & 63;
-  for (int r = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64; r < rows;
-       r += gridDim.x * (blockDim.x / 64)) {
-    const int base = min(r / width, 7) * nb;
-    for (int e = off[r] + lane; e < off[r + 1]; e += 64) keys[e] = base + (col[e] >> cshift);
-  }
-}
-
-__global__ void iota_kernel(int64_t n, int32_t* __restrict__ a) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    a[i] = (int32_t)i;
-}
-
-// inv[fwd[i]] = i
-__global__ void invert_perm_kernel(int64_t n, const int32_t* __restrict__ fwd,
-                                   int32_t* __restrict__ inv) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    inv[fwd[i]] = (int32_t)i;
+  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < nnz;
+       e += (int64_t)gridDim.x * blockDim.x)
+    keys[e] = col[e] >> cshift;
 }
 
 }  // namespace
@@ -597,68 +628,41 @@ int gd_spmv_bwd_plan_create(int rows, int cols, int64_t nnz, const int32_t* d_Ap
   if (rc) return fail(rc);
   GD_HIP_TRY(hipMemsetAsync(p->at.ptr, 0, 4 * (size_t)std::max<int64_t>(nnz, 1), p->stream));
   if (cols > 0) {
-    // g larger than one XCD's L2: the column-sliced mode (the CSC's rows are
-    // sorted; a matrix with repeated entries in a row is not, and keeps the
-    // tile mode)
     if (nnz > 0 && (int64_t)rows * 4 > (4 << 20)) {
-      rc = gd_spmv_plan_create_ex(cols, rows, nnz, p->tr.off.as<int32_t>(),
-                                  p->tr.row.as<int32_t>(), p->at.as<float>(), stream,
-                                  GD_SPMV_SLICED, &p->tplan);
-      if (rc == GD_ERR_INVALID) rc = GD_OK;  // unsorted: p->tplan stays NULL
-      if (rc) return fail(rc);
-    }
-    if (p->tplan) {
-      // The values go into the CSC plan's slice-major copy through buckets of
-      // about 2^18 entries (a slice's entries in a range of A's columns): the
-      // slice-major order reads the buckets one after another.
-      p->sliced = true;
-      DeviceBuffer perm_s, keys;
-      rc = perm_s.alloc(4 * (size_t)nnz);
-      if (!rc) rc = keys.alloc(4 * (size_t)nnz);
-      if (!rc) rc = spmv_slice_order(p->tplan, p->tr.perm.as<int32_t>(), perm_s.as<int32_t>());
-      const int64_t nb_want = std::max<int64_t>(1, nnz / (8ll << 18));
+      // buckets of about 2^18 entries: a range of A's columns, contiguous in
+      // CSC order, so the second pass reads the buckets one after another
+      p->bucketed = true;
+      DeviceBuffer keys;
+      rc = keys.alloc(4 * (size_t)nnz);
+      const int64_t nb_want = std::max<int64_t>(1, nnz >> 18);
       int cshift = 0;
       while (((int64_t)cols >> cshift) > nb_want) cshift++;
-      const int nb = (int)(((int64_t)cols + (1ll << cshift) - 1) >> cshift);
+      const int64_t nb = ((int64_t)cols + (1ll << cshift) - 1) >> cshift;
       int key_bits = 1;
-      while ((1ll << key_bits) < 8ll * nb) key_bits++;
+      while ((1ll << key_bits) < nb) key_bits++;
       if (!rc) {
-        const int width = std::max(1, (rows + 7) / 8);  // the CSC plan's slice width
-        hipLaunchKernelGGL(bucket_keys_kernel, dim3(grid_n(rows / 4 + 1)), dim3(256), 0,
-                           p->stream, rows, d_Ap, d_Aj, width, cshift, nb, keys.as<int32_t>());
+        hipLaunchKernelGGL(bucket_keys_kernel, dim3(grid_n(nnz)), dim3(256), 0, p->stream, nnz,
+                           d_Aj, cshift, keys.as<int32_t>());
         if (hipGetLastError() != hipSuccess) rc = GD_ERR_DEVICE;
       }
       if (!rc)
-        rc = build_bucketed_permutation(nnz, keys.as<int32_t>(), key_bits, perm_s.as<int32_t>(),
-                                        p->stream, &p->vperm);
-    } else {
-      rc = gd_spmv_plan_create(cols, rows, nnz, p->tr.off.as<int32_t>(), p->tr.row.as<int32_t>(),
-                               p->at.as<float>(), stream, &p->tplan);
+        rc = build_bucketed_permutation(nnz, keys.as<int32_t>(), key_bits,
+                                        p->tr.perm.as<int32_t>(), p->stream, &p->vperm);
+      if (rc) return fail(rc);
     }
+    rc = gd_spmv_plan_create(cols, rows, nnz, p->tr.off.as<int32_t>(), p->tr.row.as<int32_t>(),
+                             p->at.as<float>(), stream, &p->tplan);
   }
   if (rc) return fail(rc);
-  if (rows > 0 && nnz > 0 && (int64_t)cols * 4 > (4 << 20)) {
-    // the sliced layout's value copy (of `at`, zeros) becomes the x copy
-    rc = gd_spmv_plan_create_ex(rows, cols, nnz, d_Ap, d_Aj, p->at.as<float>(), stream,
-                                GD_SPMV_SLICED, &p->fplan);
-    if (rc == GD_ERR_INVALID) rc = GD_OK;  // unsorted rows: the edge map below
-    if (!rc && p->fplan) {
-      DeviceBuffer ids, kmap;
-      rc = ids.alloc(4 * (size_t)nnz);
-      if (!rc) rc = kmap.alloc(4 * (size_t)nnz);
-      if (!rc) rc = p->inv.alloc(4 * (size_t)nnz);
-      if (!rc) {
-        hipLaunchKernelGGL(iota_kernel, dim3(grid_n(nnz)), dim3(256), 0, p->stream, nnz,
-                           ids.as<int32_t>());
-        rc = spmv_slice_order(p->fplan, ids.as<int32_t>(), kmap.as<int32_t>());
-      }
-      if (!rc) {
-        hipLaunchKernelGGL(invert_perm_kernel, dim3(grid_n(nnz)), dim3(256), 0, p->stream, nnz,
-                           kmap.as<int32_t>(), p->inv.as<int32_t>());
-        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(p->stream) != hipSuccess)
-          rc = GD_ERR_DEVICE;
-      }
-    }
+  if (rows > 0 && (int64_t)cols * 4 > (4 << 20) && nnz >= 2 * (int64_t)cols &&
+      window_gather_fits(cols, nnz, (int64_t)p->sched.tiles.size())) {
+    rc = p->slot.alloc(4 * (size_t)nnz);
+    if (!rc) rc = p->pos.alloc(2 * (size_t)nnz);
+    std::vector<int2> segs;
+    if (!rc)
+      rc = build_tile_sort(p->sched, kBwdTile, d_Aj, p->slot.as<int32_t>(), p->pos.as<uint16_t>(),
+                           p->stream, false, 0, &segs);
+    if (!rc) rc = build_window_gather(cols, nnz, segs, p->slot.as<int32_t>(), p->stream, &p->win);
     if (rc) return fail(rc);
   }
   *out = owner.release();
@@ -671,9 +675,9 @@ int gd_spmv_bwd_run(gd_spmv_bwd_plan* p, const float* d_Ax, const float* d_x, co
   GD_CHECK_ARG(p->rows == 0 || d_g, "NULL g");
   if (d_dx && p->cols > 0) {
     GD_CHECK_ARG(p->nnz == 0 || d_Ax, "NULL Ax");
-    int rc = p->sliced ? run_bucketed_permutation(p->vperm, d_Ax, spmv_sliced_values(p->tplan),
-                                                  p->stream)
-                       : transpose_values(p->tr, p->nnz, d_Ax, p->at.as<float>(), p->stream);
+    int rc = p->bucketed
+                 ? run_bucketed_permutation(p->vperm, d_Ax, p->at.as<float>(), p->stream)
+                 : transpose_values(p->tr, p->nnz, d_Ax, p->at.as<float>(), p->stream);
     if (rc) return rc;
     hipLaunchKernelGGL(fill_kernel, dim3(grid_n(p->cols)), dim3(256), 0, p->stream, p->cols,
                        d_dx, 0.0f);
@@ -682,13 +686,14 @@ int gd_spmv_bwd_run(gd_spmv_bwd_plan* p, const float* d_Ax, const float* d_x, co
   }
   if (d_dA && p->nnz > 0) {
     GD_CHECK_ARG(d_x != nullptr, "NULL x");
-    if (p->fplan) {
-      float* xs = spmv_sliced_values(p->fplan);
-      const int rc = spmv_sliced_gather(p->fplan, d_x, xs);
-      if (rc) return rc;
-      const SpmvDaSlicedOp op{xs, p->inv.as<int32_t>(), d_g, d_dA};
-      hipLaunchKernelGGL(edge_map_kernel<SpmvDaSlicedOp>, dim3(p->n_tiles), dim3(kBlock), 0,
-                         p->stream, p->tiles.as<Tile>(), p->Ap, p->Aj, op);
+    if (p->win.on()) {
+      hipLaunchKernelGGL(bwd_expand_kernel, dim3(p->win.n_pieces), dim3(kExpandBlock), 0,
+                         p->stream, d_x, p->cols, p->win.pieces.as<int4>(),
+                         p->win.sid.as<uint16_t>(), p->win.stage.as<float>());
+      const SpmvDaSlotOp op{p->win.stage.as<float>(), d_g, d_dA};
+      hipLaunchKernelGGL((edge_map_kernel<SpmvDaSlotOp, true>), dim3(p->n_tiles), dim3(kBlock), 0,
+                         p->stream, p->tiles.as<Tile>(), p->Ap, p->slot.as<int32_t>(), op,
+                         p->pos.as<uint16_t>());
     } else {
       const SpmvDaOp op{d_x, d_g, d_dA};
       hipLaunchKernelGGL(edge_map_kernel<SpmvDaOp>, dim3(p->n_tiles), dim3(kBlock), 0, p->stream,

@@ -156,15 +156,25 @@ __device__ __forceinline__ float seq_sum(float s, const float* __restrict__ v, i
     s += o + 3u < n ? x.w : -0.0f;
   };
   masked(h, 4 * (m0 - 1));
-  for (int k = 0; k < nb; k++) {
-    load(B, m0 + 4 * (k + 1));
+  auto add = [&](const float4(&R)[4]) {
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-      s += A[q].x;
-      s += A[q].y;
-      s += A[q].z;
-      s += A[q].w;
+      s += R[q].x;
+      s += R[q].y;
+      s += R[q].z;
+      s += R[q].w;
     }
+  };
+  int k = 0;
+  for (; k + 2 <= nb; k += 2) {
+    load(B, m0 + 4 * (k + 1));
+    add(A);
+    load(A, m0 + 4 * (k + 2));
+    add(B);
+  }
+  if (k < nb) {
+    load(B, t0);
+    add(A);
 #pragma unroll
     for (int q = 0; q < 4; q++) A[q] = B[q];
   }

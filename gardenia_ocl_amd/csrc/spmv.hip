@@ -1,13 +1,21 @@
 // spmv.hip -- CSR SpMV y <- y + A x for gfx950 (src/spmv/omp_base.cc:17-28).
 //
-// Same tile engine as PageRank: products x[Aj[k]] * Ax[k] are formed during
-// the gather (rounded, this file is built with -ffp-contract=off) and staged
+// Same tile engine as PageRank: products x[Aj[k]] * Ax[k] are formed
+// (rounded, this file is built with -ffp-contract=off) and staged
 // in LDS; rows are then summed by one thread starting from
 // y[row] in CSR order, which is exactly the reference's arithmetic; so are
 // the longer rows of a tile (the owner thread's chain just runs longer).
 // Rows longer than a tile get a workgroup each that feeds one lane's
 // sequential chain in CSR order (hub_chain_sum), so every row is the
 // reference's sum bit for bit.
+//
+// Where x exceeds an XCD's L2 and the rows gather from enough of it, the
+// gathers go through windows of x (window_gather.h): a pass expands x into
+// one slot per nonzero, and the tiles read their slots in runs.  The matrix
+// values stay the caller's, read in CSR order.  Bound by HBM: 6 bytes per
+// nonzero in the first pass, 14 in the second.  2^22 x 2^22, 32 random
+// columns per row: 0.536 ms, 0.737 with one pass of the tiles per 1/8 of the
+// columns over a reordered copy of the matrix, 1.9 with plain gathers.
 
 #include <hip/hip_runtime.h>
 
@@ -19,8 +27,8 @@
 #include "gardenia_hip.h"
 #include "gd_common.h"
 #include "pull_engine.h"
-#include "spmv_internal.h"
-#include <rocprim/device/device_scan.hpp>
+#include "tile_sort.h"
+#include "window_gather.h"
 
 namespace gd {
 
@@ -31,6 +39,16 @@ struct SpGather {
   const float* __restrict__ x;
   const float* __restrict__ Ax;
   __device__ __forceinline__ float value(int e, int j) const { return x[j] * Ax[e]; }
+};
+
+// x[j] from its slot, Ax in CSR order.
+struct SpSlotGather {
+  const float* __restrict__ slots;
+  const float* __restrict__ Ax;
+  static constexpr bool kScaled = true;
+  __device__ __forceinline__ float value(int e, int slot) const { return slots[slot] * Ax[e]; }
+  __device__ __forceinline__ float raw(int slot) const { return slots[slot]; }
+  __device__ __forceinline__ float factor(int e) const { return Ax[e]; }
 };
 
 struct SpEpilogue {
@@ -44,121 +62,59 @@ struct SpEpilogue {
   }
 };
 
-// Tile mode, one launch: workgroups [0, n_long) each add one row longer than
+// Workgroups [0, n_long) each add one row longer than
 // a tile (2048 nonzeros) in CSR order on one lane (hub_chain_sum: products of
 // both signs), the rest one LDS row tile each (every row summed by its owner
 // thread in CSR order).  Every row is the reference's sum bit for bit.  LONG =
 // false (no long rows) leaves the long-row code, and its registers, out.
-template <bool LONG>
+// WIN: Aj holds slots, sorted by source within each tile, with their offsets
+// there in pos; long rows always gather x itself.
+template <bool LONG, bool WIN>
 __global__ __launch_bounds__(kBlock) void spmv_pull_kernel(
-    const Tile* __restrict__ tiles, const Tile* __restrict__ long_tiles, int n_long,
-    const int32_t* __restrict__ Ap, const int32_t* __restrict__ Aj, int e_max,
-    const float* __restrict__ Ax, const float* __restrict__ x, float* __restrict__ y) {
+    const Tile* __restrict__ tiles, int n_tiles, const Tile* __restrict__ long_tiles, int n_long,
+    const int32_t* __restrict__ Ap, const int32_t* __restrict__ Aj,
+    const uint16_t* __restrict__ pos, int e_max, const float* __restrict__ Ax,
+    const float* __restrict__ x, float* __restrict__ y) {
   // a row tile's LDS, or a long row's two chunk buffers + the broadcast sum
   static_assert(sizeof(RowTileLds<kSpIPT>) >= (2 * kHubChunk + 1) * sizeof(float), "LDS union");
   __shared__ __align__(16) unsigned char smem[sizeof(RowTileLds<kSpIPT>)];
   RowTileLds<kSpIPT>& lds = *reinterpret_cast<RowTileLds<kSpIPT>*>(smem);
-  const SpGather g{x, Ax};
+  using G = std::conditional_t<WIN, SpSlotGather, SpGather>;
+  const G g{x, Ax};
   const int b = blockIdx.x;
   if (LONG && b < n_long) {
     float* const buf = reinterpret_cast<float*>(smem);
     const Tile t = long_tiles[b];
-    const float s = hub_chain_sum<16, false>(Aj, nullptr, e_max, t.z, t.w - t.z, g, y[t.x], buf,
-                                            buf + kHubChunk, buf + 2 * kHubChunk);
+    const float s = hub_chain_sum<16, false>(Aj, nullptr, e_max, t.z, t.w - t.z, SpGather{x, Ax},
+                                             y[t.x], buf, buf + kHubChunk, buf + 2 * kHubChunk);
     if (threadIdx.x == 0) y[t.x] = s;
   } else {
-    const Tile t = tiles[b - n_long];
+    const Tile t = tiles[WIN ? xcd_run_block(b - n_long, n_tiles) : b - n_long];
     const SpEpilogue e{y};
-    (void)row_tile<kSpIPT, false, false, SpGather, SpEpilogue, true>(
-        Ap, Aj, nullptr, e_max, t.x, t.y, t.z, t.w - t.z, g, e, lds);
+    (void)row_tile<kSpIPT, false, WIN, G, SpEpilogue, true>(
+        Ap, Aj, pos, e_max, t.x, t.y, t.z, t.w - t.z, g, e, lds);
   }
 }
 
-// ---------------------------------------------------------------- column slices
-//
-// For matrices whose x does not fit in one XCD's L2 (ER 2^22: 16.8 MB of x vs
-// 4 MB) every gather of the tile engine misses L2.  The sliced mode splits the
-// columns into kSlices ranges of x (2 MB each for ER 2^22) and keeps a
-// slice-major copy of the matrix: slice 0's entries of every row (rows in
-// order, each row's entries in column order), then slice 1's, ...  One SpMV
-// runs the row engine once per slice, slice 0 first: pass q sums each row's
-// slice-q products by the row's owner thread onto y[r] (LDS-staged tiles of
-// that slice's entries; the x gathers of a pass stay in one 2 MB range, which
-// every XCD's L2 holds).  For rows with sorted columns the passes add each
-// row's products in column order -- the reference's loop
-// (src/spmv/omp_base.cc:21-26) -- so y is its result bit for bit, with y
-// itself carrying the running sum between passes.
-constexpr int kSlices = 8;
-
-// cnt[s * (rows+1) + r] = entries of row r in column slice s.
-__global__ void slice_count_kernel(int rows, const int32_t* __restrict__ Ap,
-                                   const int32_t* __restrict__ Aj, int width,
-                                   int32_t* __restrict__ cnt, int* __restrict__ unsorted) {
-  for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < rows; r += gridDim.x * blockDim.x) {
-    int c[kSlices] = {0, 0, 0, 0, 0, 0, 0, 0};
-    int prev = -1, bad = 0;
-    for (int k = Ap[r]; k < Ap[r + 1]; k++) {
-      const int j = Aj[k];
-      bad |= j <= prev;
-      prev = j;
-      c[min(j / width, kSlices - 1)]++;
-    }
-#pragma unroll
-    for (int q = 0; q < kSlices; q++) cnt[(int64_t)q * (rows + 1) + r] = c[q];
-    if (bad) atomicOr(unsorted, 1);
-  }
+// Pass 1 of a windowed SpMV (window_gather.h).
+__global__ __launch_bounds__(kExpandBlock) void spmv_expand_kernel(
+    const float* __restrict__ x, int cols, const int4* __restrict__ pieces,
+    const uint16_t* __restrict__ sid, float* __restrict__ slots) {
+  __shared__ float win[kWinSize];
+  window_expand(x, cols, pieces[blockIdx.x], sid, slots, win);
 }
 
-// Scatter each row's entries into the slice-major arrays (row order kept):
-// the column indices unless values_only, and a 4-byte payload per entry (the
-// values, or any other per-entry array).
-template <class T>
-__global__ void slice_scatter_kernel(int rows, const int32_t* __restrict__ Ap,
-                                     const int32_t* __restrict__ Aj, const T* __restrict__ Ax,
-                                     int width, const int32_t* __restrict__ soff,
-                                     const int64_t* __restrict__ sbase, int32_t* __restrict__ Aj_s,
-                                     T* __restrict__ Ax_s, int values_only) {
-  for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < rows; r += gridDim.x * blockDim.x) {
-    int64_t pos[kSlices];
-#pragma unroll
-    for (int q = 0; q < kSlices; q++) pos[q] = sbase[q] + soff[(int64_t)q * (rows + 1) + r];
-    for (int k = Ap[r]; k < Ap[r + 1]; k++) {
-      const int j = Aj[k];
-      const int q = min(j / width, kSlices - 1);
-      int64_t at = 0;
-#pragma unroll
-      for (int t = 0; t < kSlices; t++)
-        if (t == q) at = pos[t]++;
-      if (!values_only) Aj_s[at] = j;
-      Ax_s[at] = Ax[k];
-    }
+// flag |= a row's columns are not strictly increasing
+__global__ void sorted_rows_kernel(int rows, const int32_t* __restrict__ Ap,
+                                   const int32_t* __restrict__ Aj, int* __restrict__ unsorted) {
+  const int lane = threadIdx.x & 15;  // 16 lanes a row
+  int bad = 0;
+  for (int r = (blockIdx.x * blockDim.x + threadIdx.x) / 16; r < rows;
+       r += gridDim.x * blockDim.x / 16) {
+    const int b = Ap[r], e = Ap[r + 1];
+    for (int k = b + 1 + lane; k < e; k += 16) bad |= Aj[k] <= Aj[k - 1];
   }
-}
-
-// Xs[i] = x[Aj_s[i]] for every slice-major entry i.  Workgroup b takes slice
-// b % kSlices and its entries [2048 (b / kSlices), + 2048): workgroups are
-// dispatched to the 8 XCDs round-robin, so slice s runs on XCD s, whose L2
-// then holds that 1/8 of x; index loads and stores are coalesced, 8 gathers
-// in flight per thread.
-constexpr int kGatherPT = 8;
-
-__global__ __launch_bounds__(256) void slice_gather_kernel(const int64_t* __restrict__ sbase,
-                                                           const int32_t* __restrict__ Aj_s,
-                                                           const float* __restrict__ x,
-                                                           float* __restrict__ Xs) {
-  const int q = blockIdx.x % kSlices;
-  const int64_t b = sbase[q], e = sbase[q + 1];
-  const int64_t c = b + (int64_t)(blockIdx.x / kSlices) * (256 * kGatherPT);
-  if (c >= e) return;
-  int j[kGatherPT];
-  float v[kGatherPT];
-#pragma unroll
-  for (int t = 0; t < kGatherPT; t++) j[t] = Aj_s[min(c + t * 256 + threadIdx.x, e - 1)];
-#pragma unroll
-  for (int t = 0; t < kGatherPT; t++) v[t] = x[j[t]];
-#pragma unroll
-  for (int t = 0; t < kGatherPT; t++)
-    if (c + t * 256 + threadIdx.x < e) Xs[c + t * 256 + threadIdx.x] = v[t];
+  if (bad) atomicOr(unsorted, 1);
 }
 
 }  // namespace gd
@@ -177,34 +133,35 @@ struct gd_spmv_plan {
   DeviceBuffer tiles, long_tiles;
   DeviceBuffer dummy_col;  // 1 element, used as Aj when nnz == 0
   int e_max = 0;
-  // column-sliced mode: per slice, its long rows then its row tiles in
-  // slice_tiles[slice_first[q] ...]
-  bool sliced = false;
-  int width = 0;
-  DeviceBuffer soff, sbase, Aj_s, Ax_s, slice_tiles;
-  std::vector<int64_t> slice_base;
-  std::vector<int> slice_first, slice_long, slice_rows;
+  bool sliced = false;  // the reported mode
+  // windowed gather: the nonzeros' slots, sorted within tiles, and their
+  // offsets there
+  WindowGather win;
+  DeviceBuffer slot, pos;
+  // Long rows beside the tiles: their chains (3 ns per nonzero, 176 registers)
+  // run as a launch of their own on `side`, so the tiles keep their registers
+  // and do not wait for the longest chain.  Where the tiles' work is small,
+  // one launch is cheaper than the fork and the join (about 15 us).
+  hipStream_t side = nullptr;
+  hipEvent_t fork_ev = nullptr, join_ev = nullptr;
+  ~gd_spmv_plan() {
+    if (fork_ev) (void)hipEventDestroy(fork_ev);
+    if (join_ev) (void)hipEventDestroy(join_ev);
+    if (side) (void)hipStreamDestroy(side);
+  }
 };
 
 namespace {
 
-int build_sliced(gd_spmv_plan* p) {
-  const int rows = p->rows;
-  p->width = std::max(1, (p->cols + kSlices - 1) / kSlices);
-  int rc = p->soff.alloc(4 * (size_t)kSlices * (rows + 1));
-  if (!rc) rc = p->sbase.alloc(8 * (kSlices + 1));
-  if (!rc) rc = p->Aj_s.alloc(4 * (size_t)p->nnz);
-  if (!rc) rc = p->Ax_s.alloc(4 * (size_t)p->nnz);
-  if (rc) return rc;
-  DeviceBuffer cnt, bad, tmp;
-  rc = cnt.alloc(4 * (size_t)kSlices * (rows + 1));
-  if (!rc) rc = bad.alloc(4);
+// GD_ERR_INVALID unless every row's columns are strictly increasing.
+int check_sorted(const gd_spmv_plan* p) {
+  DeviceBuffer bad;
+  int rc = bad.alloc(4);
   if (rc) return rc;
   GD_HIP_TRY(hipMemsetAsync(bad.ptr, 0, 4, p->stream));
-  GD_HIP_TRY(hipMemsetAsync(cnt.ptr, 0, 4 * (size_t)kSlices * (rows + 1), p->stream));
-  const int g = std::max(1, std::min((rows + 255) / 256, 16384));
-  hipLaunchKernelGGL(slice_count_kernel, dim3(g), dim3(256), 0, p->stream, rows, p->Ap, p->Aj,
-                     p->width, cnt.as<int32_t>(), bad.as<int>());
+  const int g = (int)std::max<int64_t>(1, std::min<int64_t>(((int64_t)p->rows + 15) / 16, 16384));
+  hipLaunchKernelGGL(sorted_rows_kernel, dim3(g), dim3(256), 0, p->stream, p->rows, p->Ap, p->Aj,
+                     bad.as<int>());
   GD_HIP_TRY(hipGetLastError());
   int h_bad = 0;
   GD_HIP_TRY(hipMemcpyAsync(&h_bad, bad.ptr, 4, hipMemcpyDeviceToHost, p->stream));
@@ -213,66 +170,38 @@ int build_sliced(gd_spmv_plan* p) {
     set_error("column-sliced SpMV needs sorted columns within each row");
     return GD_ERR_INVALID;
   }
-  size_t bytes = 0;
-  GD_HIP_TRY(rocprim::exclusive_scan(nullptr, bytes, cnt.as<int32_t>(), p->soff.as<int32_t>(), 0,
-                                     (size_t)rows + 1, rocprim::plus<int32_t>(), p->stream));
-  rc = tmp.alloc(bytes);
-  if (rc) return rc;
-  for (int q = 0; q < kSlices; q++)  // each slice's row offsets from 0
-    GD_HIP_TRY(rocprim::exclusive_scan(tmp.ptr, bytes, cnt.as<int32_t>() + (size_t)q * (rows + 1),
-                                       p->soff.as<int32_t>() + (size_t)q * (rows + 1), 0,
-                                       (size_t)rows + 1, rocprim::plus<int32_t>(), p->stream));
-  std::vector<int32_t> tot(kSlices);
-  for (int q = 0; q < kSlices; q++)
-    GD_HIP_TRY(hipMemcpyAsync(&tot[q], p->soff.as<int32_t>() + (size_t)q * (rows + 1) + rows, 4,
-                              hipMemcpyDeviceToHost, p->stream));
-  GD_HIP_TRY(hipStreamSynchronize(p->stream));
-  std::vector<int64_t> base(kSlices + 1, 0);
-  for (int q = 0; q < kSlices; q++) base[q + 1] = base[q] + tot[q];
-  if (base[kSlices] != p->nnz) {
-    set_error("column-sliced SpMV: slice counts do not add up to nnz");
-    return GD_ERR_INVALID;
-  }
-  GD_HIP_TRY(hipMemcpyAsync(p->sbase.ptr, base.data(), 8 * (kSlices + 1), hipMemcpyHostToDevice,
-                            p->stream));
-  hipLaunchKernelGGL(slice_scatter_kernel<float>, dim3(g), dim3(256), 0, p->stream, rows, p->Ap,
-                     p->Aj, p->Ax, p->width, p->soff.as<int32_t>(), p->sbase.as<int64_t>(),
-                     p->Aj_s.as<int32_t>(), p->Ax_s.as<float>(), 0);
-  GD_HIP_TRY(hipGetLastError());
-  // one row-tile schedule per slice, over that slice's row offsets
-  std::vector<int32_t> h_soff((size_t)kSlices * (rows + 1));
-  GD_HIP_TRY(hipMemcpyAsync(h_soff.data(), p->soff.ptr, 4 * h_soff.size(), hipMemcpyDeviceToHost,
-                            p->stream));
-  GD_HIP_TRY(hipStreamSynchronize(p->stream));
-  std::vector<Tile> all;
-  p->slice_base.assign(base.begin(), base.end());
-  p->slice_first.assign(kSlices, 0);
-  p->slice_long.assign(kSlices, 0);
-  p->slice_rows.assign(kSlices, 0);
-  for (int q = 0; q < kSlices; q++) {
-    p->slice_first[q] = (int)all.size();
-    if (tot[q] == 0) continue;  // no entries: the pass would leave y unchanged
-    Schedule sc;
-    rc = build_schedule(rows, tot[q], h_soff.data() + (size_t)q * (rows + 1), kSpTileNnz,
-                        kTileRows, &sc, kSpTileNnz);
-    if (rc) return rc;
-    std::vector<Tile> row_tiles, longs;
-    for (const Tile& t : sc.tiles) (t.y < 0 ? longs : row_tiles).push_back(t);
-    std::stable_sort(longs.begin(), longs.end(),  // the longest rows start first
-                     [](const Tile& a, const Tile& b) { return a.w - a.z > b.w - b.z; });
-    p->slice_long[q] = (int)longs.size();
-    p->slice_rows[q] = (int)row_tiles.size();
-    all.insert(all.end(), longs.begin(), longs.end());
-    all.insert(all.end(), row_tiles.begin(), row_tiles.end());
-  }
-  rc = p->slice_tiles.alloc(sizeof(Tile) * std::max<size_t>(all.size(), 1));
-  if (rc) return rc;
-  if (!all.empty())
-    GD_HIP_TRY(hipMemcpyAsync(p->slice_tiles.ptr, all.data(), sizeof(Tile) * all.size(),
-                              hipMemcpyHostToDevice, p->stream));
-  GD_HIP_TRY(hipStreamSynchronize(p->stream));
   return GD_OK;
 }
+
+// Windows pay where x exceeds one XCD's 4 MB L2 and every window is filled
+// for at least about as many nonzeros as it holds columns (a piece of the
+// expand pass copies its window into LDS first).
+bool wants_windows(const gd_spmv_plan* p) {
+  return (int64_t)p->cols * 4 > (4 << 20) && p->nnz >= 2 * (int64_t)p->cols &&
+         window_gather_fits(p->cols, p->nnz, (int64_t)p->sched.tiles.size());
+}
+
+int build_windows(gd_spmv_plan* p) {
+  int rc = p->slot.alloc(4 * (size_t)p->nnz);
+  if (!rc) rc = p->pos.alloc(2 * (size_t)p->nnz);
+  if (rc) return rc;
+  std::vector<int2> segs;
+  rc = build_tile_sort(p->sched, kSpTileNnz, p->Aj, p->slot.as<int32_t>(), p->pos.as<uint16_t>(),
+                       p->stream, true, 0, &segs);
+  // long rows stay out: they gather x themselves, beside the expand pass
+  segs.erase(std::remove_if(segs.begin(), segs.end(), [](const int2& s) { return s.y < 0; }),
+             segs.end());
+  int64_t in_tiles = 0;
+  for (const int2& s : segs) in_tiles += s.y;
+  if (!rc)
+    rc = build_window_gather(p->cols, in_tiles, segs, p->slot.as<int32_t>(), p->stream, &p->win);
+  return rc;
+}
+
+// Power-law matrix, 2.5 M rows, 38 M nonzeros, longest row 73,996 (its chain
+// alone 220 us): 261 us; 333 in one launch, whose tiles run at 176 registers.
+// Below 2^22 nonzeros the tiles take less time than the fork and the join.
+constexpr int64_t kForkNnz = 1 << 22;
 
 }  // namespace
 
@@ -319,15 +248,16 @@ int gd_spmv_plan_create_ex(int rows, int cols, int64_t nnz, const int32_t* d_Ap,
       rc = build_schedule(rows, nnz, h_off.data(), kSpTileNnz, kTileRows, &p->sched, kSpTileNnz);
     if (!rc) rc = check_columns(d_Aj, nnz, cols, p->stream);
     if (!rc && nnz > 0 && mode != GD_SPMV_TILES) {
-      // auto: slice when x spans more than one XCD's L2 and rows are short
+      // auto: sliced when x spans more than one XCD's L2 and rows are short
       const bool want = mode == GD_SPMV_SLICED ||
                         ((int64_t)cols * 4 > (4 << 20) && p->sched.max_row_len <= kSeqRow);
       if (want) {
-        rc = build_sliced(p);
+        rc = check_sorted(p);
         if (!rc) p->sliced = true;
-        if (rc && mode == GD_SPMV_AUTO) rc = GD_OK;  // unsorted rows: tile engine
+        if (rc == GD_ERR_INVALID && mode == GD_SPMV_AUTO) rc = GD_OK;  // unsorted rows: tiles
       }
     }
+    if (!rc && wants_windows(p)) rc = build_windows(p);
     if (!rc && nnz == 0) {
       rc = p->dummy_col.alloc(4);
       if (!rc && hipMemsetAsync(p->dummy_col.ptr, 0, 4, p->stream) != hipSuccess) rc = GD_ERR_DEVICE;
@@ -341,7 +271,14 @@ int gd_spmv_plan_create_ex(int rows, int cols, int64_t nnz, const int32_t* d_Ap,
                        [](const Tile& a, const Tile& b) { return a.w - a.z > b.w - b.z; });
       p->n_tiles = (int)row_tiles.size();
       p->n_hubs = (int)longs.size();
-      rc = p->tiles.alloc(sizeof(Tile) * std::max(1, p->n_tiles));
+      if (p->n_hubs && p->n_tiles && nnz >= kForkNnz &&
+          (hipStreamCreateWithFlags(&p->side, hipStreamNonBlocking) != hipSuccess ||
+           hipEventCreateWithFlags(&p->fork_ev, hipEventDisableTiming) != hipSuccess ||
+           hipEventCreateWithFlags(&p->join_ev, hipEventDisableTiming) != hipSuccess)) {
+        set_error("creating the long rows' stream");
+        rc = GD_ERR_DEVICE;
+      }
+      if (!rc) rc = p->tiles.alloc(sizeof(Tile) * std::max(1, p->n_tiles));
       if (!rc) rc = p->long_tiles.alloc(sizeof(Tile) * std::max(1, p->n_hubs));
       hipError_t e2 = hipSuccess;
       if (!rc && p->n_tiles)
@@ -369,82 +306,41 @@ int gd_spmv_plan_run(gd_spmv_plan* p, const float* d_x, float* d_y) {
   GD_CHECK_ARG(p != nullptr, "NULL plan");
   if (p->rows == 0) return GD_OK;
   GD_CHECK_ARG(d_y != nullptr && (p->nnz == 0 || d_x != nullptr), "NULL x / y");
-  if (p->sliced) {
-    const Tile* tl = p->slice_tiles.as<Tile>();
-    for (int q = 0; q < kSlices; q++) {  // slice 0 first: each row's column order
-      const int nl = p->slice_long[q], nr = p->slice_rows[q];
-      if (nl + nr == 0) continue;
-      const Tile* lt = tl + p->slice_first[q];
-      const int32_t* off = p->soff.as<int32_t>() + (size_t)q * (p->rows + 1);
-      const int32_t* aj = p->Aj_s.as<int32_t>() + p->slice_base[q];
-      const float* ax = p->Ax_s.as<float>() + p->slice_base[q];
-      const int em = (int)std::max<int64_t>(p->slice_base[q + 1] - p->slice_base[q] - 1, 0);
-      if (nl)
-        hipLaunchKernelGGL(spmv_pull_kernel<true>, dim3(nl + nr), dim3(kBlock), 0, p->stream,
-                           lt + nl, lt, nl, off, aj, em, ax, d_x, d_y);
-      else
-        hipLaunchKernelGGL(spmv_pull_kernel<false>, dim3(nr), dim3(kBlock), 0, p->stream, lt, lt,
-                           0, off, aj, em, ax, d_x, d_y);
-    }
-    GD_HIP_TRY(hipGetLastError());
-    return GD_OK;
+  const bool fork = p->side != nullptr;
+  auto run = [&](auto kernel, int n_tiles, int n_long, const int32_t* aj, const float* src,
+                 hipStream_t s) {
+    hipLaunchKernelGGL(kernel, dim3(n_tiles + n_long), dim3(kBlock), 0, s, p->tiles.as<Tile>(),
+                       n_tiles, p->long_tiles.as<Tile>(), n_long, p->Ap, aj, p->pos.as<uint16_t>(),
+                       p->e_max, p->Ax, src, d_y);
+  };
+  if (fork) {  // the longest chains start first
+    GD_HIP_TRY(hipEventRecord(p->fork_ev, p->stream));
+    GD_HIP_TRY(hipStreamWaitEvent(p->side, p->fork_ev, 0));
+    run(spmv_pull_kernel<true, false>, 0, p->n_hubs, p->Aj, d_x, p->side);
+    GD_HIP_TRY(hipEventRecord(p->join_ev, p->side));
   }
-  if (p->n_hubs)
-    hipLaunchKernelGGL(spmv_pull_kernel<true>, dim3(p->n_hubs + p->n_tiles), dim3(kBlock), 0,
-                       p->stream, p->tiles.as<Tile>(), p->long_tiles.as<Tile>(), p->n_hubs, p->Ap,
-                       p->Aj, p->e_max, p->Ax, d_x, d_y);
-  else if (p->n_tiles)
-    hipLaunchKernelGGL(spmv_pull_kernel<false>, dim3(p->n_tiles), dim3(kBlock), 0, p->stream,
-                       p->tiles.as<Tile>(), p->long_tiles.as<Tile>(), 0, p->Ap, p->Aj, p->e_max,
-                       p->Ax, d_x, d_y);
+  const int n_long = fork ? 0 : p->n_hubs;
+  if (p->win.on()) {
+    if (n_long) run(spmv_pull_kernel<true, false>, 0, n_long, p->Aj, d_x, p->stream);
+    hipLaunchKernelGGL(spmv_expand_kernel, dim3(p->win.n_pieces), dim3(kExpandBlock), 0, p->stream,
+                       d_x, p->cols, p->win.pieces.as<int4>(), p->win.sid.as<uint16_t>(),
+                       p->win.stage.as<float>());
+    run(spmv_pull_kernel<false, true>, p->n_tiles, 0, p->slot.as<int32_t>(),
+        p->win.stage.as<float>(), p->stream);
+  } else if (n_long) {
+    run(spmv_pull_kernel<true, false>, p->n_tiles, n_long, p->Aj, d_x, p->stream);
+  } else if (p->n_tiles) {
+    run(spmv_pull_kernel<false, false>, p->n_tiles, 0, p->Aj, d_x, p->stream);
+  }
+  if (fork) GD_HIP_TRY(hipStreamWaitEvent(p->stream, p->join_ev, 0));
   GD_HIP_TRY(hipGetLastError());
   return GD_OK;
 }
 
 int gd_spmv_plan_refresh_values(gd_spmv_plan* p) {
   GD_CHECK_ARG(p != nullptr, "NULL plan");
-  if (!p->sliced) return GD_OK;  // the tile engine reads the caller's values directly
-  const int g = std::max(1, std::min((p->rows + 255) / 256, 16384));
-  hipLaunchKernelGGL(slice_scatter_kernel<float>, dim3(g), dim3(256), 0, p->stream, p->rows, p->Ap,
-                     p->Aj, p->Ax, p->width, p->soff.as<int32_t>(), p->sbase.as<int64_t>(),
-                     p->Aj_s.as<int32_t>(), p->Ax_s.as<float>(), 1);
-  GD_HIP_TRY(hipGetLastError());
-  return GD_OK;
+  return GD_OK;  // every mode reads the caller's values directly
 }
-
-}  // extern "C"
-
-float* gd::spmv_sliced_values(gd_spmv_plan* p) {
-  return (p && p->sliced) ? p->Ax_s.as<float>() : nullptr;
-}
-
-int gd::spmv_slice_order(gd_spmv_plan* p, const int32_t* d_in, int32_t* d_out) {
-  GD_CHECK_ARG(p != nullptr && p->sliced, "not a sliced SpMV plan");
-  if (p->nnz == 0) return GD_OK;
-  GD_CHECK_ARG(d_in && d_out, "NULL payload");
-  const int g = std::max(1, std::min((p->rows + 255) / 256, 16384));
-  hipLaunchKernelGGL(slice_scatter_kernel<int32_t>, dim3(g), dim3(256), 0, p->stream, p->rows,
-                     p->Ap, p->Aj, d_in, p->width, p->soff.as<int32_t>(), p->sbase.as<int64_t>(),
-                     nullptr, d_out, 1);
-  GD_HIP_TRY(hipGetLastError());
-  return GD_OK;
-}
-
-int gd::spmv_sliced_gather(gd_spmv_plan* p, const float* d_x, float* d_Xs) {
-  GD_CHECK_ARG(p != nullptr && p->sliced, "not a sliced SpMV plan");
-  if (p->nnz == 0) return GD_OK;
-  GD_CHECK_ARG(d_x && d_Xs, "NULL array");
-  int64_t most = 0;
-  for (int q = 0; q < kSlices; q++)
-    most = std::max<int64_t>(most, p->slice_base[q + 1] - p->slice_base[q]);
-  const int64_t chunks = (most + 256 * kGatherPT - 1) / (256 * kGatherPT);
-  hipLaunchKernelGGL(slice_gather_kernel, dim3((unsigned)(kSlices * chunks)), dim3(256), 0,
-                     p->stream, p->sbase.as<int64_t>(), p->Aj_s.as<int32_t>(), d_x, d_Xs);
-  GD_HIP_TRY(hipGetLastError());
-  return GD_OK;
-}
-
-extern "C" {
 
 int gd_spmv_plan_mode(const gd_spmv_plan* p) {
   return p == nullptr ? -1 : (p->sliced ? GD_SPMV_SLICED : GD_SPMV_TILES);

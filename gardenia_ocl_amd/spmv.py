@@ -48,9 +48,10 @@ class SpmvPlan:
     MODES = {"auto": 0, "tiles": 1, "sliced": 2}
 
     def __init__(self, Ap, Aj, Ax, num_cols=None, stream=None, mode="tiles"):
-        """mode: "tiles" (the tile engine), "sliced" (one tile-engine pass per
-        column slice of x sized for an XCD's L2, sorted rows only), "auto"
-        (sliced when x exceeds one XCD's L2 and rows are short)."""
+        """mode: "tiles" (any column order), "sliced" (sorted rows only), "auto"
+        (sliced when x exceeds one XCD's L2 and rows are short and sorted).
+        All give the same results; where x exceeds one XCD's L2 it is gathered
+        through windows, in a buffer that the plan's runs share."""
         import torch
 
         for t, dt in ((Ap, torch.int32), (Aj, torch.int32), (Ax, torch.float32)):
@@ -71,7 +72,8 @@ class SpmvPlan:
         self.mode = {1: "tiles", 2: "sliced"}[N.lib().gd_spmv_plan_mode(h)]
 
     def refresh_values(self):
-        """Re-read Ax after it changed (needed by the sliced mode)."""
+        """To be called after Ax changed (the sliced mode's contract; every mode
+        reads Ax itself on each run)."""
         N.call("gd_spmv_plan_refresh_values", self._h)
 
     def info(self) -> dict:

@@ -345,19 +345,17 @@ int gd_spmv_plan_info(const gd_spmv_plan *plan, int64_t *n_tiles, int64_t *n_hub
 
 int gd_spmv_plan_destroy(gd_spmv_plan *plan);
 
-/* SpMV execution modes.
- *   GD_SPMV_TILES   the tile engine over the caller's CSR (any matrix, any
- *                   row order; bit-identical to the reference).
- *   GD_SPMV_SLICED  columns split into 8 slices over a slice-major copy of the
- *                   matrix; one tile-engine pass per slice, slice 0 first,
- *                   adds each row's slice entries onto y in column order (the
- *                   pass's x gathers stay in one slice, which every XCD's L2
- *                   holds).  Needs sorted columns per row; bit-identical to
- *                   the reference for every row.  The copy holds the values:
- *                   call gd_spmv_plan_refresh_values after changing d_Ax.
- *   GD_SPMV_AUTO    SLICED when x spans more than one XCD's L2 (cols*4 > 4 MB),
- *                   every row has <= 64 nonzeros and the columns are sorted,
- *                   else TILES. */
+/* SpMV modes.  All run the tile engine over the caller's CSR, every row in
+ * CSR order, bit-identical to the reference; where x spans more than one
+ * XCD's L2 (cols*4 > 4 MB) and nnz >= 2*cols, x is gathered through windows
+ * (the plan then holds 12 bytes per nonzero: slots, tile offsets, the expanded
+ * x and its 16-bit sources).  A plan's runs share that buffer: they must not
+ * overlap on the GPU (they run in order on the plan's stream).
+ *   GD_SPMV_TILES   any matrix, any column order.
+ *   GD_SPMV_SLICED  needs sorted columns per row (GD_ERR_INVALID otherwise).
+ *                   Call gd_spmv_plan_refresh_values after changing d_Ax.
+ *   GD_SPMV_AUTO    SLICED when cols*4 > 4 MB, every row has <= 64 nonzeros and
+ *                   the columns are sorted, else TILES. */
 enum { GD_SPMV_AUTO = 0, GD_SPMV_TILES = 1, GD_SPMV_SLICED = 2 };
 
 int gd_spmv_plan_create_ex(int num_rows, int num_cols, int64_t nnz, const int32_t *d_Ap,
@@ -367,7 +365,8 @@ int gd_spmv_plan_create_ex(int num_rows, int num_cols, int64_t nnz, const int32_
 /* Mode the plan runs in (GD_SPMV_TILES or GD_SPMV_SLICED), -1 for NULL. */
 int gd_spmv_plan_mode(const gd_spmv_plan *plan);
 
-/* Re-read d_Ax into the plan's sliced copy (no-op for the tile mode). */
+/* To be called after d_Ax changed under a SLICED plan.  Every mode reads d_Ax
+ * itself on each run, so there is nothing to copy. */
 int gd_spmv_plan_refresh_values(gd_spmv_plan *plan);
 
 /* One-shot form of SpmvSolver with host arrays (src/spmv/spmv.h:29); mode AUTO. */
