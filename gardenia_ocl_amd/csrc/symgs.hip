@@ -12,19 +12,28 @@
 // when the plan is built), so updating them in parallel equals the
 // reference's sequential loop over the color, bit for bit.
 //
-// Layout in HBM (built once per plan).  The rows are gathered in sweep order
-// into a private CSR without diagonal entries: row i of the plan is row
-// indices[color_offsets[0] + i] of the matrix, so every color is a contiguous
-// range of plan rows and of edges, with diag[i] and orig[i] beside it.  Each
-// color is cut into the pull engine's LDS row tiles (rows of <= 64 off-diagonal
-// entries, summed by their owner thread in CSR order) and whole-row tiles
-// (longer rows: a workgroup gathers each 2048-entry chunk into LDS while one
-// lane adds the previous chunk in order), with a SymGS gather
-// (x[col] * val) and epilogue (the row update).  One color = one launch of
-// symgs_color_kernel; the stream orders the colors.
+// Layout in HBM (built once per plan).  Every color is a contiguous range of
+// plan rows, its rows of at most kSeqRow (64) off-diagonal entries first, by
+// falling length, then its longer rows.
+//
+// Short rows: slices of up to 64 rows (one wavefront, one lane a row), the
+// entries of a slice stored in 16-byte groups across its rows (group k of lane
+// l at off + k * rows + l), so a wavefront reads 1 KB of consecutive entries
+// with each load and every lane adds its own row in CSR order in a register:
+// no LDS, no barrier, no per-row offsets.  A group is two {column, value}
+// pairs; where all rows of the slice are of one length and the k-th entry of
+// each lies the same number of columns from its row (interior rows of a
+// stencil), it is four values, and the distances are stored once a slice.
+// Sorting by length keeps the padding to a group a row plus what the few
+// slices that straddle a length change hold; a slice of fewer rows is stored
+// that narrow, so a color of one row costs one row.
+//
+// Long rows: CSR, one workgroup each (hub_chain_sum: the workgroup gathers a
+// chunk into LDS while one lane adds the previous one in order).
+//
+// One color = one launch of symgs_color_kernel; the stream orders the colors.
 
 #include <hip/hip_runtime.h>
-#include <rocprim/device/device_scan.hpp>
 
 #include <algorithm>
 #include <chrono>
@@ -34,12 +43,50 @@
 #include "gardenia_hip.h"
 #include "gd_common.h"
 #include "pull_engine.h"
-#include "pull_iter.h"
 
 namespace gd {
 namespace {
 
-constexpr int kSgIPT = 8;  // edges per thread per row tile (tile = 2048 edges)
+constexpr int kSgXcds = 8;
+constexpr int64_t kSgDeltaMax = (1ll << 31) - 128;  // distances a plan stores at most
+
+// Up to 64 rows of one color.  A general slice (delta < 0) has `n` pairs of
+// entries a row at ent[off ...]; a uniform one, where the k-th entry of every
+// row lies the same number of columns from its row, `n` float4 of values
+// there and the `len` column distances at delta[delta ...].
+struct Slice {
+  int row0;    // first plan row
+  int n_rows;  // 1 .. 64
+  int n;
+  int len;  // entries of the longest row
+  int64_t off;
+  int delta;
+  int pad;
+};
+
+// One plan row.
+struct RowRec {
+  float diag;
+  int orig;  // its matrix row
+  int len;   // off-diagonal entries
+  int pad;
+};
+static_assert(sizeof(RowRec) == 16 && sizeof(Slice) == 32, "plan records");
+
+struct SymgsArgs {
+  float* x;
+  const float* __restrict__ b;
+  const RowRec* __restrict__ rows;
+  const Slice* __restrict__ slices;
+  int n_slices;
+  const int4* __restrict__ ent;  // {column, value, column, value} or four values
+  const int* __restrict__ delta;
+  const Tile* __restrict__ hubs;  // long rows: {plan row, -, first entry, end}
+  int n_hubs;
+  const int32_t* __restrict__ col;  // long rows
+  const float* __restrict__ val;
+  int e_max;
+};
 
 struct SymgsGather {
   const float* __restrict__ x;
@@ -48,74 +95,122 @@ struct SymgsGather {
   __device__ __forceinline__ float value(int e, int u) const { return x[u] * val[e]; }
 };
 
-struct SymgsEpilogue {
-  float* x;
-  const float* __restrict__ b;
-  const float* __restrict__ diag;
-  const int32_t* __restrict__ orig;
-  struct Pre {
-    float d;
-    float bv;
-    int r;
-  };
-  __device__ __forceinline__ Pre pre(int v) const {
-    const int r = orig[v];
-    return Pre{diag[v], b[r], r};
-  }
-  __device__ __forceinline__ float init(const Pre&) const { return 0.0f; }
-  // if (diag != 0) x[inew] = (b[inew] - rsum) / diag   (verifier.cc:63)
-  __device__ __forceinline__ double finish(int /*v*/, float rsum, const Pre& p) const {
-    if (p.d != 0.0f) x[p.r] = (p.bv - rsum) / p.d;
-    return 0.0;
-  }
-};
+// if (diag != 0) x[inew] = (b[inew] - rsum) / diag   (verifier.cc:63)
+__device__ __forceinline__ void row_update(const SymgsArgs& a, const RowRec& r, float bv,
+                                           float rsum) {
+  if (r.diag != 0.0f) a.x[r.orig] = (bv - rsum) / r.diag;
+}
 
-struct SymgsPolicy {
-  struct Args {
-    float* x;
-    const float* b;
-    const float* val;
-    const float* diag;
-    const int32_t* orig;
-  };
-  template <int NT>
-  __device__ static SymgsGather gather(const Args& a, int) {
-    return SymgsGather{a.x, a.val};
+// One general slice on one wavefront, two pairs (four entries) a step, the next
+// step's in flight.  More a step is slower (8 pairs: 261 us where 2 take 234,
+// a 27-point stencil of 97^3): neighbouring entries of a row often share a line
+// of x, which the first load of it must have brought in before the next asks.
+// The entries a lane reads past its row are the slice's padding or, past the
+// slice's end, its last pair again: their terms are replaced by -0.0, which
+// changes no sum.
+__device__ __forceinline__ float general_sum(const SymgsArgs& a, const Slice& sl,
+                                             const RowRec& r, int lane) {
+  constexpr int kP = 2;
+  const int4* __restrict__ e = a.ent + sl.off + lane;
+  const int last = sl.n - 1;
+  float sum = 0.0f;
+  int4 cur[kP], nxt[kP];
+  if (last >= 0) {
+#pragma unroll
+    for (int j = 0; j < kP; j++) cur[j] = e[(int64_t)min(j, last) * sl.n_rows];
   }
-  template <int NT>
-  __device__ static SymgsEpilogue epilogue(const Args& a, int) {
-    return SymgsEpilogue{a.x, a.b, a.diag, a.orig};
+  for (int k = 0; k <= last; k += kP) {
+    float v[2 * kP];
+#pragma unroll
+    for (int j = 0; j < kP; j++) {
+      v[2 * j] = a.x[cur[j].x];
+      v[2 * j + 1] = a.x[cur[j].z];
+    }
+#pragma unroll
+    for (int j = 0; j < kP; j++) nxt[j] = e[(int64_t)min(k + kP + j, last) * sl.n_rows];
+    const int left = r.len - 2 * k;
+#pragma unroll
+    for (int j = 0; j < kP; j++) {
+      const float t0 = v[2 * j] * __int_as_float(cur[j].y);
+      const float t1 = v[2 * j + 1] * __int_as_float(cur[j].w);
+      sum += 2 * j < left ? t0 : -0.0f;
+      sum += 2 * j + 1 < left ? t1 : -0.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < kP; j++) cur[j] = nxt[j];
   }
-};
+  return sum;
+}
 
+// One uniform slice: 4 bytes an entry instead of 8, the columns from scalar
+// registers.  Padding distances are 0.  27-point stencil, two sweeps: 97^3 212
+// us (general slices 234, LDS row tiles over a CSR 322), 128^3 382 (499, 598):
+// 12.5 MB of values a color at 97^3, most of them from the Infinity Cache, in
+// 6.6 us, about 2.5 of which is the launch.  Bound by the gathers of x: two or
+// four groups of values a step, in flight together, cost 220 and 226 us.
+__device__ __forceinline__ float uniform_sum(const SymgsArgs& a, const Slice& sl,
+                                             const RowRec& r, int lane) {
+  const float4* __restrict__ e = reinterpret_cast<const float4*>(a.ent) + sl.off + lane;
+  const int4* __restrict__ d = reinterpret_cast<const int4*>(a.delta + sl.delta);
+  float sum = 0.0f;
+  float4 cur = e[0];
+  for (int k = 0; k < sl.n; k++) {
+    const int4 c = d[k];
+    const float x0 = a.x[r.orig + c.x], x1 = a.x[r.orig + c.y], x2 = a.x[r.orig + c.z],
+                x3 = a.x[r.orig + c.w];
+    const float4 nxt = e[(int64_t)min(k + 1, sl.n - 1) * sl.n_rows];
+    const int left = sl.len - 4 * k;
+    sum += x0 * cur.x;
+    sum += 1 < left ? x1 * cur.y : -0.0f;
+    sum += 2 < left ? x2 * cur.z : -0.0f;
+    sum += 3 < left ? x3 * cur.w : -0.0f;
+    cur = nxt;
+  }
+  return sum;
+}
 
-// One color in one launch: workgroups [0, n_hub_tiles) add one long row each
-// (hub_chain_sum), the rest one LDS row tile each (owner thread per row, in
-// order).  Long rows first: they take longest.  LONG = false (colors without
-// long rows) leaves the long-row code, and its registers, out of the kernel.
-template <bool LONG>
-__global__ __launch_bounds__(kBlock) void symgs_color_kernel(const SymgsPolicy::Args a,
-                                                             const IterArgs it) {
-  // a row tile's LDS, or a long row's two chunk buffers + the broadcast sum
-  static_assert(sizeof(RowTileLds<kSgIPT>) >= (2 * kHubChunk + 1) * sizeof(float), "LDS union");
-  __shared__ __align__(16) unsigned char smem[sizeof(RowTileLds<kSgIPT>)];
-  RowTileLds<kSgIPT>& lds = *reinterpret_cast<RowTileLds<kSgIPT>*>(smem);
-  float* const buf = reinterpret_cast<float*>(smem);
-  const auto g = SymgsPolicy::gather<0>(a, 0);
-  const auto e = SymgsPolicy::epilogue<0>(a, 0);
+__device__ __forceinline__ void slice_rows(const SymgsArgs& a, const Slice& sl, int lane) {
+  if (lane >= sl.n_rows) return;
+  const RowRec r = a.rows[sl.row0 + lane];
+  const float bv = a.b[r.orig];
+  row_update(a, r, bv, sl.delta >= 0 ? uniform_sum(a, sl, r, lane) : general_sum(a, sl, r, lane));
+}
+
+// The slice of workgroup b: the slices in 8 equal runs, one an XCD, since
+// neighbouring rows share x lines.
+__device__ __forceinline__ int xcd_slice(int b, int n) {
+  const int xcd = b % kSgXcds;
+  return xcd * (n / kSgXcds) + min(xcd, n % kSgXcds) + b / kSgXcds;
+}
+
+// One color in one launch, of wavefront-sized workgroups, one slice each:
+// they spread evenly over the SIMDs however few there are (256-thread
+// workgroups of four slices: 97^3 274 us, 40^3 173; these: 261 and 106).
+__global__ __launch_bounds__(kWave) void symgs_color_kernel(const SymgsArgs a) {
+  slice_rows(a, a.slices[xcd_slice(blockIdx.x, a.n_slices)], threadIdx.x);
+}
+
+// The same for a color with long rows: workgroups [0, n_hubs) add one long row
+// each (hub_chain_sum), the rest take four slices each.  Long rows first: they
+// take longest.
+__global__ __launch_bounds__(kBlock) void symgs_long_kernel(const SymgsArgs a) {
+  __shared__ __align__(16) float buf[2 * kHubChunk + 4];
   const int b = blockIdx.x;
-  if (LONG && b < it.n_hub_tiles) {
-    const Tile t = it.hub_tiles[b];
-    const auto pre = e.pre(t.x);
+  if (b < a.n_hubs) {
+    const Tile t = a.hubs[b];
+    const RowRec r = a.rows[t.x];
+    const float bv = a.b[r.orig];
     // 16 float4 LDS reads ahead: the chains bound these sweeps (8 ahead: 9% slower)
-    const float rsum = hub_chain_sum<16, false>(it.col, nullptr, it.e_max, t.z, t.w - t.z, g, 0.0f,
-                                               buf, buf + kHubChunk, buf + 2 * kHubChunk);
-    if (threadIdx.x == 0) (void)e.finish(t.x, rsum, pre);
-  } else {
-    const Tile t = it.tiles[b - it.n_hub_tiles];
-    (void)row_tile<kSgIPT, false, false>(it.off, it.col, nullptr, it.e_max, t.x, t.y, t.z,
-                                         t.w - t.z, g, e, lds);
+    const float rsum =
+        hub_chain_sum<16, false>(a.col, nullptr, a.e_max, t.z, t.w - t.z,
+                                 SymgsGather{a.x, a.val}, 0.0f, buf, buf + kHubChunk,
+                                 buf + 2 * kHubChunk);
+    if (threadIdx.x == 0) row_update(a, r, bv, rsum);
+    return;
   }
+  const int s = __builtin_amdgcn_readfirstlane((b - a.n_hubs) * (kBlock / kWave) +
+                                               (int)threadIdx.x / kWave);
+  if (s < a.n_slices) slice_rows(a, a.slices[s], threadIdx.x % kWave);
 }
 
 #define SG_LOOP(i, n) \
@@ -148,34 +243,123 @@ __global__ void sg_rows_kernel(int n_p, const int32_t* __restrict__ idx, int m,
   }
 }
 
-// Off-diagonal count, last diagonal value, original row.
+// Off-diagonal count and last diagonal value of plan input row i; a proper
+// coloring joins no two rows of one color by an off-diagonal entry.
 __global__ void sg_count_kernel(int n_p, const int32_t* __restrict__ idx,
                                 const int32_t* __restrict__ Ap, const int32_t* __restrict__ Aj,
-                                const float* __restrict__ Ax, int32_t* __restrict__ len,
-                                float* __restrict__ diag, int32_t* __restrict__ orig) {
+                                const float* __restrict__ Ax,
+                                const int32_t* __restrict__ color_of, int32_t* __restrict__ len,
+                                float* __restrict__ diag, int* __restrict__ bad) {
   SG_LOOP(i, n_p) {
     const int r = idx[i];
-    int n = 0;
+    const int c = color_of[r];
+    int n = 0, f = 0;
     float d = 0.0f;
     for (int k = Ap[r]; k < Ap[r + 1]; k++) {
-      if (Aj[k] == r)
+      const int j = Aj[k];
+      if (j == r) {
         d = Ax[k];
-      else
+      } else {
         n++;
+        f |= color_of[j] == c;
+      }
     }
     len[i] = n;
     diag[i] = d;
-    orig[i] = r;
+    if (f) atomicOr(bad, 4);
   }
 }
 
-__global__ void sg_fill_kernel(int n_p, const int32_t* __restrict__ idx,
-                               const int32_t* __restrict__ Ap, const int32_t* __restrict__ Aj,
-                               const float* __restrict__ Ax, const int32_t* __restrict__ off,
-                               int32_t* __restrict__ col, float* __restrict__ val) {
-  SG_LOOP(i, n_p) {
-    const int r = idx[i];
-    int o = off[i];
+// Plan row q is input row order[q].
+__global__ void sg_rec_kernel(int n_p, const int32_t* __restrict__ order,
+                              const int32_t* __restrict__ idx, const int32_t* __restrict__ len,
+                              const float* __restrict__ diag, RowRec* __restrict__ rows) {
+  SG_LOOP(q, n_p) {
+    const int i = order[q];
+    rows[q] = RowRec{diag[i], idx[i], len[i], 0};
+  }
+}
+
+// The off-diagonal entries of matrix row r, in CSR order: next() -> one more.
+struct RowEntries {
+  const int32_t* __restrict__ Aj;
+  const float* __restrict__ Ax;
+  int r, k, end;
+  __device__ __forceinline__ bool next(int* c, float* v) {
+    while (k < end && Aj[k] == r) k++;
+    if (k >= end) return false;
+    *c = Aj[k];
+    *v = Ax[k];
+    k++;
+    return true;
+  }
+};
+
+// One wavefront a slice whose rows are all of one length (the others have
+// delta < 0 already): uniform, then distances to delta[slices[s].delta ...],
+// or delta = -1.
+__global__ void sg_uniform_kernel(int n_slices, Slice* __restrict__ slices,
+                                  const RowRec* __restrict__ rows, const int32_t* __restrict__ Ap,
+                                  const int32_t* __restrict__ Aj, const float* __restrict__ Ax,
+                                  int* __restrict__ delta) {
+  const int lane = threadIdx.x % kWave;
+  for (int64_t s = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave; s < n_slices;
+       s += (int64_t)gridDim.x * blockDim.x / kWave) {
+    const Slice sl = slices[s];
+    if (sl.delta < 0) continue;
+    const int r = rows[sl.row0 + min(lane, sl.n_rows - 1)].orig;
+    RowEntries e{Aj, Ax, r, Ap[r], Ap[r + 1]};
+    bool same = true;
+    for (int k = 0; k < sl.len; k++) {
+      int c = r;
+      float v = 0.0f;
+      e.next(&c, &v);
+      const int d = c - r;
+      same = same && d == __builtin_amdgcn_readfirstlane(d);
+      if (lane == 0) delta[sl.delta + k] = d;
+    }
+    if (__ballot(!same) && lane == 0) slices[s].delta = -1;
+  }
+}
+
+// The entries of slice s, by one wavefront; pads repeat the row's own column.
+__global__ void sg_slice_fill_kernel(int n_slices, const Slice* __restrict__ slices,
+                                     const RowRec* __restrict__ rows,
+                                     const int32_t* __restrict__ Ap,
+                                     const int32_t* __restrict__ Aj, const float* __restrict__ Ax,
+                                     int4* __restrict__ ent) {
+  const int lane = threadIdx.x % kWave;
+  for (int64_t s = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave; s < n_slices;
+       s += (int64_t)gridDim.x * blockDim.x / kWave) {
+    const Slice sl = slices[s];
+    if (lane >= sl.n_rows) continue;
+    const int r = rows[sl.row0 + lane].orig;
+    RowEntries e{Aj, Ax, r, Ap[r], Ap[r + 1]};
+    for (int p = 0; p < sl.n; p++) {
+      int c[4] = {r, r, r, r};
+      float v[4] = {};
+      const int n = sl.delta >= 0 ? 4 : 2;
+#pragma unroll
+      for (int h = 0; h < 4; h++)
+        if (h < n) e.next(&c[h], &v[h]);
+      int4 q = make_int4(c[0], __float_as_int(v[0]), c[1], __float_as_int(v[1]));
+      if (n == 4)
+        q = make_int4(__float_as_int(v[0]), __float_as_int(v[1]), __float_as_int(v[2]),
+                      __float_as_int(v[3]));
+      ent[sl.off + (int64_t)p * sl.n_rows + lane] = q;
+    }
+  }
+}
+
+// The entries of the long rows, one thread a row.
+__global__ void sg_hub_fill_kernel(int n_hubs, const Tile* __restrict__ hubs,
+                                   const RowRec* __restrict__ rows,
+                                   const int32_t* __restrict__ Ap,
+                                   const int32_t* __restrict__ Aj, const float* __restrict__ Ax,
+                                   int32_t* __restrict__ col, float* __restrict__ val) {
+  SG_LOOP(h, n_hubs) {
+    const int r = rows[hubs[h].x].orig;
+    int o = hubs[h].z;
     for (int k = Ap[r]; k < Ap[r + 1]; k++) {
       const int j = Aj[k];
       if (j != r) {
@@ -184,18 +368,6 @@ __global__ void sg_fill_kernel(int n_p, const int32_t* __restrict__ idx,
         o++;
       }
     }
-  }
-}
-
-// Proper coloring: no off-diagonal entry joins two rows of one color.
-__global__ void sg_proper_kernel(int n_p, const int32_t* __restrict__ off,
-                                 const int32_t* __restrict__ col, const int32_t* __restrict__ orig,
-                                 const int32_t* __restrict__ color_of, int* __restrict__ bad) {
-  SG_LOOP(i, n_p) {
-    const int c = color_of[orig[i]];
-    int f = 0;
-    for (int k = off[i]; k < off[i + 1]; k++) f |= color_of[col[k]] == c;
-    if (f) atomicOr(bad, 4);
   }
 }
 
@@ -209,10 +381,10 @@ struct gd_symgs_plan {
   int n_p = 0;  // rows swept (color_offsets[C] - color_offsets[0])
   int64_t nnz_p = 0;  // off-diagonal entries of those rows
   int n_colors = 0;
-  int ipt = kSgIPT;
+  int64_t hub_nnz = 0;  // those of the long rows
   double plan_ms = 0.0;
-  DeviceBuffer off, col, val, diag, orig, tiles, hubs;
-  std::vector<int> tile_begin, hub_begin;  // per color, n_colors + 1 entries
+  DeviceBuffer rows, slices, ent, delta, hubs, col, val;
+  std::vector<int> slice_begin, hub_begin;  // per color, n_colors + 1 entries
   int max_row_len = 0;
 };
 
@@ -239,129 +411,156 @@ int plan_build(gd_symgs_plan* p, int m, int64_t nnz, const int32_t* d_Ap, const 
     GD_CHECK_ARG(h[0] == 0 && (int64_t)h[m] == nnz, "Ap[0] must be 0 and Ap[m] must equal nnz");
     for (int i = 0; i < m; i++) GD_CHECK_ARG(h[i + 1] >= h[i], "Ap must be non-decreasing");
   }
-  const size_t np1 = (size_t)n_p + 1;
-  DeviceBuffer d_co, color_of, bad, len;
+  const size_t np = (size_t)std::max(n_p, 1);
+  DeviceBuffer d_co, color_of, bad, len, diag, order;
   rc = d_co.alloc(4 * ((size_t)C + 1));
   if (!rc) rc = color_of.alloc(4 * (size_t)std::max(m, 1));
   if (!rc) rc = bad.alloc(sizeof(int));
-  if (!rc) rc = len.alloc(4 * np1);
-  if (!rc) rc = p->off.alloc(4 * np1);
-  if (!rc) rc = p->diag.alloc(4 * std::max<size_t>(n_p, 1));
-  if (!rc) rc = p->orig.alloc(4 * std::max<size_t>(n_p, 1));
+  if (!rc) rc = len.alloc(4 * np);
+  if (!rc) rc = diag.alloc(4 * np);
+  if (!rc) rc = order.alloc(4 * np);
+  if (!rc) rc = p->rows.alloc(sizeof(RowRec) * np);
   if (rc) return rc;
   GD_HIP_TRY(hipMemcpyAsync(d_co.ptr, co, 4 * ((size_t)C + 1), hipMemcpyHostToDevice, s));
   GD_HIP_TRY(hipMemsetAsync(color_of.ptr, 0xff, 4 * (size_t)std::max(m, 1), s));  // -1
   GD_HIP_TRY(hipMemsetAsync(bad.ptr, 0, sizeof(int), s));
-  GD_HIP_TRY(hipMemsetAsync(len.ptr, 0, 4 * np1, s));
   int h_bad = 0;
+  std::vector<int32_t> h_len(n_p);
+  const int32_t* idx = n_p > 0 ? d_idx + co[0] : nullptr;
   if (n_p > 0) {
-    hipLaunchKernelGGL(sg_rows_kernel, dim3(sg_grid(n_p)), dim3(256), 0, s, n_p, d_idx + co[0], m,
+    hipLaunchKernelGGL(sg_rows_kernel, dim3(sg_grid(n_p)), dim3(256), 0, s, n_p, idx, m,
                        d_co.as<int32_t>(), C, color_of.as<int32_t>(), bad.as<int>());
     GD_HIP_TRY(hipGetLastError());
     rc = read_flag(bad, s, &h_bad);
     if (rc) return rc;
     GD_CHECK_ARG(!(h_bad & 1), "indices: row outside [0, m)");
     GD_CHECK_ARG(!(h_bad & 2), "indices: a row is listed more than once");
-    hipLaunchKernelGGL(sg_count_kernel, dim3(sg_grid(n_p)), dim3(256), 0, s, n_p, d_idx + co[0],
-                       d_Ap, d_Aj, d_Ax, len.as<int32_t>(), p->diag.as<float>(),
-                       p->orig.as<int32_t>());
-    GD_HIP_TRY(hipGetLastError());
-  }
-  {
-    size_t tb = 0;
-    GD_HIP_TRY(rocprim::exclusive_scan(nullptr, tb, len.as<int32_t>(), p->off.as<int32_t>(), 0,
-                                       (size_t)np1, rocprim::plus<int32_t>(), s));
-    DeviceBuffer tmp;
-    rc = tmp.alloc(std::max<size_t>(tb, 1));
-    if (rc) return rc;
-    GD_HIP_TRY(rocprim::exclusive_scan(tmp.ptr, tb, len.as<int32_t>(), p->off.as<int32_t>(), 0,
-                                       (size_t)np1, rocprim::plus<int32_t>(), s));
-    GD_HIP_TRY(hipStreamSynchronize(s));
-  }
-  std::vector<int32_t> h_off(np1);
-  GD_HIP_TRY(hipMemcpyAsync(h_off.data(), p->off.ptr, 4 * np1, hipMemcpyDeviceToHost, s));
-  GD_HIP_TRY(hipStreamSynchronize(s));
-  p->nnz_p = h_off[n_p];
-  const size_t ne = (size_t)std::max<int64_t>(p->nnz_p, 1);
-  rc = p->col.alloc(4 * ne);
-  if (!rc) rc = p->val.alloc(4 * ne);
-  if (rc) return rc;
-  GD_HIP_TRY(hipMemsetAsync(p->col.ptr, 0, 4 * ne, s));  // the 1-element dummy when empty
-  GD_HIP_TRY(hipMemsetAsync(p->val.ptr, 0, 4 * ne, s));
-  if (n_p > 0) {
-    hipLaunchKernelGGL(sg_fill_kernel, dim3(sg_grid(n_p)), dim3(256), 0, s, n_p, d_idx + co[0],
-                       d_Ap, d_Aj, d_Ax, p->off.as<int32_t>(), p->col.as<int32_t>(),
-                       p->val.as<float>());
-    hipLaunchKernelGGL(sg_proper_kernel, dim3(sg_grid(n_p)), dim3(256), 0, s, n_p,
-                       p->off.as<int32_t>(), p->col.as<int32_t>(), p->orig.as<int32_t>(),
-                       color_of.as<int32_t>(), bad.as<int>());
+    hipLaunchKernelGGL(sg_count_kernel, dim3(sg_grid(n_p)), dim3(256), 0, s, n_p, idx, d_Ap, d_Aj,
+                       d_Ax, color_of.as<int32_t>(), len.as<int32_t>(), diag.as<float>(),
+                       bad.as<int>());
     GD_HIP_TRY(hipGetLastError());
     rc = read_flag(bad, s, &h_bad);
     if (rc) return rc;
     GD_CHECK_ARG(!(h_bad & 4), "coloring is not proper: an off-diagonal entry joins two rows of one color");
+    GD_HIP_TRY(hipMemcpyAsync(h_len.data(), len.ptr, 4 * (size_t)n_p, hipMemcpyDeviceToHost, s));
+    GD_HIP_TRY(hipStreamSynchronize(s));
   }
-  // Per-color schedules: LDS row tiles and whole-row exact tiles (rows of
-  // more than kSeqRow off-diagonal entries), in plan-row / edge coordinates.
-  std::vector<Tile> all_tiles, all_hubs;
-  p->tile_begin.assign(1, 0);
+  // Per color: short rows by falling length (stable, so neighbours of one
+  // length stay neighbours), cut into slices; long rows, the longest first
+  // (the color lasts as long as its longest row).
+  std::vector<int32_t> h_order(n_p);
+  std::vector<Slice> slices;
+  std::vector<Tile> hubs;
+  std::vector<int32_t> longs;
+  p->slice_begin.assign(1, 0);
   p->hub_begin.assign(1, 0);
-  std::vector<int32_t> reb;
+  int64_t deltas = 0, hub_nnz = 0;
   for (int c = 0; c < C; c++) {
     const int r0 = co[c] - co[0], r1 = co[c + 1] - co[0];
-    const int nr = r1 - r0;
-    const int32_t e0 = h_off[r0];
-    if (nr > 0) {
-      reb.resize((size_t)nr + 1);
-      for (int i = 0; i <= nr; i++) reb[i] = h_off[r0 + i] - e0;
-      Schedule sc;
-      rc = build_schedule(nr, reb[nr], reb.data(), kBlock * p->ipt, kTileRows, &sc, kSeqRow);
-      if (rc) return rc;
-      p->max_row_len = std::max(p->max_row_len, (int)sc.max_row_len);
-      const size_t h0 = all_hubs.size();
-      for (const Tile& t : sc.tiles) {
-        const Tile u{t.x + r0, t.y >= 0 ? t.y + r0 : t.y, t.z + e0, t.w + e0};
-        (t.y < 0 ? all_hubs : all_tiles).push_back(u);
-      }
-      // the color lasts as long as its longest row: start the longest first
-      std::stable_sort(all_hubs.begin() + h0, all_hubs.end(),
-                       [](const Tile& x, const Tile& y) { return x.w - x.z > y.w - y.z; });
+    int start[kSeqRow + 1] = {};  // rows of length l, then where they go
+    longs.clear();
+    for (int i = r0; i < r1; i++) {
+      p->nnz_p += h_len[i];
+      p->max_row_len = std::max(p->max_row_len, (int)h_len[i]);
+      if (h_len[i] <= kSeqRow)
+        start[h_len[i]]++;
+      else
+        longs.push_back(i);
     }
-    p->tile_begin.push_back((int)all_tiles.size());
-    p->hub_begin.push_back((int)all_hubs.size());
+    int at = r0;
+    for (int l = kSeqRow; l >= 0; l--) {
+      const int n = start[l];
+      start[l] = at;
+      at += n;
+    }
+    for (int i = r0; i < r1; i++)
+      if (h_len[i] <= kSeqRow) h_order[start[h_len[i]]++] = i;
+    for (int q = r0; q < at; q += kWave) {
+      const int n = std::min(kWave, at - q);
+      const int len = h_len[h_order[q]];
+      const bool one_len = len > 0 && h_len[h_order[q + n - 1]] == len && deltas < kSgDeltaMax;
+      slices.push_back(Slice{q, n, 0, len, 0, one_len ? (int)deltas : -1, 0});
+      if (one_len) deltas += (len + 3) & ~3;
+    }
+    std::stable_sort(longs.begin(), longs.end(),
+                     [&](int32_t x, int32_t y) { return h_len[x] > h_len[y]; });
+    for (const int32_t i : longs) {
+      hubs.push_back(Tile{at, -1, (int)hub_nnz, (int)hub_nnz + h_len[i]});
+      h_order[at++] = i;
+      hub_nnz += h_len[i];
+    }
+    p->slice_begin.push_back((int)slices.size());
+    p->hub_begin.push_back((int)hubs.size());
   }
-  rc = p->tiles.alloc(sizeof(Tile) * std::max<size_t>(all_tiles.size(), 1));
-  if (!rc) rc = p->hubs.alloc(sizeof(Tile) * std::max<size_t>(all_hubs.size(), 1));
+  p->hub_nnz = hub_nnz;
+  const int n_sl = (int)slices.size();
+  rc = p->slices.alloc(sizeof(Slice) * std::max<size_t>(slices.size(), 1));
+  if (!rc) rc = p->delta.alloc(4 * (size_t)std::max<int64_t>(deltas, 1));
+  if (!rc) rc = p->hubs.alloc(sizeof(Tile) * std::max<size_t>(hubs.size(), 1));
+  if (!rc) rc = p->col.alloc(4 * (size_t)std::max<int64_t>(hub_nnz, 1));
+  if (!rc) rc = p->val.alloc(4 * (size_t)std::max<int64_t>(hub_nnz, 1));
   if (rc) return rc;
-  if (!all_tiles.empty())
-    GD_HIP_TRY(hipMemcpyAsync(p->tiles.ptr, all_tiles.data(), sizeof(Tile) * all_tiles.size(),
+  if (n_p > 0) {
+    GD_HIP_TRY(hipMemcpyAsync(order.ptr, h_order.data(), 4 * (size_t)n_p, hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(sg_rec_kernel, dim3(sg_grid(n_p)), dim3(256), 0, s, n_p,
+                       order.as<int32_t>(), idx, len.as<int32_t>(), diag.as<float>(),
+                       p->rows.as<RowRec>());
+  }
+  if (n_sl > 0) {
+    const size_t bytes = sizeof(Slice) * slices.size();
+    const dim3 grid(sg_grid((int64_t)n_sl * kWave));
+    GD_HIP_TRY(hipMemcpyAsync(p->slices.ptr, slices.data(), bytes, hipMemcpyHostToDevice, s));
+    GD_HIP_TRY(hipMemsetAsync(p->delta.ptr, 0, 4 * (size_t)std::max<int64_t>(deltas, 1), s));
+    hipLaunchKernelGGL(sg_uniform_kernel, grid, dim3(256), 0, s, n_sl, p->slices.as<Slice>(),
+                       p->rows.as<RowRec>(), d_Ap, d_Aj, d_Ax, p->delta.as<int>());
+    GD_HIP_TRY(hipGetLastError());
+    GD_HIP_TRY(hipMemcpyAsync(slices.data(), p->slices.ptr, bytes, hipMemcpyDeviceToHost, s));
+    GD_HIP_TRY(hipStreamSynchronize(s));
+    int64_t at = 0;
+    for (Slice& sl : slices) {
+      sl.n = sl.delta >= 0 ? (sl.len + 3) / 4 : (sl.len + 1) / 2;
+      sl.off = at;
+      at += (int64_t)sl.n * sl.n_rows;
+    }
+    rc = p->ent.alloc(sizeof(int4) * (size_t)std::max<int64_t>(at, 1));
+    if (rc) return rc;
+    GD_HIP_TRY(hipMemcpyAsync(p->slices.ptr, slices.data(), bytes, hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(sg_slice_fill_kernel, grid, dim3(256), 0, s, n_sl, p->slices.as<Slice>(),
+                       p->rows.as<RowRec>(), d_Ap, d_Aj, d_Ax, p->ent.as<int4>());
+  }
+  if (!hubs.empty()) {
+    GD_HIP_TRY(hipMemcpyAsync(p->hubs.ptr, hubs.data(), sizeof(Tile) * hubs.size(),
                               hipMemcpyHostToDevice, s));
-  if (!all_hubs.empty())
-    GD_HIP_TRY(hipMemcpyAsync(p->hubs.ptr, all_hubs.data(), sizeof(Tile) * all_hubs.size(),
-                              hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(sg_hub_fill_kernel, dim3(sg_grid((int64_t)hubs.size())), dim3(256), 0, s,
+                       (int)hubs.size(), p->hubs.as<Tile>(), p->rows.as<RowRec>(), d_Ap, d_Aj,
+                       d_Ax, p->col.as<int32_t>(), p->val.as<float>());
+  }
+  GD_HIP_TRY(hipGetLastError());
   GD_HIP_TRY(hipStreamSynchronize(s));  // host vectors and scratch go out of scope
   return GD_OK;
 }
 
 // One color: one launch of symgs_color_kernel on s.
-int sweep_color(gd_symgs_plan* p, int c, const SymgsPolicy::Args& a, hipStream_t s) {
-  const int tb = p->tile_begin[c], nt = p->tile_begin[c + 1] - tb;
-  const int hb = p->hub_begin[c], nh = p->hub_begin[c + 1] - hb;
-  const IterArgs it{p->tiles.as<Tile>() + tb,
-                    nt,
-                    p->hubs.as<Tile>() + hb,
+int sweep_color(gd_symgs_plan* p, int c, float* x, const float* b, hipStream_t s) {
+  const int s0 = p->slice_begin[c], ns = p->slice_begin[c + 1] - s0;
+  const int h0 = p->hub_begin[c], nh = p->hub_begin[c + 1] - h0;
+  const SymgsArgs a{x,
+                    b,
+                    p->rows.as<RowRec>(),
+                    p->slices.as<Slice>() + s0,
+                    ns,
+                    p->ent.as<int4>(),
+                    p->delta.as<int>(),
+                    p->hubs.as<Tile>() + h0,
                     nh,
-                    nt,
-                    p->off.as<int32_t>(),
                     p->col.as<int32_t>(),
-                    (int)std::max<int64_t>(p->nnz_p - 1, 0),
-                    nullptr,
-                    nullptr,
-                    nullptr,
-                    nullptr};
+                    p->val.as<float>(),
+                    (int)std::max<int64_t>(p->hub_nnz - 1, 0)};
+  constexpr int per = kBlock / kWave;
   if (nh > 0)
-    hipLaunchKernelGGL(symgs_color_kernel<true>, dim3(nt + nh), dim3(kBlock), 0, s, a, it);
-  else if (nt > 0)
-    hipLaunchKernelGGL(symgs_color_kernel<false>, dim3(nt), dim3(kBlock), 0, s, a, it);
+    hipLaunchKernelGGL(symgs_long_kernel, dim3((ns + per - 1) / per + nh), dim3(kBlock), 0, s, a);
+  else if (ns > 0)
+    hipLaunchKernelGGL(symgs_color_kernel, dim3(ns), dim3(kWave), 0, s, a);
   GD_HIP_TRY(hipGetLastError());
   return GD_OK;
 }
@@ -409,15 +608,13 @@ int gd_symgs_plan_run(gd_symgs_plan* p, float* d_x, const float* d_b, int sweeps
   GD_CHECK_ARG(sweeps >= 0, "negative sweep count");
   GD_CHECK_ARG(p->n_p == 0 || (d_x && d_b), "NULL x / b");
   hipStream_t s = (hipStream_t)stream;
-  const SymgsPolicy::Args a{d_x, d_b, p->val.as<float>(), p->diag.as<float>(),
-                            p->orig.as<int32_t>()};
   for (int k = 0; k < sweeps; k++) {
     for (int c = 0; c < p->n_colors; c++) {
-      const int rc = sweep_color(p, c, a, s);
+      const int rc = sweep_color(p, c, d_x, d_b, s);
       if (rc) return rc;
     }
     for (int c = p->n_colors - 1; c >= 0; c--) {
-      const int rc = sweep_color(p, c, a, s);
+      const int rc = sweep_color(p, c, d_x, d_b, s);
       if (rc) return rc;
     }
   }
@@ -430,7 +627,7 @@ int gd_symgs_plan_info(const gd_symgs_plan* p, gd_symgs_plan_info_t* info) {
   info->rows = p->n_p;
   info->offdiag_nnz = p->nnz_p;
   info->n_colors = p->n_colors;
-  info->n_tiles = p->tile_begin.back();
+  info->n_tiles = p->slice_begin.back();
   info->n_exact_rows = p->hub_begin.back();
   info->max_row_len = p->max_row_len;
   info->plan_ms = p->plan_ms;

@@ -468,7 +468,7 @@ typedef struct gd_symgs_plan_info_t {
   int32_t rows;         /* rows swept: color_offsets[C] - color_offsets[0] */
   int32_t n_colors;
   int64_t offdiag_nnz;  /* off-diagonal entries of the swept rows */
-  int32_t n_tiles;      /* LDS row tiles over all colors */
+  int32_t n_tiles;      /* slices of up to 64 short rows, over all colors */
   int32_t n_exact_rows; /* rows of more than 64 off-diagonal entries */
   int32_t max_row_len;
   double plan_ms;
