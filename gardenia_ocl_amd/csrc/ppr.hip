@@ -3,20 +3,20 @@
 // The same pull iteration as pr.hip, k columns wide: column j teleports its
 // (1-d) mass to seed vertex seeds[j] instead of (1-d)/m to every vertex.
 // Scores are stored vertex-major with the k seeds of a vertex contiguous
-// (X[v*k + j]), so one gathered index u feeds k additions: a wavefront owns a
-// chunk of kc = 64*VEC columns, lane l holds columns l*VEC..l*VEC+VEC-1, and
-// the gathered row segment C[u][chunk] is one coalesced 256*VEC-byte load.
+// (X[v*k + j]).  The columns are taken in groups of 32, one 128-byte line of a
+// vertex's k-vector: 8 lanes gather an edge's line and each adds its 4 columns.
 //
 // Each column of every row is summed sequentially in CSR order, the scalar
 // personalised loop's order and FP32 rounding, so every column is the
-// single-seed run's bit for bit.  Rows longer than kSegEdges (hubs) run
-// beside the tiles: one workgroup per (hub row, 16 columns), three waves
+// single-seed run's bit for bit.  Rows longer than kHubEdges (hubs) run
+// beside the tiles: one workgroup per (hub row, column group), three waves
 // gathering chunks of the row into LDS while the fourth adds them in edge
-// order, one column per lane.  The per-iteration update is base + d*sum with
-// two roundings (built with -ffp-contract=off).
+// order, one column per lane.  Rows without in-edges keep their first score
+// and run in two iterations only.  The per-iteration update is base + d*sum
+// with two roundings (built with -ffp-contract=off).
 //
 // A persistent grid of workgroups walks the tile list; each workgroup keeps
-// per-column L1 partials for the whole sweep, and two small kernels reduce
+// per-column L1 partials for the whole sweep, and one small kernel reduces
 // them (deterministically) to per-column L1 values, their maximum and the
 // convergence flag.
 //
@@ -29,6 +29,10 @@
 // the run ends.
 
 #include <hip/hip_runtime.h>
+
+#include <rocprim/device/device_scan.hpp>
+#include <rocprim/iterator/counting_iterator.hpp>
+#include <rocprim/iterator/transform_iterator.hpp>
 
 #include <algorithm>
 #include <cmath>
@@ -45,297 +49,361 @@ namespace {
 
 constexpr int kPBlock = 256;
 constexpr int kPWaves = kPBlock / 64;
-constexpr int kSegEdges = 4096;   // rows longer than this are hubs (ppr_hub_chain_kernel)
-constexpr int kTileEdges = 1024;  // edges per wavefront tile
-constexpr int kTileRowsP = 256;   // rows per wavefront tile
-constexpr int kUnroll = 8;        // gathers in flight per lane
-constexpr int kSlices = 32;       // first-level L1 reduction slices
+constexpr int kGroup = 32;        // columns per group: one 128-byte line of a vertex's k-vector
+constexpr int kSub = 8;           // lanes that walk one row: 4 columns each
+constexpr int kSubs = kPBlock / kSub;
+constexpr int kHubEdges = 1024;   // rows longer than this are hubs (ppr_hub_chain_kernel)
+constexpr int kTileEdges = 256;   // edges per tile, at most (one tile: one 16-lane subgroup)
+constexpr int kMinTileEdges = 32;
+constexpr int kMaxSlots = 2048;   // workgroups that sweep one column group
+constexpr int kEmptySlots = 256;  // workgroups per column group in ppr_empty_kernel
+constexpr int kRedSplits = 16;    // workgroups per column group in ppr_reduce_kernel
 
 struct PprState {
   int iter;
   int done;
   int max_iter;
-  int pad;
+  unsigned ticket;  // ppr_reduce_kernel workgroups arrived in this iteration
   double tol;
 };
 
-template <int VEC>
-struct Vec {
-  float v[VEC];
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+// score / outdeg, correctly rounded, from inv = 1 / outdeg in FP64.  The FP64
+// product is within 2^-52 of the quotient of two 24-bit numbers, which is never
+// closer than 2^-49 to a midpoint of two normal floats (a - m*d is a nonzero
+// integer over m*d < 2^49), so it rounds to the same float as the IEEE division,
+// at a third of its instructions.  Subnormal results may lie on a midpoint:
+// they are divided.
+__device__ __forceinline__ float div_outdeg(float a, double inv, const int32_t* outdeg) {
+  const float q = (float)((double)a * inv);
+  if (fabsf(q) < 0x1p-125f && a != 0.0f) return a / (float)*outdeg;
+  return q;
+}
+
+// This lane's 4 columns of a vertex.
+struct Lane {
+  int seed[4];
+  bool fz[4];  // frozen columns keep their score
+  double err[4];
+
+  __device__ __forceinline__ Lane(const int32_t* __restrict__ seeds,
+                                  const int32_t* __restrict__ frozen, int col0) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      seed[j] = seeds[col0 + j];
+      fz[j] = frozen[col0 + j] != 0;
+      err[j] = 0.0;
+    }
+  }
+
+  // X[o..] <- the new scores of row r, Cn[o..] <- their contributions (iv NaN:
+  // nothing gathers this vertex), err += |change| (not read where frozen).
+  __device__ __forceinline__ void update(int r, f4 sum, f4 old, double iv,
+                                         const int32_t* __restrict__ outdeg, float teleport,
+                                         float damp, float* __restrict__ X,
+                                         float* __restrict__ Cn, int64_t o) {
+    f4 nx;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const float b = seed[j] == r ? teleport : 0.0f;
+      const float upd = b + damp * sum[j];
+      nx[j] = fz[j] ? old[j] : upd;
+      err[j] += (double)fabsf(nx[j] - old[j]);
+    }
+    __builtin_nontemporal_store(nx, reinterpret_cast<f4*>(X + o));
+    if (iv == iv) {
+      f4 nc;
+#pragma unroll
+      for (int j = 0; j < 4; j++) nc[j] = div_outdeg(nx[j], iv, outdeg + r);
+      __builtin_nontemporal_store(nc, reinterpret_cast<f4*>(Cn + o));
+    }
+  }
+
+  // The workgroup's partial per column: subgroups in order, through LDS.
+  __device__ __forceinline__ void store_err(double* __restrict__ part) const {
+    __shared__ double s_err[kSubs][kGroup];
+    const int lane = threadIdx.x & (kSub - 1), sub = threadIdx.x / kSub;
+#pragma unroll
+    for (int j = 0; j < 4; j++) s_err[sub][4 * lane + j] = err[j];
+    __syncthreads();
+    if (threadIdx.x < kGroup) {
+      double s = 0.0;
+#pragma unroll
+      for (int w = 0; w < kSubs; w++) s += s_err[w][threadIdx.x];
+      part[threadIdx.x] = s;
+    }
+  }
 };
 
-template <int VEC>
-__device__ __forceinline__ Vec<VEC> load_vec(const float* __restrict__ p) {
-  Vec<VEC> r;
-  if constexpr (VEC == 4) {
-    const float4 t = *reinterpret_cast<const float4*>(p);
-    r.v[0] = t.x; r.v[1] = t.y; r.v[2] = t.z; r.v[3] = t.w;
-  } else if constexpr (VEC == 2) {
-    const float2 t = *reinterpret_cast<const float2*>(p);
-    r.v[0] = t.x; r.v[1] = t.y;
-  } else {
-    r.v[0] = *p;
-  }
-  return r;
-}
-
-template <int VEC>
-__device__ __forceinline__ void store_vec(float* __restrict__ p, const float (&v)[VEC]) {
-  if constexpr (VEC == 4) {
-    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-  } else if constexpr (VEC == 2) {
-    *reinterpret_cast<float2*>(p) = make_float2(v[0], v[1]);
-  } else {
-    *p = v[0];
-  }
-}
-
-// acc[j] += C[u][col0 + j] over the edges [b, e) in order, kUnroll gathers in
-// flight.  b, e, k, col0 are wavefront-uniform.
-template <int VEC>
-__device__ __forceinline__ void sum_edges(const int32_t* __restrict__ col,
-                                          const float* __restrict__ C, int64_t k, int col0,
-                                          int b, int e, float (&acc)[VEC]) {
-  int i = b;
-  for (; i + kUnroll <= e; i += kUnroll) {
-    Vec<VEC> g[kUnroll];
-#pragma unroll
-    for (int q = 0; q < kUnroll; q++) {
-      const int u = __builtin_amdgcn_readfirstlane(col[i + q]);
-      g[q] = load_vec<VEC>(C + (int64_t)u * k + col0);
-    }
-#pragma unroll
-    for (int q = 0; q < kUnroll; q++)
-#pragma unroll
-      for (int j = 0; j < VEC; j++) acc[j] += g[q].v[j];
-  }
-  for (; i < e; i++) {
-    const int u = __builtin_amdgcn_readfirstlane(col[i]);
-    const Vec<VEC> g = load_vec<VEC>(C + (int64_t)u * k + col0);
-#pragma unroll
-    for (int j = 0; j < VEC; j++) acc[j] += g.v[j];
-  }
-}
-
-// Frozen columns (fz) keep their score and add nothing to the L1 change.
-template <int VEC>
-__device__ __forceinline__ void row_update(int v, const float (&acc)[VEC], const int (&seed)[VEC],
-                                           const int (&fz)[VEC], float* __restrict__ X,
-                                           float* __restrict__ Cn,
-                                           const int32_t* __restrict__ outdeg, int64_t k,
-                                           int col0, float teleport, float damp,
-                                           double (&err)[VEC]) {
-  const int64_t o = (int64_t)v * k + col0;
-  const Vec<VEC> old = load_vec<VEC>(X + o);
-  const float deg = (float)outdeg[v];
-  float nx[VEC], nc[VEC];
-#pragma unroll
-  for (int j = 0; j < VEC; j++) {
-    const float b = (seed[j] == v) ? teleport : 0.0f;
-    const float upd = b + damp * acc[j];
-    nx[j] = fz[j] ? old.v[j] : upd;
-    nc[j] = nx[j] / deg;
-    err[j] += fz[j] ? 0.0 : (double)fabsf(nx[j] - old.v[j]);
-  }
-  store_vec<VEC>(X + o, nx);
-  store_vec<VEC>(Cn + o, nc);
-}
-
-template <int VEC>
-__global__ __launch_bounds__(kPBlock) void ppr_pull_kernel(
-    const Tile* __restrict__ tiles, int n_tiles, const int32_t* __restrict__ off,
-    const int32_t* __restrict__ col, const int32_t* __restrict__ outdeg,
-    const int32_t* __restrict__ seeds, const int32_t* __restrict__ frozen, int ka, int64_t k,
-    float* __restrict__ X, float* __restrict__ C0, float* __restrict__ C1,
-    double* __restrict__ err_part, const PprState* __restrict__ st, float teleport, float damp) {
+// Rows without in-edges.  Their score is the teleport from the first iteration
+// on, so they run in the first two (X and both contribution buffers), and once
+// after the columns were permuted (the buffer that was not).
+__global__ __launch_bounds__(kPBlock) void ppr_empty_kernel(
+    const int32_t* __restrict__ rows, int n_rows, const int32_t* __restrict__ outdeg,
+    const double* __restrict__ inv, const int32_t* __restrict__ seeds,
+    const int32_t* __restrict__ frozen, int64_t k, float* __restrict__ X, float* __restrict__ C0,
+    float* __restrict__ C1, double* __restrict__ err_part, const PprState* __restrict__ st,
+    float teleport, float damp) {
   if (st->done) return;
-  const int odd = st->iter & 1;
-  const float* __restrict__ C = odd ? C1 : C0;
-  float* __restrict__ Cn = odd ? C0 : C1;
-  const int lane = threadIdx.x & 63;
-  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int col0 = blockIdx.y * 64 * VEC + lane * VEC;
-  int seed[VEC], fz[VEC];
-#pragma unroll
-  for (int j = 0; j < VEC; j++) {
-    seed[j] = seeds[col0 + j];
-    fz[j] = frozen[col0 + j];
+  float* __restrict__ Cn = (st->iter & 1) ? C0 : C1;
+  const int lane = threadIdx.x & (kSub - 1), sub = threadIdx.x / kSub;
+  const int col0 = blockIdx.y * kGroup + 4 * lane;
+  Lane me(seeds, frozen, col0);
+  for (int i = blockIdx.x * kSubs + sub; i < n_rows; i += gridDim.x * kSubs) {
+    const int r = rows[i];
+    const int64_t o = (int64_t)r * k + col0;
+    const f4 old = *reinterpret_cast<const f4*>(X + o);
+    me.update(r, (f4){0.0f, 0.0f, 0.0f, 0.0f}, old, inv[r], outdeg, teleport, damp, X, Cn, o);
   }
-  double err[VEC];
+  me.store_err(err_part + (int64_t)blockIdx.x * k + blockIdx.y * kGroup);
+}
+
+// Rows of 1 to kHubEdges edges.  An 8-lane subgroup walks the rows of a tile
+// for one group of 32 columns (lane l: columns 4l .. 4l+3 of the group), 8 edges
+// of one row in flight, each column added in edge order by its lane.  The ids of
+// the next 8 edges are loaded a step ahead, by one lane each.  Edges past the
+// row's end read vertex m, whose contributions are -0.0: they add nothing.
+//
+// Bound: bytes that miss the L2.  A column group is swept over all rows before
+// the next one starts (gp groups at a time, each on 8/gp XCDs), so an XCD's 4 MB
+// L2 holds the 32 columns of 4 times as many of the often gathered vertices as
+// a sweep with 128 columns per edge did, and the Infinity Cache most of a
+// group's.  Per iteration of 0.7 M vertices, 10.5 M edges, 128 columns (rows of
+// up to 1024 edges): 462 us alone, 2.4 GB read past the L2; beside the hubs 500
+// us against 890 before.  With 16 lanes of 2 columns and masked loads it was 704
+// us: 241 M vector instructions against 73 M.  Gathers of rarely used vertices
+// marked non-temporal miss the L2 less (2.0 GB) but are slower (594 us): they
+// pass by the Infinity Cache, too.
+__global__ __launch_bounds__(kPBlock) void ppr_pull_kernel(
+    const Tile* __restrict__ tiles, int n_tiles, int m, const int2* __restrict__ rows,
+    const int32_t* __restrict__ col, const int32_t* __restrict__ outdeg,
+    const double* __restrict__ inv, const int32_t* __restrict__ seeds,
+    const int32_t* __restrict__ frozen, int ka, int64_t k, int gp_log2, float* __restrict__ X,
+    float* __restrict__ C0, float* __restrict__ C1, double* __restrict__ err_part,
+    const PprState* __restrict__ st, float teleport, float damp) {
+  if (st->done) return;
+  const int xcd = blockIdx.x & 7;  // workgroups go to the XCDs in turn
+  const int grp = (blockIdx.y << gp_log2) + (xcd & ((1 << gp_log2) - 1));
+  if (grp * kGroup >= ka) return;
+  const int slot = (blockIdx.x >> 3) * (8 >> gp_log2) + (xcd >> gp_log2);
+  const int slots = gridDim.x >> gp_log2;
+  const float* __restrict__ C = (st->iter & 1) ? C1 : C0;
+  float* __restrict__ Cn = (st->iter & 1) ? C0 : C1;
+  const int lane = threadIdx.x & (kSub - 1), sub = threadIdx.x / kSub;
+  const int first = (threadIdx.x & 63 & ~(kSub - 1)) * 4;  // ds_bpermute address of lane 0
+  const int col0 = grp * kGroup + 4 * lane;
+  const float* __restrict__ Cc = C + col0;
+  Lane me(seeds, frozen, col0);
+  for (int t = slot * kSubs + sub; t < n_tiles; t += slots * kSubs) {
+    const Tile tl = tiles[t];
+    int at = tl.x, i = tl.z;
+    int2 row = rows[at];  // vertex, end of its edges
+    int32_t id = i + lane < tl.w ? col[i + lane] : m;
+    f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    while (at < tl.y) {  // every step ends a row or takes 8 edges of it
+      const int n = row.y - i;
+      const bool last = n <= kSub;
+      const int mine = lane < n ? id : m;
+      f4 g[kSub];
 #pragma unroll
-  for (int j = 0; j < VEC; j++) err[j] = 0.0;
-  const int nw = gridDim.x * kPWaves;
-  if (col0 < ka) {  // lanes past the running columns gather nothing
-    for (int t = blockIdx.x * kPWaves + wid; t < n_tiles; t += nw) {
-      const Tile tl = tiles[t];
-      for (int r = tl.x; r < tl.y; r++) {
-        float acc[VEC];
+      for (int q = 0; q < kSub; q++) {
+        const uint32_t u = (uint32_t)__builtin_amdgcn_ds_bpermute(first + 4 * q, mine);
+        g[q] = *reinterpret_cast<const f4*>(Cc + (uint64_t)u * (uint32_t)k);
+      }
+      i += min(n, kSub);
+      id = i + lane < tl.w ? col[i + lane] : m;
+      f4 old = acc;
+      double iv = 0.0;
+      int2 next = row;
+      const int64_t o = (int64_t)row.x * k + col0;
+      if (last) {
+        old = __builtin_nontemporal_load(reinterpret_cast<const f4*>(X + o));
+        iv = inv[row.x];
+        if (at + 1 < tl.y) next = rows[at + 1];
+      }
 #pragma unroll
-        for (int j = 0; j < VEC; j++) acc[j] = 0.0f;
-        sum_edges<VEC>(col, C, k, col0, off[r], off[r + 1], acc);
-        row_update<VEC>(r, acc, seed, fz, X, Cn, outdeg, k, col0, teleport, damp, err);
+      for (int q = 0; q < kSub; q++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[j] += g[q][j];
+      if (last) {
+        me.update(row.x, acc, old, iv, outdeg, teleport, damp, X, Cn, o);
+        acc = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+        row = next;
+        at++;
       }
     }
   }
-  // workgroup partial per column: waves in order, through LDS
-  __shared__ double s_err[kPWaves][64 * VEC];
-#pragma unroll
-  for (int j = 0; j < VEC; j++) s_err[wid][lane * VEC + j] = err[j];
-  __syncthreads();
-  for (int c = threadIdx.x; c < 64 * VEC; c += kPBlock) {
-    double s = 0.0;
-#pragma unroll
-    for (int w = 0; w < kPWaves; w++) s += s_err[w][c];
-    err_part[(int64_t)blockIdx.x * k + blockIdx.y * 64 * VEC + c] = s;
-  }
+  me.store_err(err_part + (int64_t)slot * k + grp * kGroup);
 }
 
-// Hub rows: workgroup b adds hub row hub_row[b / G] for the kHubCols columns
-// (16, 32 or 64: gd_ppr_plan_config.hub_cols) of group g = b % G (all groups
-// of the longest row are dispatched first) in
-// edge order, then runs their row updates.  Lane c < kHubCols of wave 0 adds
-// column kHubCols*g + c chunk by chunk from LDS (its own dependent chain: the
-// scalar loop's order and rounding) while waves 1..3 gather the next chunk.
-// A gathering instruction loads 64/kHubCols edges' column groups at once
-// (lane l: edge l / kHubCols, column l % kHubCols), so each gathering wave
-// keeps kHubLoads * 64/kHubCols edges in flight: the chain of a 10^5-edge row
-// is bound by load latency, and narrower column groups put more of its edges
-// in flight (and spread the row over more workgroups).  hub_err row b / G
-// receives the row's per-column |change|.
-constexpr int kHubLoads = 32;  // gathering instructions per wave per chunk
+// Hub rows: workgroup b adds hub row hub_row[b / groups] for the COLS columns
+// (gd_ppr_plan_config.hub_cols) of group b % groups, longest row first, in edge
+// order.  Waves 1..3 gather 16 bytes a lane, 16 instructions in flight each, so
+// a chunk is 48 KB (384 edges of 32 columns); lane c < COLS of wave 0 adds
+// column c of the chunk from LDS while the next one is in flight.  One LDS
+// buffer: the gathered chunk waits in registers until the adds are done.
+// Rows are cut at 1024 edges: at 512 or 2048 an iteration takes 7 or 11
+// percent longer.  98 rows of more than 4096 edges alone took 890 us with 96
+// edges of 64 columns in flight; 1224 of more than 1024 take 284 us.
+// hub_err row b / groups receives the row's per-column |change|.
+constexpr int kHubLoads = 16;  // gathering instructions per wave per chunk
 
-template <int kHubCols>  // columns per workgroup: 16, 32 or 64
+template <int COLS>  // columns per workgroup: 16, 32 or 64
 __global__ __launch_bounds__(kPBlock) void ppr_hub_chain_kernel(
     const int32_t* __restrict__ hub_row, int groups, const int32_t* __restrict__ off,
     const int32_t* __restrict__ col, const int32_t* __restrict__ outdeg,
     const int32_t* __restrict__ seeds, const int32_t* __restrict__ frozen, int ka, int64_t k,
     float* __restrict__ X, float* __restrict__ C0, float* __restrict__ C1,
     double* __restrict__ hub_err, const PprState* __restrict__ st, float teleport, float damp) {
-  constexpr int kHubEpi = 64 / kHubCols;           // edges per gathering instruction
-  constexpr int kHubEdgesW = kHubLoads * kHubEpi;  // edges per gathering wave per chunk
-  constexpr int kHubChunkE = 3 * kHubEdgesW;       // edges per chunk
-  constexpr int kHubIdRegs = (kHubEdgesW + 63) / 64;
+  constexpr int kLanes = COLS / 4;           // lanes per edge
+  constexpr int kEpi = 64 / kLanes;          // edges per gathering instruction
+  constexpr int kEdgesW = kHubLoads * kEpi;  // edges per gathering wave per chunk
+  constexpr int kChunkE = 3 * kEdgesW;       // edges per chunk
+  constexpr int kIdRegs = kEdgesW / 64;
   if (st->done) return;
-  __shared__ float buf[2][kHubChunkE * kHubCols];
-  const int odd = st->iter & 1;
-  const float* __restrict__ C = odd ? C1 : C0;
-  float* __restrict__ Cn = odd ? C0 : C1;
+  __shared__ float buf[kChunkE * COLS];
+  const float* __restrict__ C = (st->iter & 1) ? C1 : C0;
+  float* __restrict__ Cn = (st->iter & 1) ? C0 : C1;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = blockIdx.x / groups;
-  const int g0 = (blockIdx.x % groups) * kHubCols;  // first column of the group (< k)
+  const int g0 = (blockIdx.x % groups) * COLS;  // first column of the group (< k)
   const int row = hub_row[h];
   const int e0 = off[row];
   const int ne = off[row + 1] - e0;
-  const int nchunks = (ne + kHubChunkE - 1) / kHubChunkE;
-  const bool running = g0 < ka;  // uniform: a group past the running columns idles
+  const int nchunks = (ne + kChunkE - 1) / kChunkE;
   const int gw = wid - 1;  // gathering wave 0..2
-  const int my_col = g0 + (lane % kHubCols);
-  // source ids of this wave's edges of chunk c: lane l holds edge l + 64 q
-  auto load_ids = [&](int c, int (&ids)[kHubIdRegs]) {
+  const float* __restrict__ Cc = C + g0 + 4 * (lane % kLanes);
+  int32_t ids[kIdRegs];
+  f4 v[kHubLoads];
+  // source ids of this wave's edges of chunk c: lane l holds edge l + 64 q; 0
+  // (a valid vertex) past the row
+  auto load_ids = [&](int c) {
 #pragma unroll
-    for (int q = 0; q < kHubIdRegs; q++) {
-      const int e = c * kHubChunkE + gw * kHubEdgesW + q * 64 + lane;
-      ids[q] = (q * 64 + lane < kHubEdgesW && e < ne) ? col[e0 + e] : 0;
+    for (int q = 0; q < kIdRegs; q++) {
+      const int e = c * kChunkE + gw * kEdgesW + q * 64 + lane;
+      ids[q] = e < ne ? col[e0 + e] : 0;
     }
   };
-  auto produce = [&](int c, const int (&ids)[kHubIdRegs], float* dst) {
-    const int base = c * kHubChunkE + gw * kHubEdgesW;  // first edge of this wave's part
-    const int cnt = min(kHubEdgesW, ne - base);
-    float v[kHubLoads];
+  auto gather = [&]() {
 #pragma unroll
     for (int i = 0; i < kHubLoads; i++) {
-      const int e = i * kHubEpi + lane / kHubCols;  // this lane's edge in the wave's part
-      const int u = __shfl(ids[(i * kHubEpi) / 64], e % 64, 64);  // 0 past the row: valid
-      v[i] = C[(int64_t)u * k + my_col];
+      const int e = i * kEpi + lane / kLanes;  // this lane's edge in the wave's part
+      const uint32_t u = (uint32_t)__shfl(ids[(i * kEpi) / 64], e % 64, 64);
+      v[i] = *reinterpret_cast<const f4*>(Cc + (uint64_t)u * (uint32_t)k);
     }
-#pragma unroll
-    for (int i = 0; i < kHubLoads; i++)
-      if (i * kHubEpi + lane / kHubCols < cnt)
-        dst[(gw * kHubEdgesW) * kHubCols + i * 64 + lane] = v[i];
   };
   float s = 0.0f;
-  if (running) {
-    int ids[kHubIdRegs], nxt[kHubIdRegs];
-    if (wid != 0 && nchunks > 0) {
-      load_ids(0, ids);
-      if (nchunks > 1) load_ids(1, nxt);
-      produce(0, ids, buf[0]);
+  if (wid != 0) {
+    load_ids(0);
+    gather();
+    load_ids(1);
+  }
+  for (int c = 0; c < nchunks; c++) {
+    if (wid != 0) {
+      f4* dst = reinterpret_cast<f4*>(buf) + gw * kHubLoads * 64 + lane;
 #pragma unroll
-      for (int q = 0; q < kHubIdRegs; q++) ids[q] = nxt[q];
+      for (int i = 0; i < kHubLoads; i++) dst[i * 64] = v[i];
     }
     __syncthreads();
-    for (int c = 0; c < nchunks; c++) {
-      if (wid == 0) {
-        if (lane < kHubCols) {
-          const float* __restrict__ b = buf[c & 1] + lane;
-          const int nc = min(kHubChunkE, ne - c * kHubChunkE);
-          int e = 0;
-          for (; e + 8 <= nc; e += 8) {
-            float a[8];
+    if (wid != 0) {
+      if (c + 1 < nchunks) gather();
+      load_ids(c + 2);
+    } else if (lane < COLS) {
+      const float* __restrict__ b = buf + lane;
+      const int nc = min(kChunkE, ne - c * kChunkE);
+      int e = 0;
+      if (nc >= 16) {
+        float a[16];
 #pragma unroll
-            for (int q = 0; q < 8; q++) a[q] = b[(e + q) * kHubCols];
+        for (int q = 0; q < 16; q++) a[q] = b[q * COLS];
+        for (; e + 32 <= nc; e += 16) {  // the next 16 terms are read ahead of the adds
+          float nx[16];
 #pragma unroll
-            for (int q = 0; q < 8; q++) s += a[q];
-          }
-          for (; e < nc; e++) s += b[e * kHubCols];
+          for (int q = 0; q < 16; q++) nx[q] = b[(e + 16 + q) * COLS];
+#pragma unroll
+          for (int q = 0; q < 16; q++) s += a[q];
+#pragma unroll
+          for (int q = 0; q < 16; q++) a[q] = nx[q];
         }
-      } else if (c + 1 < nchunks) {
-        if (c + 2 < nchunks) load_ids(c + 2, nxt);  // in flight across the barrier
-        produce(c + 1, ids, buf[(c + 1) & 1]);
 #pragma unroll
-        for (int q = 0; q < kHubIdRegs; q++) ids[q] = nxt[q];
+        for (int q = 0; q < 16; q++) s += a[q];
+        e += 16;
       }
-      __syncthreads();
+      for (; e < nc; e++) s += b[e * COLS];
     }
+    __syncthreads();
   }
-  if (wid == 0 && lane < kHubCols) {
-    double err[1] = {0.0};
+  if (wid == 0 && lane < COLS) {
+    const int my_col = g0 + lane;
+    double err = 0.0;
     if (my_col < ka) {
-      const float acc[1] = {s};
-      const int sd[1] = {seeds[my_col]}, fz[1] = {frozen[my_col]};
-      row_update<1>(row, acc, sd, fz, X, Cn, outdeg, k, my_col, teleport, damp, err);
+      const int64_t o = (int64_t)row * k + my_col;
+      const float old = X[o];
+      const float b = seeds[my_col] == row ? teleport : 0.0f;
+      const float upd = b + damp * s;
+      const float nx = frozen[my_col] ? old : upd;
+      X[o] = nx;
+      Cn[o] = nx / (float)outdeg[row];
+      err = (double)fabsf(nx - old);
     }
-    hub_err[(int64_t)h * k + my_col] = err[0];
+    hub_err[(int64_t)h * k + my_col] = err;
   }
 }
 
-// First level: fin[s][c] = sum over the rows of err_part in slice s (fixed order).
-__global__ __launch_bounds__(kPBlock) void ppr_err_slices_kernel(const double* __restrict__ part,
-                                                                 int rows, int64_t k,
-                                                                 int64_t kact,
-                                                                 double* __restrict__ fin,
-                                                                 const PprState* __restrict__ st) {
-  if (st->done) return;
-  const int64_t c = (int64_t)blockIdx.x * kPBlock + threadIdx.x;
-  if (c >= kact) return;
-  const int per = (rows + kSlices - 1) / kSlices;
-  const int lo = blockIdx.y * per, hi = min(lo + per, rows);
-  double s = 0.0;
-  for (int r = lo; r < hi; r++) s += part[(int64_t)r * k + c];
-  fin[(int64_t)blockIdx.y * k + c] = s;
-}
-
-// Second level: per-column L1 (slices in order) of the columns still running
-// (c < kact, not frozen), their maximum, the per-column stop and the state
-// update.  With column_stop a column whose L1 change is below tol is frozen.
-__global__ __launch_bounds__(kPBlock) void ppr_finalize_kernel(
-    const double* __restrict__ fin, int64_t k, int64_t kact, double* __restrict__ col_err,
+// Per-column L1 of one iteration: workgroup (g, s) adds column group g's rows
+// r = s mod kRedSplits of the partials (err_part's `slots`, then hub_err's
+// `hubs`) in a fixed order; the last workgroup to arrive adds the splits of the
+// columns still running (c < kact, not frozen), takes their maximum, stops the
+// columns whose change is below tol (column_stop) and advances the state.
+__global__ __launch_bounds__(kPBlock) void ppr_reduce_kernel(
+    const double* __restrict__ err_part, int slots, const double* __restrict__ hub_err, int hubs,
+    int64_t k, int kact, double* __restrict__ fin, double* __restrict__ col_err,
     int32_t* __restrict__ frozen, int32_t* __restrict__ col_iters, int column_stop,
     PprState* __restrict__ st, double* __restrict__ errors) {
   if (st->done) return;
+  constexpr int kParts = kPBlock / kGroup;
+  __shared__ double s_part[kParts][kGroup];
   __shared__ double s_max[kPBlock];
+  __shared__ unsigned s_last;
   const int it = st->iter;
   const double tol = st->tol;
+  const int lc = threadIdx.x % kGroup, part = threadIdx.x / kGroup;
+  const int64_t c0 = (int64_t)blockIdx.x * kGroup + lc;
+  double s = 0.0;
+#pragma unroll 4
+  for (int r = blockIdx.y * kParts + part; r < slots; r += kRedSplits * kParts)
+    s += err_part[(int64_t)r * k + c0];
+#pragma unroll 4
+  for (int r = blockIdx.y * kParts + part; r < hubs; r += kRedSplits * kParts)
+    s += hub_err[(int64_t)r * k + c0];
+  s_part[part][lc] = s;
+  __syncthreads();
+  if (part == 0) {
+    s = 0.0;
+#pragma unroll
+    for (int q = 0; q < kParts; q++) s += s_part[q][lc];
+    fin[(int64_t)blockIdx.y * k + c0] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __threadfence();  // release fin before taking a ticket
+    s_last = atomicAdd(&st->ticket, 1u) + 1 == gridDim.x * gridDim.y;
+  }
+  __syncthreads();
+  if (!s_last) return;
+  __threadfence();  // acquire: every workgroup's fin is visible
   double mx = 0.0;
-  for (int64_t c = threadIdx.x; c < kact; c += kPBlock) {
+  for (int c = threadIdx.x; c < kact; c += kPBlock) {
     if (frozen[c]) continue;
-    double s = 0.0;
-    for (int q = 0; q < 2 * kSlices; q++) s += fin[(int64_t)q * k + c];
-    col_err[c] = s;
+    double t = 0.0;
+#pragma unroll
+    for (int q = 0; q < kRedSplits; q++) t += fin[(int64_t)q * k + c];
+    col_err[c] = t;
     col_iters[c] = it + 1;
-    mx = fmax(mx, s);
-    if (column_stop && s < tol) frozen[c] = 1;
+    mx = fmax(mx, t);
+    if (column_stop && t < tol) frozen[c] = 1;
   }
   s_max[threadIdx.x] = mx;
   __syncthreads();
@@ -345,6 +413,7 @@ __global__ __launch_bounds__(kPBlock) void ppr_finalize_kernel(
   }
   if (threadIdx.x == 0) {
     errors[it] = s_max[0];
+    st->ticket = 0;
     st->iter = it + 1;
     // every running column below tol <=> the max over them is
     if (s_max[0] < tol || it + 1 >= st->max_iter) st->done = 1;
@@ -386,6 +455,53 @@ __global__ __launch_bounds__(kPBlock) void ppr_permute_cols_kernel(int m, int64_
   }
 }
 
+__global__ void ppr_mark_sources_kernel(int64_t nnz, const int32_t* __restrict__ col,
+                                        uint8_t* __restrict__ mark) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nnz;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    const int u = col[i];
+    if (!mark[u]) mark[u] = 1;
+  }
+}
+
+// inv: 1 / outdeg in FP64, NaN for a vertex that no edge leaves; and vertex m's
+// contributions of -0.0
+__global__ void ppr_inv_kernel(int m, int k, const int32_t* __restrict__ outdeg,
+                               const uint8_t* __restrict__ mark,
+                               double* __restrict__ inv, float* __restrict__ C0,
+                               float* __restrict__ C1) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v < m) inv[v] = mark[v] ? 1.0 / (double)(float)outdeg[v] : __builtin_nan("");
+  if (v < k) C0[(int64_t)m * k + v] = C1[(int64_t)m * k + v] = -0.0f;
+}
+
+struct HasEdges {
+  const int32_t* off;
+  __device__ int operator()(int r) const { return off[r + 1] > off[r]; }
+};
+
+// Rows with edges to rows / ends, the others to empty, in order: at[r] rows with
+// edges come before r.
+__global__ void ppr_split_rows_kernel(int m, const int32_t* __restrict__ off,
+                                      const int32_t* __restrict__ at, int2* __restrict__ rows,
+                                      int32_t* __restrict__ ends, int32_t* __restrict__ empty) {
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= m) return;
+  const int e = off[r + 1];
+  if (e > off[r]) {
+    rows[at[r]] = make_int2(r, e);
+    ends[at[r]] = e;
+  } else {
+    empty[r - at[r]] = r;
+  }
+}
+
+__global__ void ppr_hub_vertex_kernel(int n, const int2* __restrict__ rows,
+                                      int32_t* __restrict__ hub_row) {
+  const int h = blockIdx.x * blockDim.x + threadIdx.x;
+  if (h < n) hub_row[h] = rows[hub_row[h]].x;
+}
+
 __global__ void ppr_init_kernel(int64_t n, int64_t k, const float* __restrict__ X,
                                 const int32_t* __restrict__ outdeg, float* __restrict__ C0,
                                 PprState* __restrict__ st, int max_iter, double tol) {
@@ -396,6 +512,7 @@ __global__ void ppr_init_kernel(int64_t n, int64_t k, const float* __restrict__ 
     st->iter = 0;
     st->done = max_iter <= 0;
     st->max_iter = max_iter;
+    st->ticket = 0;
     st->tol = tol;
   }
 }
@@ -435,8 +552,9 @@ __global__ void check_seeds_kernel(int k, const int32_t* __restrict__ seeds, int
 using namespace gd;
 
 struct gd_ppr_plan {
-  int m = 0, k = 0, kc = 64;
-  int hub_cols = 64;  // columns per hub-row workgroup
+  int m = 0, k = 0;
+  int kc = kGroup;         // columns swept at once
+  int hub_cols = kGroup;   // columns per hub-row workgroup
   int64_t nnz = 0;
   hipStream_t stream = nullptr;
   bool relabel = false;
@@ -445,7 +563,7 @@ struct gd_ppr_plan {
   const int32_t* outdeg = nullptr;
   Relabel rl;
   Schedule sched;
-  int n_tiles = 0, n_hubs = 0, grid = 0;
+  int n_tiles = 0, n_hubs = 0, n_empty = 0, grid = 0;
   // hub rows run on the plan's stream beside the tiles on `side` (fork / join)
   hipStream_t side = nullptr;
   hipEvent_t fork_ev = nullptr, join_ev = nullptr;
@@ -454,7 +572,7 @@ struct gd_ppr_plan {
     if (join_ev) (void)hipEventDestroy(join_ev);
     if (side) (void)hipStreamDestroy(side);
   }
-  DeviceBuffer tiles, hub_row, err_part, hub_err, fin, col_err,
+  DeviceBuffer tiles, rows, empty, hub_row, inv, err_part, hub_err, fin, col_err,
       C0, C1, Xint, seeds, state, errors, frozen, col_iters, newcol, cperm;
   int errors_cap = 0;
   bool column_stop = true;
@@ -472,7 +590,6 @@ int ppr_build(gd_ppr_plan* p, const int32_t* d_off, const int32_t* d_col,
   if (rc) return rc;
   rc = check_offsets(d_off, m, p->nnz, p->stream);  // before any device walk
   if (rc) return rc;
-  std::vector<int32_t> h_off(m + 1);
   p->off = d_off;
   p->col = d_col;
   p->outdeg = d_outdeg;
@@ -483,50 +600,77 @@ int ppr_build(gd_ppr_plan* p, const int32_t* d_off, const int32_t* d_col,
     p->col = p->rl.col.as<int32_t>();
     p->outdeg = p->rl.outdeg.as<int32_t>();
   }
-  GD_HIP_TRY(hipMemcpyAsync(h_off.data(), p->off, 4 * ((size_t)m + 1), hipMemcpyDeviceToHost,
-                            p->stream));
+  // the rows with edges (vertex, end of its edges), and the others
+  DeviceBuffer at, ends, tmp, mark;
+  rocprim::transform_iterator<rocprim::counting_iterator<int>, HasEdges, int> flags(
+      rocprim::counting_iterator<int>(0), HasEdges{p->off});
+  size_t bytes = 0;
+  GD_HIP_TRY(rocprim::exclusive_scan(nullptr, bytes, flags, (int32_t*)nullptr, 0, (size_t)m,
+                                     rocprim::plus<int>(), p->stream));
+  rc = at.alloc(4 * (size_t)m);
+  if (!rc) rc = ends.alloc(4 * (size_t)m);
+  if (!rc) rc = tmp.alloc(bytes);
+  if (!rc) rc = mark.alloc((size_t)m);
+  if (!rc) rc = p->rows.alloc(sizeof(int2) * (size_t)m);
+  if (!rc) rc = p->empty.alloc(4 * (size_t)m);
+  if (rc) return rc;
+  GD_HIP_TRY(rocprim::exclusive_scan(tmp.ptr, bytes, flags, at.as<int32_t>(), 0, (size_t)m,
+                                     rocprim::plus<int>(), p->stream));
+  hipLaunchKernelGGL(ppr_split_rows_kernel, dim3((m + 255) / 256), dim3(256), 0, p->stream, m,
+                     p->off, at.as<int32_t>(), p->rows.as<int2>(), ends.as<int32_t>(),
+                     p->empty.as<int32_t>());
+  GD_HIP_TRY(hipGetLastError());
+  int32_t last[3];  // rows with edges before the last row, and its offsets
+  GD_HIP_TRY(hipMemcpyAsync(last, at.as<int32_t>() + m - 1, 4, hipMemcpyDeviceToHost, p->stream));
+  GD_HIP_TRY(hipMemcpyAsync(last + 1, p->off + m - 1, 8, hipMemcpyDeviceToHost, p->stream));
   GD_HIP_TRY(hipStreamSynchronize(p->stream));
-  // wavefront tiles: <= kTileEdges edges / kTileRowsP rows; rows > kSegEdges are
+  const int n_rows = last[0] + (last[2] > last[1] ? 1 : 0);
+  p->n_empty = m - n_rows;
+  std::vector<int32_t> row_off((size_t)n_rows + 1);  // edge offsets of the rows with edges
+  row_off[0] = 0;
+  if (n_rows)
+    GD_HIP_TRY(hipMemcpyAsync(row_off.data() + 1, ends.ptr, 4 * (size_t)n_rows,
+                              hipMemcpyDeviceToHost, p->stream));
+  GD_HIP_TRY(hipStreamSynchronize(p->stream));
+  // tiles: rows packed to tile_edges edges and a quarter as many rows, for each of
+  // the kMaxSlots * kSubs subgroups of a sweep one or more; rows > kHubEdges are
   // hubs (ppr_hub_chain_kernel), longest first
+  const int tile_edges = (int)std::max<int64_t>(
+      kMinTileEdges, std::min<int64_t>(kTileEdges, p->nnz / (kMaxSlots * kSubs)));
   Schedule& s = p->sched;
   {
-    Schedule hubs;
-    rc = build_schedule(m, p->nnz, h_off.data(), kSegEdges, m, &hubs);
+    Schedule packed;
+    rc = build_schedule(n_rows, p->nnz, row_off.data(), tile_edges, tile_edges / 4, &packed);
     if (rc) return rc;
-    s.hub_row = hubs.hub_row;
-    s.max_row_len = hubs.max_row_len;
-    std::stable_sort(s.hub_row.begin(), s.hub_row.end(), [&](int32_t a, int32_t b) {
-      return h_off[a + 1] - h_off[a] > h_off[b + 1] - h_off[b];
-    });
-    // re-tile the non-hub rows with the smaller wavefront tiles
-    Schedule small;
-    rc = build_schedule(m, p->nnz, h_off.data(), kTileEdges, kTileRowsP, &small);
-    if (rc) return rc;
-    // heaviest work first: single rows of (kTileEdges, kSegEdges] edges, then
+    s.max_row_len = packed.max_row_len;
+    auto len = [&](int32_t i) { return row_off[i + 1] - row_off[i]; };
+    std::stable_sort(packed.hub_row.begin(), packed.hub_row.end(),
+                     [&](int32_t a, int32_t b) { return len(a) > len(b); });
+    // heaviest work first: single rows of (tile_edges, kHubEdges] edges, then
     // the packed row tiles
-    for (size_t h = 0; h < small.hub_row.size(); h++) {
-      const int r = small.hub_row[h];
-      const int d = h_off[r + 1] - h_off[r];
-      if (d <= kSegEdges) s.tiles.push_back(Tile{r, r + 1, h_off[r], h_off[r + 1]});
+    for (const int32_t i : packed.hub_row) {
+      if (len(i) > kHubEdges)
+        s.hub_row.push_back(i);  // its vertex below
+      else
+        s.tiles.push_back(Tile{i, i + 1, row_off[i], row_off[i + 1]});
     }
-    for (const Tile& t : small.tiles)
+    for (const Tile& t : packed.tiles)
       if (t.y >= 0) s.tiles.push_back(t);
   }
   p->n_tiles = (int)s.tiles.size();
   p->n_hubs = (int)s.hub_row.size();
-  int dev = 0, cus = 256;
-  (void)hipGetDevice(&dev);
-  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  p->grid = std::max(1, std::min(cus * 8, (p->n_tiles + kPWaves - 1) / kPWaves));
+  // a multiple of 8 workgroups per group, so that every XCD keeps its share
+  p->grid = std::max(8, std::min(kMaxSlots, (p->n_tiles + kSubs * 8 - 1) / (kSubs * 8) * 8));
   const size_t mk = (size_t)m * p->k;
   rc = p->tiles.alloc(sizeof(Tile) * p->n_tiles);
   if (!rc) rc = p->hub_row.alloc(4 * (size_t)std::max(1, p->n_hubs));
-  if (!rc) rc = p->err_part.alloc(8 * (size_t)p->grid * p->k);
+  if (!rc) rc = p->err_part.alloc(8 * (size_t)(p->grid + kEmptySlots) * p->k);
   if (!rc) rc = p->hub_err.alloc(8 * (size_t)std::max(1, p->n_hubs) * p->k);
-  if (!rc) rc = p->fin.alloc(8 * (size_t)2 * kSlices * p->k);
+  if (!rc) rc = p->fin.alloc(8 * (size_t)kRedSplits * p->k);
   if (!rc) rc = p->col_err.alloc(8 * (size_t)p->k);
-  if (!rc) rc = p->C0.alloc(4 * mk);
-  if (!rc) rc = p->C1.alloc(4 * mk);
+  if (!rc) rc = p->inv.alloc(8 * (size_t)m);
+  if (!rc) rc = p->C0.alloc(4 * (mk + p->k));  // vertex m: edges past a row's end
+  if (!rc) rc = p->C1.alloc(4 * (mk + p->k));
   if (!rc && p->relabel) rc = p->Xint.alloc(4 * mk);
   if (!rc) rc = p->seeds.alloc(4 * (size_t)p->k);
   if (!rc) rc = p->frozen.alloc(4 * (size_t)p->k);
@@ -535,11 +679,24 @@ int ppr_build(gd_ppr_plan* p, const int32_t* d_off, const int32_t* d_col,
   if (!rc) rc = p->cperm.alloc(4 * (size_t)p->k);
   if (!rc) rc = p->state.alloc(sizeof(PprState));
   if (rc) return rc;
-  GD_HIP_TRY(hipMemcpyAsync(p->tiles.ptr, s.tiles.data(), sizeof(Tile) * p->n_tiles,
-                            hipMemcpyHostToDevice, p->stream));
+  GD_HIP_TRY(hipMemsetAsync(mark.ptr, 0, (size_t)m, p->stream));
+  if (p->nnz)
+    hipLaunchKernelGGL(ppr_mark_sources_kernel,
+                       dim3((unsigned)std::min<int64_t>((p->nnz + 255) / 256, 16384)), dim3(256), 0,
+                       p->stream, p->nnz, p->col, mark.as<uint8_t>());
+  hipLaunchKernelGGL(ppr_inv_kernel, dim3((std::max(m, p->k) + 255) / 256), dim3(256), 0, p->stream,
+                     m, p->k, p->outdeg, mark.as<uint8_t>(), p->inv.as<double>(), p->C0.as<float>(),
+                     p->C1.as<float>());
+  GD_HIP_TRY(hipGetLastError());
+  if (p->n_tiles)
+    GD_HIP_TRY(hipMemcpyAsync(p->tiles.ptr, s.tiles.data(), sizeof(Tile) * p->n_tiles,
+                              hipMemcpyHostToDevice, p->stream));
   if (p->n_hubs) {
     GD_HIP_TRY(hipMemcpyAsync(p->hub_row.ptr, s.hub_row.data(), 4 * p->n_hubs,
                               hipMemcpyHostToDevice, p->stream));
+    hipLaunchKernelGGL(ppr_hub_vertex_kernel, dim3((p->n_hubs + 255) / 256), dim3(256), 0,
+                       p->stream, p->n_hubs, p->rows.as<int2>(), p->hub_row.as<int32_t>());
+    GD_HIP_TRY(hipGetLastError());
     GD_HIP_TRY(hipStreamCreateWithFlags(&p->side, hipStreamNonBlocking));
     GD_HIP_TRY(hipEventCreateWithFlags(&p->fork_ev, hipEventDisableTiming));
     GD_HIP_TRY(hipEventCreateWithFlags(&p->join_ev, hipEventDisableTiming));
@@ -548,16 +705,23 @@ int ppr_build(gd_ppr_plan* p, const int32_t* d_off, const int32_t* d_col,
   return GD_OK;
 }
 
-// One iteration over the running columns [0, ka) (whole chunks of 64*VEC).
-template <int VEC>
-void ppr_launch_iteration(gd_ppr_plan* p, float* X, PprState* st, float teleport, float damp,
-                          int ka) {
-  const int kc = 64 * VEC;
-  const int chunks = (ka + kc - 1) / kc;
-  const int64_t kact = (int64_t)chunks * kc;
-  float* C0 = p->C0.as<float>();
-  float* C1 = p->C1.as<float>();
-  const int32_t* frozen = p->frozen.as<int32_t>();
+template <int COLS>
+void ppr_launch_hubs(gd_ppr_plan* p, float* X, PprState* st, float teleport, float damp, int ka,
+                     int kact) {
+  const int groups = (kact + COLS - 1) / COLS;
+  hipLaunchKernelGGL(ppr_hub_chain_kernel<COLS>, dim3((unsigned)(p->n_hubs * groups)),
+                     dim3(kPBlock), 0, p->stream, p->hub_row.as<int32_t>(), groups, p->off, p->col,
+                     p->outdeg, p->seeds.as<int32_t>(), p->frozen.as<int32_t>(), ka,
+                     (int64_t)p->k, X, p->C0.as<float>(), p->C1.as<float>(),
+                     p->hub_err.as<double>(), st, teleport, damp);
+}
+
+// One iteration over the running columns [0, ka); `empty`: with the rows that
+// have no in-edges.
+void ppr_launch(gd_ppr_plan* p, float* X, PprState* st, float teleport, float damp, int ka,
+                bool empty) {
+  const int groups = (ka + kGroup - 1) / kGroup;
+  const int kact = groups * kGroup;
   // hub rows first, on the plan's stream, so their workgroups are placed before
   // the tiles fill the CUs; the tiles fork onto the side stream and join back
   hipStream_t ts = p->stream;
@@ -565,52 +729,37 @@ void ppr_launch_iteration(gd_ppr_plan* p, float* X, PprState* st, float teleport
     (void)hipEventRecord(p->fork_ev, p->stream);
     (void)hipStreamWaitEvent(p->side, p->fork_ev, 0);
     ts = p->side;
-    const int groups = (int)(kact / p->hub_cols);
-    const dim3 hg((unsigned)(p->n_hubs * groups));
     if (p->hub_cols == 16)
-      hipLaunchKernelGGL(ppr_hub_chain_kernel<16>, hg, dim3(kPBlock), 0, p->stream,
-                         p->hub_row.as<int32_t>(), groups, p->off, p->col, p->outdeg,
-                         p->seeds.as<int32_t>(), frozen, ka, (int64_t)p->k, X, C0, C1,
-                         p->hub_err.as<double>(), st, teleport, damp);
+      ppr_launch_hubs<16>(p, X, st, teleport, damp, ka, kact);
     else if (p->hub_cols == 32)
-      hipLaunchKernelGGL(ppr_hub_chain_kernel<32>, hg, dim3(kPBlock), 0, p->stream,
-                         p->hub_row.as<int32_t>(), groups, p->off, p->col, p->outdeg,
-                         p->seeds.as<int32_t>(), frozen, ka, (int64_t)p->k, X, C0, C1,
-                         p->hub_err.as<double>(), st, teleport, damp);
+      ppr_launch_hubs<32>(p, X, st, teleport, damp, ka, kact);
     else
-      hipLaunchKernelGGL(ppr_hub_chain_kernel<64>, hg, dim3(kPBlock), 0, p->stream,
-                         p->hub_row.as<int32_t>(), groups, p->off, p->col, p->outdeg,
-                         p->seeds.as<int32_t>(), frozen, ka, (int64_t)p->k, X, C0, C1,
-                         p->hub_err.as<double>(), st, teleport, damp);
+      ppr_launch_hubs<64>(p, X, st, teleport, damp, ka, kact);
   }
-  hipLaunchKernelGGL(ppr_pull_kernel<VEC>, dim3(p->grid, chunks), dim3(kPBlock), 0, ts,
-                     p->tiles.as<Tile>(), p->n_tiles, p->off, p->col, p->outdeg,
-                     p->seeds.as<int32_t>(), frozen, ka, (int64_t)p->k, X, C0, C1,
-                     p->err_part.as<double>(), st, teleport, damp);
+  int gp_log2 = 0;  // column groups swept at once: kc / kGroup = 1, 2, 4 or 8
+  while ((kGroup << gp_log2) < p->kc) gp_log2++;
+  const int gp = 1 << gp_log2;
+  hipLaunchKernelGGL(ppr_pull_kernel, dim3(p->grid * gp, (groups + gp - 1) / gp), dim3(kPBlock),
+                     0, ts, p->tiles.as<Tile>(), p->n_tiles, p->m, p->rows.as<int2>(), p->col, p->outdeg,
+                     p->inv.as<double>(), p->seeds.as<int32_t>(), p->frozen.as<int32_t>(), ka, (int64_t)p->k, gp_log2,
+                     X, p->C0.as<float>(), p->C1.as<float>(), p->err_part.as<double>(), st,
+                     teleport, damp);
+  empty = empty && p->n_empty;
+  if (empty)
+    hipLaunchKernelGGL(ppr_empty_kernel, dim3(kEmptySlots, groups), dim3(kPBlock), 0, ts,
+                       p->empty.as<int32_t>(), p->n_empty, p->outdeg, p->inv.as<double>(),
+                       p->seeds.as<int32_t>(), p->frozen.as<int32_t>(), (int64_t)p->k, X,
+                       p->C0.as<float>(), p->C1.as<float>(),
+                       p->err_part.as<double>() + (size_t)p->grid * p->k, st, teleport, damp);
   if (p->n_hubs) {
     (void)hipEventRecord(p->join_ev, p->side);
     (void)hipStreamWaitEvent(p->stream, p->join_ev, 0);
   }
-  const dim3 sg((unsigned)((kact + kPBlock - 1) / kPBlock), kSlices);
-  double* fin = p->fin.as<double>();
-  hipLaunchKernelGGL(ppr_err_slices_kernel, sg, dim3(kPBlock), 0, p->stream,
-                     p->err_part.as<double>(), p->grid, (int64_t)p->k, kact, fin, st);
-  hipLaunchKernelGGL(ppr_err_slices_kernel, sg, dim3(kPBlock), 0, p->stream,
-                     p->hub_err.as<double>(), p->n_hubs, (int64_t)p->k, kact,
-                     fin + (size_t)kSlices * p->k, st);
-  hipLaunchKernelGGL(ppr_finalize_kernel, dim3(1), dim3(kPBlock), 0, p->stream, fin,
-                     (int64_t)p->k, kact, p->col_err.as<double>(), p->frozen.as<int32_t>(),
-                     p->col_iters.as<int32_t>(), p->column_stop ? 1 : 0, st,
-                     p->errors.as<double>());
-}
-
-void ppr_launch(gd_ppr_plan* p, float* X, PprState* st, float teleport, float damp, int ka) {
-  if (p->kc == 256)
-    ppr_launch_iteration<4>(p, X, st, teleport, damp, ka);
-  else if (p->kc == 128)
-    ppr_launch_iteration<2>(p, X, st, teleport, damp, ka);
-  else
-    ppr_launch_iteration<1>(p, X, st, teleport, damp, ka);
+  hipLaunchKernelGGL(ppr_reduce_kernel, dim3(groups, kRedSplits), dim3(kPBlock), 0, p->stream,
+                     p->err_part.as<double>(), p->grid + (empty ? kEmptySlots : 0), p->hub_err.as<double>(), p->n_hubs,
+                     (int64_t)p->k, kact, p->fin.as<double>(), p->col_err.as<double>(),
+                     p->frozen.as<int32_t>(), p->col_iters.as<int32_t>(), p->column_stop ? 1 : 0,
+                     st, p->errors.as<double>());
 }
 
 // Applies `order` (new column c <- old column order[c], c < ka) to the rows of
@@ -699,13 +848,13 @@ int gd_ppr_plan_create(int m, int64_t nnz, const int32_t* d_off, const int32_t* 
   p->m = m;
   p->nnz = nnz;
   p->k = k;
-  p->kc = c.k_chunk ? c.k_chunk : (k % 256 == 0 ? 256 : (k % 128 == 0 ? 128 : 64));
+  p->kc = c.k_chunk ? c.k_chunk : kGroup;
   p->stream = (hipStream_t)stream;
   p->relabel = (c.relabel == 1) || (c.relabel == -1 && nnz >= (1 << 20));
   p->column_stop = c.column_stop != 0;
   // LDS of the in-place column permutation: kPWaves rows of k floats <= 64 KB
   p->compact = p->column_stop && c.compact != 0 && k <= 4096;
-  p->hub_cols = c.hub_cols ? c.hub_cols : 64;
+  p->hub_cols = c.hub_cols ? c.hub_cols : kGroup;
   int rc = GD_OK;
   if (m > 0) {
     hipEvent_t t0 = nullptr, t1 = nullptr;
@@ -814,11 +963,13 @@ int gd_ppr_plan_run(gd_ppr_plan* p, const int32_t* d_seeds, float* d_X,
   for (int j = 0; j < k; j++) cperm[j] = j;
   int ka = k;  // columns [0, ka) may still be running; the rest are frozen
   int launched = 0;
+  int permuted_at = 0;  // the last iteration before which columns were permuted
   PprState h{};
   std::vector<int32_t> fz;
   while (launched < o.max_iter) {
     const int nl = std::min(chunk, o.max_iter - launched);
-    for (int q = 0; q < nl; q++) ppr_launch(p, X, st, teleport, damp, ka);
+    for (int q = launched; q < launched + nl; q++)
+      ppr_launch(p, X, st, teleport, damp, ka, q < 2 || q == permuted_at);
     GD_HIP_TRY(hipGetLastError());
     launched += nl;
     GD_HIP_TRY(hipMemcpyAsync(&h, st, sizeof(PprState), hipMemcpyDeviceToHost, p->stream));
@@ -841,6 +992,7 @@ int gd_ppr_plan_run(gd_ppr_plan* p, const int32_t* d_seeds, float* d_X,
     float* Cnext = (h.iter & 1) ? p->C1.as<float>() : p->C0.as<float>();
     const int rc = ppr_compact(p, X, Cnext, ka, order, cperm);
     if (rc) return rc;
+    permuted_at = launched;
     ka -= nf;
   }
   // back to the user's vertex and column order

@@ -272,19 +272,18 @@ typedef struct gd_ppr_plan gd_ppr_plan;
 
 typedef struct gd_ppr_plan_config {
   int relabel; /* as gd_pr_plan_config.relabel */
-  int k_chunk; /* columns per wavefront pass: 64, 128 or 256 (one 256*k_chunk/64-byte
-                  gather per edge); 0: the largest that divides k */
+  int k_chunk; /* columns swept over all rows at once: 64, 128 or 256 (must divide k; each 32
+                  of them on their own set of XCDs); 0: 32, on all of them */
   int column_stop; /* 1 (default, -1): each column stops after its first iteration whose
                       L1 change is below tol, as k independent runs would; 0: every
                       column iterates until the largest L1 change is below tol */
   int compact;     /* 1 (default, -1; needs k <= 4096): stopped columns are moved behind
                       the running ones between host checks, so their lanes stop gathering;
                       0: stopped columns stay in place (masked) */
-  int hub_cols;    /* columns per workgroup of a hub row (> 4096 in-edges, added in edge
+  int hub_cols;    /* columns per workgroup of a hub row (> 1024 in-edges, added in edge
                       order per column): 16, 32 or 64; narrower groups keep more of the
                       row's edges in flight per workgroup, wider ones gather each
-                      edge's columns in fewer requests; 0: auto (64, the fastest of
-                      the three for RMAT-22 at k = 256) */
+                      edge's columns in fewer requests; 0: 32 */
 } gd_ppr_plan_config;
 
 void gd_ppr_default_plan_config(gd_ppr_plan_config *cfg);
@@ -295,7 +294,7 @@ typedef struct gd_ppr_plan_info_t {
   int32_t k;
   int32_t k_chunk;
   int32_t relabel;
-  int32_t grid; /* persistent workgroups per column chunk */
+  int32_t grid; /* persistent workgroups per group of 32 columns */
   float plan_ms;
   int32_t hub_cols;
 } gd_ppr_plan_info_t;
