@@ -25,9 +25,15 @@ struct wide_tiles : std::false_type {};
 template <class P>
 struct wide_tiles<P, std::void_t<decltype(P::kWideTiles)>> : std::bool_constant<P::kWideTiles> {};
 
-// Windowed gathers above this many sources: 4 MB of them, one XCD's L2, which
-// serves a smaller vector's gathers by itself.
-constexpr int kWindowMin = 1 << 20;
+// Windowed gathers above this many sources.  An XCD's 4 MB L2 serves a vector
+// of 2^20 floats by itself, and of a longer one the part that is gathered most;
+// relabelled, that part lies together.  us per solve, plain / windowed gather.
+// Relabelled, 20 iterations: 1.1 M vertices, 33 M edges 2026 / 2921; 4.2 M, 67 M
+// 5108 / 6011; 6 M, 96 M 7762 / 8159; 7 M, 112 M 9155 / 9141; 8.4 M, 134 M 11462 /
+// 10899; 12 M, 96 M 9537 / 8629.  Original order (weighted, forward and adjoint):
+// 1.3 M, 18 M 15281 / 17272; 2 M, 24 M 22964 / 22688; 3 M, 24 M 23632 / 21562.
+constexpr int kWindowMin = 1 << 21;
+constexpr int kWindowMinRelabelled = 7 << 20;
 
 struct IterEngine {
   int m = 0;
@@ -43,6 +49,7 @@ struct IterEngine {
   // Windowed gather (window_gather.h) where the gathered vector exceeds an
   // XCD's L2; sorted tiles only.
   bool windows = false;
+  int window_min = kWindowMin;
   WindowGather win;
   int32_t* col_owned = nullptr;  // the caller's private copy of col: sorted in place
   int pull_grid = 0;
@@ -138,7 +145,7 @@ struct IterEngine {
       }
       // exact hub rows are kept in edge order, or sorted in staging blocks
       const int64_t segs = (int64_t)sched.tiles.size() + nnz / kScanChunk + sched.n_slots;
-      const bool win_on = windows && stage_hubs != 0 && !persistent && m > kWindowMin &&
+      const bool win_on = windows && stage_hubs != 0 && !persistent && m > window_min &&
                           window_gather_fits(m, nnz, segs);
       std::vector<int2> seg;
       rc = build_tile_sort(sched, block * ipt, col, dst, pos.as<uint16_t>(), stream,

@@ -157,6 +157,7 @@ int gd_pr_plan_create_ex(int m, int64_t nnz, const int32_t* d_off, const int32_t
   p->eng.persistent = c.persistent == 1;
   p->eng.sort_tiles = c.sort_tiles != 0;
   p->eng.windows = p->eng.sort_tiles;
+  p->eng.window_min = p->relabel ? kWindowMinRelabelled : kWindowMin;
   p->eng.block = (c.block > kBlock && !p->eng.persistent) ? c.block : kBlock;
   // Rows longer than hub_threshold (256*ipt by default) edges are whole-row
   // hubs summed in the reference's order and rounding (exact_hub_kernel);

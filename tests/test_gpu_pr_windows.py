@@ -62,3 +62,23 @@ def test_windows_match_oracle_and_plain_gather(device, m, form):
         got.append(s.cpu().numpy())
         plan.close()
     np.testing.assert_array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("m,relabel", [((1 << 21) + 1, False), ((1 << 21) + 32769, False),
+                                       ((7 << 20) + 1, True), ((7 << 20) + 32768, True)])
+@pytest.mark.parametrize("form", ["spread", "ends", "hubs"])
+def test_windows_past_their_lines(device, m, relabel, form):
+    import torch
+
+    rng = np.random.default_rng(m)
+    off, col, deg = _graph(m, form, rng)
+    t = lambda a: torch.from_numpy(a).to(device)  # noqa: E731
+    init = rng.random(m).astype(np.float32) / np.float32(m)
+    ref, _, _ = oracle.pr(m, off, col, deg, init, tol=0.0, max_iter=3)
+    for kw in ({}, {"block": 512}, {"hub_threshold": 64}):
+        plan = PageRankPlan(t(off), t(col), t(deg), relabel=relabel, **kw)
+        for _ in range(2):  # direct launches, then the captured graph
+            s = t(init.copy())
+            plan.run(s, tol=0.0, max_iter=3)
+            np.testing.assert_array_equal(s.cpu().numpy(), ref, err_msg=str(kw))
+        plan.close()
