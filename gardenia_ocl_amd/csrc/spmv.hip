@@ -138,10 +138,7 @@ struct gd_spmv_plan {
   // offsets there
   WindowGather win;
   DeviceBuffer slot, pos;
-  // Long rows beside the tiles: their chains (3 ns per nonzero, 176 registers)
-  // run as a launch of their own on `side`, so the tiles keep their registers
-  // and do not wait for the longest chain.  Where the tiles' work is small,
-  // one launch is cheaper than the fork and the join (about 15 us).
+  // long rows on `stream`, the tiles beside them on `side` (long_rows_beside)
   hipStream_t side = nullptr;
   hipEvent_t fork_ev = nullptr, join_ev = nullptr;
   ~gd_spmv_plan() {
@@ -173,11 +170,27 @@ int check_sorted(const gd_spmv_plan* p) {
   return GD_OK;
 }
 
+// Whether the long rows run as a launch of their own beside the tiles.  Their
+// chain (3 ns per nonzero of the longest) holds 176 registers; tiles in the
+// same launch run at 2 wavefronts per SIMD and take about 8 ps per nonzero.
+// While the chain lasts longer than that, one launch costs the chain alone,
+// two cost the fork and the join (15 us) as well.  Power-law matrices, us in
+// one launch / beside (with windows where x is large): 0.6 M rows, 9 M
+// nonzeros 100 / 142, 2 M, 8 M 88 / 99, 2 M, 19 M 166 / 182; 2.5 M, 38 M 337 /
+// 252, 4 M, 61 M 538 / 379.
+bool long_rows_beside(const gd_spmv_plan* p) {
+  return !p->sched.hub_row.empty() &&
+         (double)p->nnz * 8e-3 >= p->sched.max_row_len * 3.0 + 15000.0;
+}
+
 // Windows pay where x exceeds one XCD's 4 MB L2 and every window is filled
 // for at least about as many nonzeros as it holds columns (a piece of the
-// expand pass copies its window into LDS first).
+// expand pass copies its window into LDS first); long rows must not wait for
+// the expand pass.
 bool wants_windows(const gd_spmv_plan* p) {
   return (int64_t)p->cols * 4 > (4 << 20) && p->nnz >= 2 * (int64_t)p->cols &&
+         (p->sched.hub_row.empty() || long_rows_beside(p)) &&
+         p->sched.tiles.size() > p->sched.hub_row.size() &&  // rows in tiles
          window_gather_fits(p->cols, p->nnz, (int64_t)p->sched.tiles.size());
 }
 
@@ -197,11 +210,6 @@ int build_windows(gd_spmv_plan* p) {
     rc = build_window_gather(p->cols, in_tiles, segs, p->slot.as<int32_t>(), p->stream, &p->win);
   return rc;
 }
-
-// Power-law matrix, 2.5 M rows, 38 M nonzeros, longest row 73,996 (its chain
-// alone 220 us): 261 us; 333 in one launch, whose tiles run at 176 registers.
-// Below 2^22 nonzeros the tiles take less time than the fork and the join.
-constexpr int64_t kForkNnz = 1 << 22;
 
 }  // namespace
 
@@ -271,7 +279,7 @@ int gd_spmv_plan_create_ex(int rows, int cols, int64_t nnz, const int32_t* d_Ap,
                        [](const Tile& a, const Tile& b) { return a.w - a.z > b.w - b.z; });
       p->n_tiles = (int)row_tiles.size();
       p->n_hubs = (int)longs.size();
-      if (p->n_hubs && p->n_tiles && nnz >= kForkNnz &&
+      if (p->n_hubs && p->n_tiles && long_rows_beside(p) &&
           (hipStreamCreateWithFlags(&p->side, hipStreamNonBlocking) != hipSuccess ||
            hipEventCreateWithFlags(&p->fork_ev, hipEventDisableTiming) != hipSuccess ||
            hipEventCreateWithFlags(&p->join_ev, hipEventDisableTiming) != hipSuccess)) {
@@ -306,33 +314,36 @@ int gd_spmv_plan_run(gd_spmv_plan* p, const float* d_x, float* d_y) {
   GD_CHECK_ARG(p != nullptr, "NULL plan");
   if (p->rows == 0) return GD_OK;
   GD_CHECK_ARG(d_y != nullptr && (p->nnz == 0 || d_x != nullptr), "NULL x / y");
-  const bool fork = p->side != nullptr;
   auto run = [&](auto kernel, int n_tiles, int n_long, const int32_t* aj, const float* src,
                  hipStream_t s) {
     hipLaunchKernelGGL(kernel, dim3(n_tiles + n_long), dim3(kBlock), 0, s, p->tiles.as<Tile>(),
                        n_tiles, p->long_tiles.as<Tile>(), n_long, p->Ap, aj, p->pos.as<uint16_t>(),
                        p->e_max, p->Ax, src, d_y);
   };
-  if (fork) {  // the longest chains start first
+  hipStream_t ts = p->stream;
+  int n_long = p->n_hubs;
+  if (p->side) {  // long rows first, so that they are placed before the tiles fill the CUs
     GD_HIP_TRY(hipEventRecord(p->fork_ev, p->stream));
     GD_HIP_TRY(hipStreamWaitEvent(p->side, p->fork_ev, 0));
-    run(spmv_pull_kernel<true, false>, 0, p->n_hubs, p->Aj, d_x, p->side);
-    GD_HIP_TRY(hipEventRecord(p->join_ev, p->side));
+    ts = p->side;
+    run(spmv_pull_kernel<true, false>, 0, n_long, p->Aj, d_x, p->stream);
+    n_long = 0;
   }
-  const int n_long = fork ? 0 : p->n_hubs;
   if (p->win.on()) {
-    if (n_long) run(spmv_pull_kernel<true, false>, 0, n_long, p->Aj, d_x, p->stream);
-    hipLaunchKernelGGL(spmv_expand_kernel, dim3(p->win.n_pieces), dim3(kExpandBlock), 0, p->stream,
-                       d_x, p->cols, p->win.pieces.as<int4>(), p->win.sid.as<uint16_t>(),
+    hipLaunchKernelGGL(spmv_expand_kernel, dim3(p->win.n_pieces), dim3(kExpandBlock), 0, ts, d_x,
+                       p->cols, p->win.pieces.as<int4>(), p->win.sid.as<uint16_t>(),
                        p->win.stage.as<float>());
     run(spmv_pull_kernel<false, true>, p->n_tiles, 0, p->slot.as<int32_t>(),
-        p->win.stage.as<float>(), p->stream);
+        p->win.stage.as<float>(), ts);
   } else if (n_long) {
-    run(spmv_pull_kernel<true, false>, p->n_tiles, n_long, p->Aj, d_x, p->stream);
+    run(spmv_pull_kernel<true, false>, p->n_tiles, n_long, p->Aj, d_x, ts);
   } else if (p->n_tiles) {
-    run(spmv_pull_kernel<false, false>, p->n_tiles, 0, p->Aj, d_x, p->stream);
+    run(spmv_pull_kernel<false, false>, p->n_tiles, 0, p->Aj, d_x, ts);
   }
-  if (fork) GD_HIP_TRY(hipStreamWaitEvent(p->stream, p->join_ev, 0));
+  if (p->side) {
+    GD_HIP_TRY(hipEventRecord(p->join_ev, p->side));
+    GD_HIP_TRY(hipStreamWaitEvent(p->stream, p->join_ev, 0));
+  }
   GD_HIP_TRY(hipGetLastError());
   return GD_OK;
 }

@@ -38,6 +38,8 @@ CASES = [
     (70001, BASE + 32768, [31, 0, 64, 33, 1, 65, 17], "sorted"),
     (70001, BASE + 32769, [31, 0, 64, 33, 1, 65, 17], "ends"),
     (2100000, BASE + 100003, [1, 0, 2, 3, 0, 0, 1], "random"),        # tiles full of rows
+    (3000, 5000, [2049, 1500, 0, 9000, 700], "random"),               # side stream, no windows
+    (1200, BASE + 1, [3000], "random"),                               # long rows only
 ]
 
 
