@@ -69,6 +69,10 @@ struct MgArgs {
   float damp;
 };
 
+struct MgEpilogue : PrEpilogue<0> {
+  static constexpr int kWaveRowMin = 640;  // see kWaveRow
+};
+
 __global__ __launch_bounds__(kBlock) void mg_pull_kernel(const MgArgs a) {
   const int g = a.tile_graph[blockIdx.x];
   if (a.gs[g].done) return;
@@ -84,7 +88,7 @@ __global__ __launch_bounds__(kBlock) void mg_pull_kernel(const MgArgs a) {
   const Tile t = a.tiles[blockIdx.x];
   const PrGather gat{odd ? a.c1 : a.c0};
   double err = 0.0;
-  const PrEpilogue<0> e{a.scores, odd ? a.c0 : a.c1, a.outdeg, a.gs[g].base, a.damp, -1};
+  const MgEpilogue e{{a.scores, odd ? a.c0 : a.c1, a.outdeg, a.gs[g].base, a.damp, -1}};
   if (t.y >= 0) {
     err = row_tile<kMgIPT, false, true, decltype(gat), decltype(e), true>(
         a.off, a.col, a.pos, a.e_max, t.x, t.y, t.z, t.w - t.z, gat, e, lds.tile);

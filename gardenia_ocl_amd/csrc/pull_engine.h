@@ -134,7 +134,8 @@ __device__ __forceinline__ float lane_seq_sum(float s, const float* __restrict__
 // then up to 4 granules; terms outside the row are replaced by -0.0, which
 // added to any s gives s.  Reading the ends of a row term by term made each of
 // up to 34 terms wait for its own LDS read: the sums took 4-7 us of a row
-// tile's 11-16 us.
+// tile's 11-16 us.  The scheduling barriers keep a block's reads ahead of the
+// previous block's adds (20 iterations on 2000 vertices 284 to 272 us).
 __device__ __forceinline__ float seq_sum(float s, const float* __restrict__ v, int b, int e) {
   if (b >= e) return s;
   const float4* __restrict__ v4 = reinterpret_cast<const float4*>(v);
@@ -168,9 +169,13 @@ __device__ __forceinline__ float seq_sum(float s, const float* __restrict__ v, i
   int k = 0;
   for (; k + 2 <= nb; k += 2) {
     load(B, m0 + 4 * (k + 1));
+    __builtin_amdgcn_sched_barrier(0);
     add(A);
+    __builtin_amdgcn_sched_barrier(0);
     load(A, m0 + 4 * (k + 2));
+    __builtin_amdgcn_sched_barrier(0);
     add(B);
+    __builtin_amdgcn_sched_barrier(0);
   }
   if (k < nb) {
     load(B, t0);
@@ -624,12 +629,24 @@ __device__ __forceinline__ float segment_sum(const int32_t* __restrict__ col,
 // Rows of a tile longer than this are added by a wavefront (wave_exact_row)
 // where the epilogue's terms are never negative (E::kWaveRows); shorter ones
 // by their owner threads, side by side, which lasts as long as the longest.
+// A wavefront's sum of 512 .. 640 edges starts at about the cost of the chain;
+// with many small graphs in one launch, whose tiles share the CUs, the chain is
+// the cheaper one up to 640 (E::kWaveRowMin): 30 graphs of 500 .. 2000 vertices
+// 525 to 463 us.  One graph of 9001 .. 12000 vertices or 1 M: 512 is 1 to 8
+// percent faster than 640, 768 or 1024.
 constexpr int kWaveRow = 512;
 
 template <class E, class = void>
 struct wave_rows : std::false_type {};
 template <class E>
 struct wave_rows<E, std::void_t<decltype(E::kWaveRows)>> : std::bool_constant<E::kWaveRows> {};
+template <class E, class = void>
+struct wave_row_min : std::integral_constant<int, kWaveRow> {};
+template <class E>
+struct wave_row_min<E, std::void_t<decltype(E::kWaveRowMin)>>
+    : std::integral_constant<int, E::kWaveRowMin> {
+  static_assert(E::kWaveRowMin >= kWaveRow, "long_row holds NB * IPT / kWaveRow rows");
+};
 
 // LDS of one row tile of a workgroup of NB threads.
 template <int IPT, int NB = kBlock>
@@ -700,7 +717,7 @@ __device__ __forceinline__ double reduce_row_tile(int r0, int nr, const E& e,
     sum[q] = 0.0f;
     if (i < nr) {
       const int b = lds.off[i], en = lds.off[i + 1];
-      if (kWaves1 && en - b > kWaveRow) {
+      if (kWaves1 && en - b > wave_row_min<E>::value) {
         lds.long_row[atomicAdd(&lds.n_long, 1)] = (int16_t)i;
         lds.longsum[i] = e.init(pre[q]);
       } else if (SEQ_ALL || en - b <= kSeqRow)
@@ -723,7 +740,8 @@ __device__ __forceinline__ double reduce_row_tile(int r0, int nr, const E& e,
 #pragma unroll
       for (int q = 0; q < kRowsPerThread; q++) {
         const int i = tid + q * NB;
-        if (i < nr && lds.off[i + 1] - lds.off[i] > kWaveRow) sum[q] = lds.longsum[i];
+        if (i < nr && lds.off[i + 1] - lds.off[i] > wave_row_min<E>::value)
+          sum[q] = lds.longsum[i];
       }
     }
   }
