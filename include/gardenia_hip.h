@@ -346,7 +346,8 @@ int gd_spmv_plan_destroy(gd_spmv_plan *plan);
 
 /* SpMV modes.  All run the tile engine over the caller's CSR, every row in
  * CSR order, bit-identical to the reference; where x spans more than one
- * XCD's L2 (cols*4 > 4 MB) and nnz >= 2*cols, x is gathered through windows
+ * XCD's L2 (cols*4 > 4 MB) and nnz >= 2*cols, and the longest row's chain does
+ * not outlast the rest, x is gathered through windows
  * (the plan then holds 12 bytes per nonzero: slots, tile offsets, the expanded
  * x and its 16-bit sources).  A plan's runs share that buffer: they must not
  * overlap on the GPU (they run in order on the plan's stream).
