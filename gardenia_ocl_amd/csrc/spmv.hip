@@ -186,11 +186,13 @@ bool long_rows_beside(const gd_spmv_plan* p) {
 // Windows pay where x exceeds one XCD's 4 MB L2 and every window is filled
 // for at least about as many nonzeros as it holds columns (a piece of the
 // expand pass copies its window into LDS first); long rows must not wait for
-// the expand pass.
+// the expand pass.  Only nonzeros in row tiles count: long rows gather x
+// itself, and the tiles may hold none (empty rows beside long ones).
 bool wants_windows(const gd_spmv_plan* p) {
-  return (int64_t)p->cols * 4 > (4 << 20) && p->nnz >= 2 * (int64_t)p->cols &&
+  int64_t in_tiles = 0;
+  for (const Tile& t : p->sched.tiles) in_tiles += t.y >= 0 ? t.w - t.z : 0;
+  return (int64_t)p->cols * 4 > (4 << 20) && in_tiles >= 2 * (int64_t)p->cols &&
          (p->sched.hub_row.empty() || long_rows_beside(p)) &&
-         p->sched.tiles.size() > p->sched.hub_row.size() &&  // rows in tiles
          window_gather_fits(p->cols, p->nnz, (int64_t)p->sched.tiles.size());
 }
 

@@ -53,7 +53,7 @@ bool window_gather_fits(int n_src, int64_t nnz, int64_t segs);
 
 // Slots for the edges of the segments (x: first edge, y: edges; each
 // segment's sources ascending in `col`).  col[e] is replaced by the edge's
-// slot.  Synchronises `stream`.
+// slot.  Without segments the gather stays off.  Synchronises `stream`.
 int build_window_gather(int n_src, int64_t nnz, const std::vector<int2>& segs, int32_t* d_col,
                         hipStream_t stream, WindowGather* g);
 

@@ -80,6 +80,7 @@ int build_window_gather(int n_src, int64_t nnz, const std::vector<int2>& segs, i
                         hipStream_t stream, WindowGather* g) {
   const int windows = (int)(((int64_t)n_src + kWinSize - 1) >> kWinBits);
   const int64_t ns = (int64_t)segs.size();
+  if (ns == 0) return GD_OK;  // no edge to lay out: off
   const size_t table = (size_t)windows * ns;
   DeviceBuffer d_segs, cnt, at, start, tmp;
   int rc = d_segs.alloc(sizeof(int2) * (size_t)ns);
