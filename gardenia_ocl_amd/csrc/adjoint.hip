@@ -23,6 +23,7 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "gardenia_hip.h"
@@ -568,6 +569,7 @@ struct gd_spmv_bwd_plan {
   // x larger than one XCD's L2: dA reads x through windows (window_gather.h)
   WindowGather win;
   DeviceBuffer slot, pos;
+  std::mutex run_lock;  // a run's launches share `at`, vperm and win: threads queue whole runs
   ~gd_spmv_bwd_plan() {
     gd_spmv_plan_destroy(tplan);
   }
@@ -673,6 +675,7 @@ int gd_spmv_bwd_run(gd_spmv_bwd_plan* p, const float* d_Ax, const float* d_x, co
                     float* d_dx, float* d_dA) {
   GD_CHECK_ARG(p != nullptr, "NULL plan");
   GD_CHECK_ARG(p->rows == 0 || d_g, "NULL g");
+  const std::lock_guard<std::mutex> lock(p->run_lock);
   if (d_dx && p->cols > 0) {
     GD_CHECK_ARG(p->nnz == 0 || d_Ax, "NULL Ax");
     int rc = p->bucketed

@@ -22,6 +22,7 @@
 #include <algorithm>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "gardenia_hip.h"
@@ -141,6 +142,9 @@ struct gd_spmv_plan {
   // long rows on `stream`, the tiles beside them on `side` (long_rows_beside)
   hipStream_t side = nullptr;
   hipEvent_t fork_ev = nullptr, join_ev = nullptr;
+  // A run's launches pass x through `win` and order themselves by the events:
+  // host threads queue whole runs.
+  std::mutex run_lock;
   ~gd_spmv_plan() {
     if (fork_ev) (void)hipEventDestroy(fork_ev);
     if (join_ev) (void)hipEventDestroy(join_ev);
@@ -316,6 +320,8 @@ int gd_spmv_plan_run(gd_spmv_plan* p, const float* d_x, float* d_y) {
   GD_CHECK_ARG(p != nullptr, "NULL plan");
   if (p->rows == 0) return GD_OK;
   GD_CHECK_ARG(d_y != nullptr && (p->nnz == 0 || d_x != nullptr), "NULL x / y");
+  std::unique_lock<std::mutex> lock(p->run_lock, std::defer_lock);
+  if (p->side || p->win.on()) lock.lock();
   auto run = [&](auto kernel, int n_tiles, int n_long, const int32_t* aj, const float* src,
                  hipStream_t s) {
     hipLaunchKernelGGL(kernel, dim3(n_tiles + n_long), dim3(kBlock), 0, s, p->tiles.as<Tile>(),

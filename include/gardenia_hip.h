@@ -349,8 +349,10 @@ int gd_spmv_plan_destroy(gd_spmv_plan *plan);
  * XCD's L2 (cols*4 > 4 MB) and nnz >= 2*cols, and the longest row's chain does
  * not outlast the rest, x is gathered through windows
  * (the plan then holds 12 bytes per nonzero: slots, tile offsets, the expanded
- * x and its 16-bit sources).  A plan's runs share that buffer: they must not
- * overlap on the GPU (they run in order on the plan's stream).
+ * x and its 16-bit sources).  A plan's runs share the expanded x.  Host
+ * threads may run one plan at the same time: each run's launches are queued
+ * together on the plan's stream.  Graphs captured from a plan's runs must not
+ * be replayed beside one another, or beside its runs, on other streams.
  *   GD_SPMV_TILES   any matrix, any column order.
  *   GD_SPMV_SLICED  needs sorted columns per row (GD_ERR_INVALID otherwise).
  *                   Call gd_spmv_plan_refresh_values after changing d_Ax.
