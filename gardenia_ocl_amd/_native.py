@@ -183,6 +183,7 @@ SIGNATURES = {
                                   ctypes.POINTER(_P)]),
     "gd_pr_plan_create": (_i, [_i, _i64, _P, _P, _P, _P, ctypes.POINTER(_P)]),
     "gd_pr_plan_run": (_i, [_P, _P, ctypes.POINTER(PrOptions), ctypes.POINTER(PrStats), _P]),
+    "gd_pr_plan_windowed": (_i, [_P]),
     "gd_pr_plan_info": (_i, [_P, ctypes.POINTER(PrPlanInfo)]),
     "gd_pr_plan_destroy": (_i, [_P]),
     "gd_pr_solve": (_i, [_i, _i, _P, _P, _P, _P, _P, _P, ctypes.POINTER(PrOptions),
@@ -222,12 +223,15 @@ SIGNATURES = {
     "gd_wpr_forward": (_i, [_P, _P, ctypes.POINTER(PrOptions), ctypes.POINTER(PrStats), _P]),
     "gd_wpr_backward": (_i, [_P, _P, _P, _P, _P, ctypes.POINTER(PrOptions),
                              ctypes.POINTER(PrStats)]),
+    "gd_wpr_plan_windowed": (_i, [_P]),
     "gd_wpr_plan_destroy": (_i, [_P]),
     "gd_spmv_bwd_plan_create": (_i, [_i, _i, _i64, _P, _P, _P, ctypes.POINTER(_P)]),
     "gd_spmv_bwd_run": (_i, [_P, _P, _P, _P, _P, _P]),
+    "gd_spmv_bwd_plan_windowed": (_i, [_P]),
     "gd_spmv_bwd_plan_destroy": (_i, [_P]),
     "gd_spmv_plan_create": (_i, [_i, _i, _i64, _P, _P, _P, _P, ctypes.POINTER(_P)]),
     "gd_spmv_plan_create_ex": (_i, [_i, _i, _i64, _P, _P, _P, _P, _i, ctypes.POINTER(_P)]),
+    "gd_spmv_plan_windowed": (_i, [_P]),
     "gd_spmv_plan_mode": (_i, [_P]),
     "gd_spmv_plan_refresh_values": (_i, [_P]),
     "gd_spmv_plan_run": (_i, [_P, _P, _P]),

@@ -39,6 +39,12 @@ class WeightedPageRankPlan:
                ctypes.c_void_p(self.stream.cuda_stream), ctypes.byref(h))
         self._h = h
 
+    @property
+    def windowed(self) -> tuple:
+        """Whether the forward and the adjoint gather through windows."""
+        w = N.lib().gd_wpr_plan_windowed(self._h)
+        return bool(w & 1), bool(w & 2)
+
     def forward(self, x, *, damping=0.85, tol=1e-7, max_iter=200):
         opts = make_options(damping, tol, max_iter)
         st = N.PrStats()
@@ -106,6 +112,11 @@ class SpmvBackwardPlan:
         N.call("gd_spmv_bwd_plan_create", self.rows, self.cols, self.nnz, Ap.data_ptr(),
                Aj.data_ptr(), ctypes.c_void_p(self.stream.cuda_stream), ctypes.byref(h))
         self._h = h
+
+    @property
+    def windowed(self) -> bool:
+        """Whether dA reads x through windows."""
+        return bool(N.lib().gd_spmv_bwd_plan_windowed(self._h))
 
     def run(self, values, x, g, dx=None, dA=None):
         N.call("gd_spmv_bwd_run", self._h, values.data_ptr(), x.data_ptr(), g.data_ptr(),

@@ -450,6 +450,10 @@ int gd_wpr_plan_create(int m, int64_t nnz, const int32_t* d_off, const int32_t* 
   return GD_OK;
 }
 
+int gd_wpr_plan_windowed(const gd_wpr_plan* p) {
+  return p ? (p->fwd.win.on() ? 1 : 0) | (p->adj.win.on() ? 2 : 0) : 0;
+}
+
 int gd_wpr_plan_destroy(gd_wpr_plan* p) {
   if (!p) return GD_OK;
   gd_spmv_plan_destroy(p->qplan);
@@ -586,10 +590,30 @@ __global__ void bucket_keys_kernel(int64_t nnz, const int32_t* __restrict__ col,
     keys[e] = col[e] >> cshift;
 }
 
+// dA reads x through windows as the forward does (spmv.hip), but each value is
+// used once, with no row sum to wait for: up to twice the L2 plain gathers of
+// less spread columns are the faster ones.  us plain / windowed, 1.1 M columns x
+// 32: lines per nonzero 0.43 200 / 200, 0.78 216 / 200, 0.97 245 / 204; x 8 0.78
+// 50 / 55, 0.97 60 / 56; RMAT 1.2 M x 4 0.72 38 / 46.  4 M x 32 0.06 598 / 622,
+// 0.43 736 / 620; x 16 in runs of 4 0.25 316 / 333, of 2 0.50 507 / 333.
+int wants_windows(const gd_spmv_bwd_plan* p, bool* want) {
+  const int64_t cols = p->cols;
+  const bool large = cols > 2 << 20;
+  *want = p->rows > 0 && cols > 1 << 20 && p->nnz >= (large ? cols / 2 : 2 * cols) &&
+          window_gather_fits(p->cols, p->nnz, (int64_t)p->sched.tiles.size());
+  if (!*want) return GD_OK;
+  double lines = 0.0;
+  const int rc = gathered_lines(p->nnz, kBwdTile, p->Aj, p->stream, &lines);
+  *want = lines >= (large ? 0.45 : 0.75);
+  return rc;
+}
+
 }  // namespace
 }  // namespace gd
 
 extern "C" {
+
+int gd_spmv_bwd_plan_windowed(const gd_spmv_bwd_plan* p) { return p && p->win.on() ? 1 : 0; }
 
 int gd_spmv_bwd_plan_create(int rows, int cols, int64_t nnz, const int32_t* d_Ap,
                             const int32_t* d_Aj, void* stream, gd_spmv_bwd_plan** out) {
@@ -656,8 +680,10 @@ int gd_spmv_bwd_plan_create(int rows, int cols, int64_t nnz, const int32_t* d_Ap
                              p->at.as<float>(), stream, &p->tplan);
   }
   if (rc) return fail(rc);
-  if (rows > 0 && (int64_t)cols * 4 > (4 << 20) && nnz >= 2 * (int64_t)cols &&
-      window_gather_fits(cols, nnz, (int64_t)p->sched.tiles.size())) {
+  bool want = false;
+  rc = wants_windows(p, &want);
+  if (rc) return fail(rc);
+  if (want) {
     rc = p->slot.alloc(4 * (size_t)nnz);
     if (!rc) rc = p->pos.alloc(2 * (size_t)nnz);
     std::vector<int2> segs;

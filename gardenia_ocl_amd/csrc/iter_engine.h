@@ -35,6 +35,19 @@ struct wide_tiles<P, std::void_t<decltype(P::kWideTiles)>> : std::bool_constant<
 constexpr int kWindowMin = 1 << 21;
 constexpr int kWindowMinRelabelled = 7 << 20;
 
+// ... and only where tiles that run side by side share few lines: the gathers
+// of a grid, a band matrix or another order in which neighbours are near hit
+// the L2, and the windows' two passes are the longer ones.  Distinct lines per
+// edge of runs of kWindowRunEdges edges, us per iteration plain / windowed.
+// PageRank: grid of 9 M vertices 0.01, 96 / 213; 8 M vertices x 8 within 500 of
+// the row 0.004, 135 / 289, within 100,000 (original order) 0.10, 248 / 286;
+// 8 M x 16 in runs of 8 neighbours 0.12, 402 / 487, 3 M x 16 in runs of 4 0.23,
+// 216 / 213; RMAT 8 M x 8 0.31, 305 / 299; 8 M x 8 at random 0.87, 1056 / 289.
+// Weighted, forward and adjoint: 8 M x 8 within 100,000 0.10, 918 / 943; RMAT
+// 2.2 M x 16 0.27, 598 / 578.
+constexpr int kWindowRunEdges = 1 << 16;
+constexpr double kWindowLines = 0.2;
+
 struct IterEngine {
   int m = 0;
   int64_t nnz = 0;
@@ -47,7 +60,7 @@ struct IterEngine {
   int exact_len = 0;         // > 0: rows longer than this are whole-row exact hub tiles
   bool sort_tiles = false;   // gather each tile's edges in source order (tile_sort.h)
   // Windowed gather (window_gather.h) where the gathered vector exceeds an
-  // XCD's L2; sorted tiles only.
+  // XCD's L2 and the gathers are spread (kWindowLines); sorted tiles only.
   bool windows = false;
   int window_min = kWindowMin;
   WindowGather win;
@@ -145,8 +158,14 @@ struct IterEngine {
       }
       // exact hub rows are kept in edge order, or sorted in staging blocks
       const int64_t segs = (int64_t)sched.tiles.size() + nnz / kScanChunk + sched.n_slots;
-      const bool win_on = windows && stage_hubs != 0 && !persistent && m > window_min &&
-                          window_gather_fits(m, nnz, segs);
+      bool win_on = windows && stage_hubs != 0 && !persistent && m > window_min &&
+                    window_gather_fits(m, nnz, segs);
+      if (win_on) {
+        double lines = 0.0;
+        rc = gathered_lines(nnz, kWindowRunEdges, col, stream, &lines);
+        if (rc) return rc;
+        win_on = lines >= kWindowLines;
+      }
       std::vector<int2> seg;
       rc = build_tile_sort(sched, block * ipt, col, dst, pos.as<uint16_t>(), stream,
                            exact_len > 0, win_on ? kScanChunk : 0, &seg);

@@ -193,6 +193,8 @@ int gd_pr_plan_create(int m, int64_t nnz, const int32_t* d_off, const int32_t* d
   return gd_pr_plan_create_ex(m, nnz, d_off, d_col, d_outdeg, stream, nullptr, out);
 }
 
+int gd_pr_plan_windowed(const gd_pr_plan* p) { return p && p->eng.win.on() ? 1 : 0; }
+
 int gd_pr_plan_info(const gd_pr_plan* p, gd_pr_plan_info_t* info) {
   GD_CHECK_ARG(p != nullptr && info != nullptr, "NULL plan / info");
   info->n_tiles = p->eng.n_tiles + p->eng.n_hub_tiles;

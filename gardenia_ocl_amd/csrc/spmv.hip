@@ -187,17 +187,37 @@ bool long_rows_beside(const gd_spmv_plan* p) {
          (double)p->nnz * 8e-3 >= p->sched.max_row_len * 3.0 + 15000.0;
 }
 
-// Windows pay where x exceeds one XCD's 4 MB L2 and every window is filled
-// for at least about as many nonzeros as it holds columns (a piece of the
-// expand pass copies its window into LDS first); long rows must not wait for
-// the expand pass.  Only nonzeros in row tiles count: long rows gather x
-// itself, and the tiles may hold none (empty rows beside long ones).
-bool wants_windows(const gd_spmv_plan* p) {
+// Windows pay where x exceeds one XCD's 4 MB L2, its windows are filled for
+// enough nonzeros (a piece of the expand pass copies its window into LDS
+// first), and a tile gathers from many lines of x: the gathers of a band or of
+// columns in runs hit the L1 and L2.  Only nonzeros in row tiles count: long
+// rows gather x itself, and must not wait for the expand pass.
+// us plain / windowed, nonzeros per column at random: 1 M columns x 1 14.5 /
+// 17.2, 1.2 M x 1 14.7 / 15.6, x 2 21.7 / 19.4; 2 M x 1 31.5 / 23.2, 4 M x 0.5
+// 36 / 21, x 1.75 107 / 40.
+// Lines per nonzero: 4 M x 32 within 250 of the row 0.01, 230 / 511, within
+// 16,000 0.43, 573 / 510; 4 M x 16 in runs of 4 0.25, 308 / 280, of 2 0.50, 503
+// / 280.  Up to twice the L2 most of x stays there: 1.1 M x 16 in runs of 2
+// 0.49, 68 / 77, x 8 within 16,000 0.43, 42.5 / 45.5, within 64,000 0.78, 47.8 /
+// 45.3.
+int wants_windows(const gd_spmv_plan* p, bool* want) {
   int64_t in_tiles = 0;
-  for (const Tile& t : p->sched.tiles) in_tiles += t.y >= 0 ? t.w - t.z : 0;
-  return (int64_t)p->cols * 4 > (4 << 20) && in_tiles >= 2 * (int64_t)p->cols &&
-         (p->sched.hub_row.empty() || long_rows_beside(p)) &&
-         window_gather_fits(p->cols, p->nnz, (int64_t)p->sched.tiles.size());
+  std::vector<int2> runs;
+  for (const Tile& t : p->sched.tiles) {
+    if (t.y < 0 || t.w == t.z) continue;
+    runs.push_back(make_int2(t.z, t.w - t.z));
+    in_tiles += t.w - t.z;
+  }
+  const int64_t cols = p->cols;
+  const bool large = cols > 2 << 20;
+  *want = cols > 1 << 20 && in_tiles >= (large ? cols / 2 : 2 * cols) &&
+          (p->sched.hub_row.empty() || long_rows_beside(p)) &&
+          window_gather_fits(p->cols, p->nnz, (int64_t)p->sched.tiles.size());
+  if (!*want) return GD_OK;
+  double lines = 0.0;
+  const int rc = gathered_lines(runs, p->Aj, p->stream, &lines);
+  *want = lines >= (large ? 0.45 : 0.6);
+  return rc;
 }
 
 int build_windows(gd_spmv_plan* p) {
@@ -271,7 +291,11 @@ int gd_spmv_plan_create_ex(int rows, int cols, int64_t nnz, const int32_t* d_Ap,
         if (rc == GD_ERR_INVALID && mode == GD_SPMV_AUTO) rc = GD_OK;  // unsorted rows: tiles
       }
     }
-    if (!rc && wants_windows(p)) rc = build_windows(p);
+    if (!rc && nnz > 0) {
+      bool want = false;
+      rc = wants_windows(p, &want);
+      if (!rc && want) rc = build_windows(p);
+    }
     if (!rc && nnz == 0) {
       rc = p->dummy_col.alloc(4);
       if (!rc && hipMemsetAsync(p->dummy_col.ptr, 0, 4, p->stream) != hipSuccess) rc = GD_ERR_DEVICE;
@@ -364,6 +388,8 @@ int gd_spmv_plan_refresh_values(gd_spmv_plan* p) {
 int gd_spmv_plan_mode(const gd_spmv_plan* p) {
   return p == nullptr ? -1 : (p->sliced ? GD_SPMV_SLICED : GD_SPMV_TILES);
 }
+
+int gd_spmv_plan_windowed(const gd_spmv_plan* p) { return p && p->win.on() ? 1 : 0; }
 
 int gd_spmv_plan_info(const gd_spmv_plan* p, int64_t* n_tiles, int64_t* n_hubs,
                       int32_t* max_row_len) {

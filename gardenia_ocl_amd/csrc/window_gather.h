@@ -51,6 +51,18 @@ struct WindowGather {
 // 32-bit slots).
 bool window_gather_fits(int n_src, int64_t nnz, int64_t segs);
 
+// Distinct 128-byte lines of the gathered float vector per edge, each of the
+// runs of edges (x: first, y: edges) by itself, over up to kLineRuns of them
+// spread evenly: about 1 for sources at random, 1/32 for neighbouring ones.
+// What the gathers of a workgroup, or of those that run side by side, share in
+// the caches.  Synchronises `stream`.
+constexpr int kLineRuns = 512;
+int gathered_lines(const std::vector<int2>& runs, const int32_t* d_col, hipStream_t stream,
+                   double* lines_per_edge);
+// The same over runs of `run` edges of all nnz.
+int gathered_lines(int64_t nnz, int run, const int32_t* d_col, hipStream_t stream,
+                   double* lines_per_edge);
+
 // Slots for the edges of the segments (x: first edge, y: edges; each
 // segment's sources ascending in `col`).  col[e] is replaced by the edge's
 // slot.  Without segments the gather stays off.  Synchronises `stream`.

@@ -68,7 +68,68 @@ __global__ void window_starts_kernel(int windows, int64_t segs, const int32_t* _
   if (w < windows) start[w] = at[(int64_t)w * segs];
 }
 
+// lines[b] = distinct lines of 32 sources among the edges of the b-th range
+// (x: first edge, y: edges).  A bit of LDS per line; vectors of more than
+// 2^25 sources have several lines to a bit.
+constexpr int kLineBits = 1 << 20;
+
+__global__ __launch_bounds__(kExpandBlock) void count_lines_kernel(
+    const int2* __restrict__ range, const int32_t* __restrict__ col, int32_t* __restrict__ lines) {
+  __shared__ uint32_t s_set[kLineBits / 32];
+  __shared__ int s_n;
+  for (int i = threadIdx.x; i < kLineBits / 32; i += kExpandBlock) s_set[i] = 0u;
+  if (threadIdx.x == 0) s_n = 0;
+  __syncthreads();
+  const int2 g = range[blockIdx.x];
+  int mine = 0;
+  for (int i = threadIdx.x; i < g.y; i += kExpandBlock) {
+    const uint32_t line = ((uint32_t)col[g.x + i] >> 5) % kLineBits, bit = 1u << (line & 31);
+    mine += (atomicOr(&s_set[line >> 5], bit) & bit) == 0u;
+  }
+  atomicAdd(&s_n, mine);
+  __syncthreads();
+  if (threadIdx.x == 0) lines[blockIdx.x] = s_n;
+}
+
 }  // namespace
+
+int gathered_lines(const std::vector<int2>& runs, const int32_t* d_col, hipStream_t stream,
+                   double* lines_per_edge) {
+  *lines_per_edge = 0.0;
+  std::vector<int2> range;
+  int64_t edges = 0;
+  const size_t step = std::max<size_t>(1, runs.size() / kLineRuns);
+  for (size_t i = 0; i < runs.size(); i += step) {
+    range.push_back(runs[i]);
+    edges += runs[i].y;
+  }
+  if (edges == 0) return GD_OK;
+  DeviceBuffer d_range, d_lines;
+  int rc = d_range.alloc(sizeof(int2) * range.size());
+  if (!rc) rc = d_lines.alloc(4 * range.size());
+  if (rc) return rc;
+  std::vector<int32_t> lines(range.size());
+  GD_HIP_TRY(hipMemcpyAsync(d_range.ptr, range.data(), sizeof(int2) * range.size(),
+                            hipMemcpyHostToDevice, stream));
+  hipLaunchKernelGGL(count_lines_kernel, dim3((unsigned)range.size()), dim3(kExpandBlock), 0,
+                     stream, d_range.as<int2>(), d_col, d_lines.as<int32_t>());
+  GD_HIP_TRY(hipGetLastError());
+  GD_HIP_TRY(hipMemcpyAsync(lines.data(), d_lines.ptr, 4 * range.size(), hipMemcpyDeviceToHost,
+                            stream));
+  GD_HIP_TRY(hipStreamSynchronize(stream));
+  int64_t n = 0;
+  for (const int32_t l : lines) n += l;
+  *lines_per_edge = (double)n / (double)edges;
+  return GD_OK;
+}
+
+int gathered_lines(int64_t nnz, int run, const int32_t* d_col, hipStream_t stream,
+                   double* lines_per_edge) {
+  std::vector<int2> runs;
+  for (int64_t e = 0; e < nnz; e += run)
+    runs.push_back(make_int2((int)e, (int)std::min<int64_t>(run, nnz - e)));
+  return gathered_lines(runs, d_col, stream, lines_per_edge);
+}
 
 bool window_gather_fits(int n_src, int64_t nnz, int64_t segs) {
   const int64_t windows = ((int64_t)n_src + kWinSize - 1) >> kWinBits;

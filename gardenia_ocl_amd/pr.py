@@ -222,6 +222,11 @@ class PageRankPlan:
                ctypes.c_void_p(self.stream.cuda_stream), ctypes.byref(cfg), ctypes.byref(h))
         self._h = h
 
+    @property
+    def windowed(self) -> bool:
+        """Whether the plan gathers through windows of the source vector."""
+        return bool(N.lib().gd_pr_plan_windowed(self._h))
+
     def info(self) -> dict:
         inf = N.PrPlanInfo()
         N.call("gd_pr_plan_info", self._h, ctypes.byref(inf))

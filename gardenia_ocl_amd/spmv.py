@@ -76,6 +76,11 @@ class SpmvPlan:
         reads Ax itself on each run)."""
         N.call("gd_spmv_plan_refresh_values", self._h)
 
+    @property
+    def windowed(self) -> bool:
+        """Whether the plan gathers through windows of the source vector."""
+        return bool(N.lib().gd_spmv_plan_windowed(self._h))
+
     def info(self) -> dict:
         t, hb = ctypes.c_int64(), ctypes.c_int64()
         mx = ctypes.c_int32()

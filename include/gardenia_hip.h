@@ -147,6 +147,11 @@ int gd_pr_plan_run(gd_pr_plan *plan, float *d_scores, const gd_pr_options *opts,
                    gd_pr_stats *stats, double *errors);
 
 int gd_pr_plan_info(const gd_pr_plan *plan, gd_pr_plan_info_t *info);
+/* 1 if the plan gathers through windows of the source vector, else 0: more than
+ * 2^21 vertices (7 * 2^20 relabelled), sort_tiles, no persistent grid,
+ * stage_hubs not 0, and sources spread over many cache lines.  A windowed plan
+ * stages every hub row and holds 6 bytes per edge more. */
+int gd_pr_plan_windowed(const gd_pr_plan *plan);
 
 int gd_pr_plan_destroy(gd_pr_plan *plan);
 
@@ -346,8 +351,9 @@ int gd_spmv_plan_destroy(gd_spmv_plan *plan);
 
 /* SpMV modes.  All run the tile engine over the caller's CSR, every row in
  * CSR order, bit-identical to the reference; where x spans more than one
- * XCD's L2 (cols*4 > 4 MB) and nnz >= 2*cols, and the longest row's chain does
- * not outlast the rest, x is gathered through windows
+ * XCD's L2 (cols*4 > 4 MB), nnz >= 2*cols (cols/2 above 2^21 columns), a tile's
+ * nonzeros are spread over many cache lines of x, and the longest row's chain
+ * does not outlast the rest, x is gathered through windows
  * (the plan then holds 12 bytes per nonzero: slots, tile offsets, the expanded
  * x and its 16-bit sources).  A plan's runs share the expanded x.  Host
  * threads may run one plan at the same time: each run's launches are queued
@@ -366,6 +372,9 @@ int gd_spmv_plan_create_ex(int num_rows, int num_cols, int64_t nnz, const int32_
 
 /* Mode the plan runs in (GD_SPMV_TILES or GD_SPMV_SLICED), -1 for NULL. */
 int gd_spmv_plan_mode(const gd_spmv_plan *plan);
+
+/* 1 if the plan gathers x through windows, else 0. */
+int gd_spmv_plan_windowed(const gd_spmv_plan *plan);
 
 /* To be called after d_Ax changed under a SLICED plan.  Every mode reads d_Ax
  * itself on each run, so there is nothing to copy. */
@@ -437,6 +446,9 @@ int gd_wpr_forward(gd_wpr_plan *plan, float *d_x, const gd_pr_options *opts, gd_
 int gd_wpr_backward(gd_wpr_plan *plan, const float *d_x, const float *d_w, float *d_lambda,
                     float *d_grad, const gd_pr_options *opts, gd_pr_stats *stats);
 
+/* As gd_pr_plan_windowed: 1 the forward, 2 the adjoint, 3 both. */
+int gd_wpr_plan_windowed(const gd_wpr_plan *plan);
+
 int gd_wpr_plan_destroy(gd_wpr_plan *plan);
 
 /* Backward of y = A x (+ y0): dx = A^T g (the SpMV engine over a CSC built once
@@ -449,6 +461,9 @@ int gd_spmv_bwd_plan_create(int num_rows, int num_cols, int64_t nnz, const int32
 
 int gd_spmv_bwd_run(gd_spmv_bwd_plan *plan, const float *d_Ax, const float *d_x, const float *d_g,
                     float *d_dx, float *d_dA);
+
+/* 1 if dA reads x through windows (as gd_spmv_plan_windowed), else 0. */
+int gd_spmv_bwd_plan_windowed(const gd_spmv_bwd_plan *plan);
 
 int gd_spmv_bwd_plan_destroy(gd_spmv_bwd_plan *plan);
 
