@@ -69,7 +69,7 @@ struct IterEngine {
   const int32_t* off = nullptr;
   const int32_t* col = nullptr;
   int e_max = 0;
-  DeviceBuffer dummy_col, col_sorted, pos;
+  DeviceBuffer dummy_col, col_sorted, pos, wave_from;
   Schedule sched;
   int n_tiles = 0, n_hubs = 0, n_hub_tiles = 0, fin_blocks = 1;
   bool fused = false;  // the pull launches finish each iteration (no finalize launch)
@@ -233,6 +233,13 @@ struct IterEngine {
       return n ? hipMemcpyAsync(b.ptr, src, n, hipMemcpyHostToDevice, stream) : hipSuccess;
     };
     GD_HIP_TRY(up(tiles, sched.tiles.data(), sizeof(Tile) * n_tiles));
+    rc = wave_from.alloc(4 * (size_t)std::max(1, n_tiles));
+    if (rc) return rc;
+    if (n_tiles) {
+      hipLaunchKernelGGL(wave_rows_kernel, dim3((n_tiles + kWaves - 1) / kWaves), dim3(kBlock), 0,
+                         stream, tiles.as<Tile>(), n_tiles, off, wave_from.as<int32_t>());
+      GD_HIP_TRY(hipGetLastError());
+    }
     GD_HIP_TRY(up(hub_row, sched.hub_row.data(), 4 * (size_t)n_hubs));
     GD_HIP_TRY(up(hub_slot, sched.hub_slot.data(), 4 * (size_t)n_hubs));
     GD_HIP_TRY(up(hub_nseg, sched.hub_nseg.data(), 4 * (size_t)n_hubs));
@@ -278,7 +285,7 @@ struct IterEngine {
                     hub_part.as<float>(), err_part.as<double>(), state.as<IterState>(),
                     fused ? parts : 0, errors.as<double>(),
                     staged ? hub_soff.as<int32_t>() : nullptr, stage.as<float>(),
-                    win.on() ? win.stage.as<float>() : nullptr};
+                    win.on() ? win.stage.as<float>() : nullptr, wave_from.as<int32_t>()};
   }
 
   // exact hubs finish their rows in the pull launch: no hub epilogues here

@@ -53,6 +53,7 @@ struct MgArgs {
   const int32_t* __restrict__ col;
   int e_max;
   const uint16_t* __restrict__ pos;  // each edge's offset in its tile (tile_sort.h)
+  const int32_t* __restrict__ wave_from;  // per tile: see wave_rows_kernel
   const int32_t* __restrict__ outdeg;
   float* __restrict__ scores;
   float* __restrict__ c0;
@@ -67,10 +68,6 @@ struct MgArgs {
   int max_iter;
   double tol;
   float damp;
-};
-
-struct MgEpilogue : PrEpilogue<0> {
-  static constexpr int kWaveRowMin = 640;  // see kWaveRow
 };
 
 __global__ __launch_bounds__(kBlock) void mg_pull_kernel(const MgArgs a) {
@@ -88,10 +85,11 @@ __global__ __launch_bounds__(kBlock) void mg_pull_kernel(const MgArgs a) {
   const Tile t = a.tiles[blockIdx.x];
   const PrGather gat{odd ? a.c1 : a.c0};
   double err = 0.0;
-  const MgEpilogue e{{a.scores, odd ? a.c0 : a.c1, a.outdeg, a.gs[g].base, a.damp, -1}};
+  const PrEpilogue<0> e{a.scores, odd ? a.c0 : a.c1, a.outdeg, a.gs[g].base, a.damp, -1};
   if (t.y >= 0) {
     err = row_tile<kMgIPT, false, true, decltype(gat), decltype(e), true>(
-        a.off, a.col, a.pos, a.e_max, t.x, t.y, t.z, t.w - t.z, gat, e, lds.tile);
+        a.off, a.col, a.pos, a.e_max, t.x, t.y, t.z, t.w - t.z, gat, e, lds.tile,
+        a.wave_from[blockIdx.x]);
   } else {  // whole hub row in the reference's order, as the single-graph plan
     const auto pre = e.pre(t.x);
     const float sum = exact_row_sum<false>(a.col, a.e_max, t.z, t.w - t.z, gat, e.init(pre),
@@ -175,7 +173,7 @@ struct gd_multi_pr_plan {
   hipStream_t user_stream = nullptr;
   hipStream_t stream = nullptr;  // private stream (graph capture needs a non-null one)
   std::vector<int32_t> m, vbase;
-  DeviceBuffer off, col, pos, deg, scores, c0, c1, tiles, tile_graph, hub_row, hub_slot, hub_nseg,
+  DeviceBuffer off, col, pos, wave_from, deg, scores, c0, c1, tiles, tile_graph, hub_row, hub_slot, hub_nseg,
       hub_part, err_part, gs, errors, d_vbase, d_user_ptrs;
   int n_tiles = 0;
   int e_max = 0;
@@ -296,6 +294,7 @@ int gd_multi_pr_plan_create(int n_graphs, const int32_t* m, const int64_t* nnz,
   }
   const int nh = (int)hub_row.size();
   rc = p->tiles.alloc(sizeof(Tile) * p->n_tiles);
+  if (!rc) rc = p->wave_from.alloc(4 * (size_t)p->n_tiles);
   if (!rc) rc = p->tile_graph.alloc(4 * (size_t)p->n_tiles);
   if (!rc) rc = p->hub_row.alloc(4 * (size_t)std::max(1, nh));
   if (!rc) rc = p->hub_slot.alloc(4 * (size_t)std::max(1, nh));
@@ -310,6 +309,11 @@ int gd_multi_pr_plan_create(int n_graphs, const int32_t* m, const int64_t* nnz,
     return n ? hipMemcpyAsync(b.ptr, src, n, hipMemcpyHostToDevice, p->stream) : hipSuccess;
   };
   GD_HIP_TRY(up(p->tiles, tiles.data(), sizeof(Tile) * p->n_tiles));
+  if (p->n_tiles)
+    hipLaunchKernelGGL(wave_rows_kernel, dim3((p->n_tiles + kWaves - 1) / kWaves), dim3(kBlock), 0,
+                       p->stream, p->tiles.as<Tile>(), p->n_tiles, p->off.as<int32_t>(),
+                       p->wave_from.as<int32_t>());
+  GD_HIP_TRY(hipGetLastError());
   GD_HIP_TRY(up(p->tile_graph, tile_graph.data(), 4 * (size_t)p->n_tiles));
   GD_HIP_TRY(up(p->hub_row, hub_row.data(), 4 * (size_t)nh));
   GD_HIP_TRY(up(p->hub_slot, hub_slot.data(), 4 * (size_t)nh));
@@ -358,7 +362,8 @@ int gd_multi_pr_run(gd_multi_pr_plan* p, float* const* d_scores, const gd_pr_opt
   GD_HIP_TRY(hipMemcpyAsync(p->d_user_ptrs.ptr, d_scores, sizeof(float*) * G,
                             hipMemcpyHostToDevice, p->stream));
   const MgArgs a{p->tiles.as<Tile>(), p->tile_graph.as<int32_t>(), p->off.as<int32_t>(),
-                 p->col.as<int32_t>(), p->e_max, p->pos.as<uint16_t>(), p->deg.as<int32_t>(), p->scores.as<float>(),
+                 p->col.as<int32_t>(), p->e_max, p->pos.as<uint16_t>(),
+                 p->wave_from.as<int32_t>(), p->deg.as<int32_t>(), p->scores.as<float>(),
                  p->c0.as<float>(), p->c1.as<float>(), p->hub_part.as<float>(),
                  p->err_part.as<double>(), p->gs.as<GraphState>(), p->hub_row.as<int32_t>(),
                  p->hub_slot.as<int32_t>(), p->hub_nseg.as<int32_t>(), p->errors.as<double>(),

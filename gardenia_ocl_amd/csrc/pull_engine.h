@@ -81,17 +81,15 @@ __device__ __forceinline__ T block_sum(T v, T* s_tmp) {
   return t;
 }
 
-// s + v[0] + ... + v[n-1] in order with FP32 rounding, by the calling lane,
-// from 16-byte aligned LDS: 4*kQ values per step, the next step's LDS reads in
-// flight while the current step is added (the adds are one dependent chain).
+// s + the first nb blocks of 4*kQ floats of v, in order with FP32 rounding, by
+// the calling lane, from 16-byte aligned LDS: the next block's reads in flight
+// while the current one is added (the adds are one dependent chain).
 // kQ = 8 (reads 32 terms ahead) hides the LDS latency behind the chain: at
 // RMAT-24 the pull phase took 1.339 ms against 1.367 ms with kQ = 4, at
-// RMAT-16 32.8 against 35.5 µs per iteration; kQ = 12 was no faster and costs
+// RMAT-16 32.8 against 35.5 us per iteration; kQ = 12 was no faster and costs
 // the row tiles 24 more VGPRs.
-template <int kQ>  // float4 reads per step
-__device__ __forceinline__ float lane_seq_sum(float s, const float* __restrict__ v, int n) {
-  const float4* __restrict__ v4 = reinterpret_cast<const float4*>(v);
-  const int nb = n / (4 * kQ);
+template <int kQ>  // float4 reads per block
+__device__ __forceinline__ float lane_chain(float s, const float4* __restrict__ v4, int nb) {
   float4 A[kQ], B[kQ];
   auto load = [&](float4(&R)[kQ], int blk) {
 #pragma unroll
@@ -123,20 +121,69 @@ __device__ __forceinline__ float lane_seq_sum(float s, const float* __restrict__
     }
     if (b < nb) add(A);
   }
+  return s;
+}
+
+// s + v[0] + ... + v[n-1], v 16-byte aligned.
+template <int kQ>
+__device__ __forceinline__ float lane_seq_sum(float s, const float* __restrict__ v, int n) {
+  const int nb = n / (4 * kQ);
+  s = lane_chain<kQ>(s, reinterpret_cast<const float4*>(v), nb);
   for (int i = nb * 4 * kQ; i < n; i++) s += v[i];
   return s;
 }
 
 // Sequential sum s + v[b] + ... + v[e-1] from LDS (`v` 16-byte aligned, the
 // granule of 4 that holds e - 1 readable) by the calling lane, in order with
-// FP32 rounding.  All reads are whole granules issued ahead of the adds that
-// need them: the row's first granule, blocks of 4 granules double-buffered,
-// then up to 4 granules; terms outside the row are replaced by -0.0, which
-// added to any s gives s.  Reading the ends of a row term by term made each of
-// up to 34 terms wait for its own LDS read: the sums took 4-7 us of a row
-// tile's 11-16 us.  The scheduling barriers keep a block's reads ahead of the
-// previous block's adds (20 iterations on 2000 vertices 284 to 272 us).
+// FP32 rounding.  All reads are whole granules, issued ahead of the adds that
+// need them; terms outside the row are replaced by -0.0, which added to any s
+// gives s.  (Reading the ends of a row term by term made each of up to 34 terms
+// wait for its own LDS read: the sums took 4-7 us of a row tile's 11-16 us.)
+//
+// seq_sum, for plans of many iterations over one graph: little code, since a
+// launch of a few tiles waits for its instructions most of the time.  Rows of
+// more than kChainRow terms take the first granule, blocks of 8 (lane_chain) and
+// the rest a granule at a time; shorter ones all of it that way, two granules
+// read ahead.
+// seq_sum_wide, for the others (SpMV, the adjoint): blocks of 4 granules
+// double-buffered, up to 4 granules at the end, unrolled.
+// us, seq_sum / seq_sum_wide: 20 PageRank iterations on 3,000 vertices x 24 264 /
+// 298, 9,001 x 32 298 / 350, 1,000 x 4 206 / 215; 64 graphs 3750 / 3851; but SpMV
+// 2^22 x 32 548 / 537, weighted RMAT-20 16,410 / 16,220.
+constexpr int kChainRow = 48;
+
 __device__ __forceinline__ float seq_sum(float s, const float* __restrict__ v, int b, int e) {
+  if (b >= e) return s;
+  const float4* __restrict__ v4 = reinterpret_cast<const float4*>(v);
+  const int g1 = (e + 3) >> 2;
+  int g = b >> 2;
+  auto add = [&](const float4& x) {  // granule g
+    const unsigned n = (unsigned)(e - b), o = (unsigned)(4 * g - b);
+    s += o < n ? x.x : -0.0f;
+    s += o + 1u < n ? x.y : -0.0f;
+    s += o + 2u < n ? x.z : -0.0f;
+    s += o + 3u < n ? x.w : -0.0f;
+    g++;
+  };
+  if (e - b > kChainRow) {
+    add(v4[g]);
+    const int nb = ((e >> 2) - g) >> 3;
+    s = lane_chain<8>(s, v4 + g, nb);
+    g += 8 * nb;
+    if (g >= g1) return s;
+  }
+  float4 x = v4[g], y = v4[min(g + 1, g1 - 1)];
+#pragma unroll 1
+  do {
+    const float4 z = v4[min(g + 2, g1 - 1)];
+    add(x);
+    x = y;
+    y = z;
+  } while (g < g1);
+  return s;
+}
+
+__device__ __forceinline__ float seq_sum_wide(float s, const float* __restrict__ v, int b, int e) {
   if (b >= e) return s;
   const float4* __restrict__ v4 = reinterpret_cast<const float4*>(v);
   const int g1 = (e + 3) >> 2, m0 = (b >> 2) + 1;
@@ -626,32 +673,42 @@ __device__ __forceinline__ float segment_sum(const int32_t* __restrict__ col,
   return block_sum<kWaves>(s, val);
 }
 
-// Rows of a tile longer than this are added by a wavefront (wave_exact_row)
-// where the epilogue's terms are never negative (E::kWaveRows); shorter ones
-// by their owner threads, side by side, which lasts as long as the longest.
-// A wavefront's sum of 512 .. 640 edges starts at about the cost of the chain;
-// with many small graphs in one launch, whose tiles share the CUs, the chain is
-// the cheaper one up to 640 (E::kWaveRowMin): 30 graphs of 500 .. 2000 vertices
-// 525 to 463 us.  One graph of 9001 .. 12000 vertices or 1 M: 512 is 1 to 8
-// percent faster than 640, 768 or 1024.
+// Where the epilogue's terms are never negative (E::kWaveRows), a tile whose
+// longest row exceeds kWaveTile has its rows of more than kWaveRow edges added
+// by a wavefront each (wave_exact_row), the shorter ones by their owner
+// threads, side by side.  The wavefronts start when the longest of those chains
+// (3 ns a term) has ended and cost about 2 us themselves, so a tile whose
+// longest row is near kWaveRow is better off with the chain.  20 iterations,
+// us, kWaveTile 512 / 1200 / 1536 / 2000: 5,000 vertices x 24 332 / 330 / 291 / 300,
+// 9,001 x 32 340 / 337 / 298 / 307, 12,000 x 8 338 / 331 / 292 / 299, 12,000 x 32 328
+// / 325 / 323 / 329.
 constexpr int kWaveRow = 512;
+constexpr int kWaveTile = 1536;
+constexpr int kNoWaveRows = 0x7fffffff;
 
 template <class E, class = void>
 struct wave_rows : std::false_type {};
 template <class E>
 struct wave_rows<E, std::void_t<decltype(E::kWaveRows)>> : std::bool_constant<E::kWaveRows> {};
-template <class E, class = void>
-struct wave_row_min : std::integral_constant<int, kWaveRow> {};
-template <class E>
-struct wave_row_min<E, std::void_t<decltype(E::kWaveRowMin)>>
-    : std::integral_constant<int, E::kWaveRowMin> {
-  static_assert(E::kWaveRowMin >= kWaveRow, "long_row holds NB * IPT / kWaveRow rows");
-};
+
+// from[t] = kWaveRow where tile t has wavefront rows, else kNoWaveRows; one
+// wavefront per tile.
+[[maybe_unused]] static __global__ __launch_bounds__(kBlock) void wave_rows_kernel(
+    const Tile* __restrict__ tiles, int n, const int32_t* __restrict__ off,
+    int32_t* __restrict__ from) {
+  const int t = blockIdx.x * kWaves + threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+  if (t >= n) return;
+  const Tile tile = tiles[t];
+  int longest = 0;
+  for (int r = tile.x + lane; r < tile.y; r += kWave) longest = max(longest, off[r + 1] - off[r]);
+  const bool any = __ballot(longest > kWaveTile) != 0;
+  if (lane == 0) from[t] = any ? kWaveRow : kNoWaveRows;
+}
 
 // LDS of one row tile of a workgroup of NB threads.
 template <int IPT, int NB = kBlock>
 struct RowTileLds {
-  alignas(16) float val[NB * IPT];           // gathered per-edge values
+  alignas(16) float val[NB * IPT + 4];       // gathered per-edge values, a spare place
   int off[kRowsPerThread * NB + 1];          // row offsets, rebased to the tile on use
   float longsum[kRowsPerThread * NB];        // sums of the rows that wavefronts add
   // rows of more than kWaveRow edges, added by a wavefront each (wave_rows epilogues)
@@ -706,7 +763,8 @@ __device__ __forceinline__ void issue_tile_loads(const Tile& t, const int32_t* _
 template <int IPT, class E, bool SEQ_ALL = false, int NB = kBlock>
 __device__ __forceinline__ double reduce_row_tile(int r0, int nr, const E& e,
                                                   const typename E::Pre (&pre)[kRowsPerThread],
-                                                  RowTileLds<IPT, NB>& lds) {
+                                                  RowTileLds<IPT, NB>& lds,
+                                                  int wave_from = kNoWaveRows) {
   const int tid = threadIdx.x;
   float sum[kRowsPerThread];
   bool have_long = false;
@@ -714,22 +772,23 @@ __device__ __forceinline__ double reduce_row_tile(int r0, int nr, const E& e,
 #pragma unroll
   for (int q = 0; q < kRowsPerThread; q++) {
     const int i = tid + q * NB;
-    sum[q] = 0.0f;
+    sum[q] = e.init(pre[q]);
     if (i < nr) {
       const int b = lds.off[i], en = lds.off[i + 1];
-      if (kWaves1 && en - b > wave_row_min<E>::value) {
+      if (kWaves1 && en - b > wave_from) {
         lds.long_row[atomicAdd(&lds.n_long, 1)] = (int16_t)i;
-        lds.longsum[i] = e.init(pre[q]);
+        lds.longsum[i] = sum[q];
       } else if (SEQ_ALL || en - b <= kSeqRow)
-        sum[q] = seq_sum(e.init(pre[q]), lds.val, b, en);
+        sum[q] = wave_rows<E>::value ? seq_sum(sum[q], lds.val, b, en)
+                                     : seq_sum_wide(sum[q], lds.val, b, en);
       else
         have_long = true;
     }
   }
   if constexpr (kWaves1) {
-    __syncthreads();
-    const int n = lds.n_long;
-    if (n) {
+    if (wave_from < kNoWaveRows) {
+      __syncthreads();
+      const int n = lds.n_long;
       for (int k = uniform((int)(tid / kWave)); k < n; k += NB / kWave) {
         const int row = uniform((int)lds.long_row[k]);
         const float s = wave_exact_row(uniform(lds.longsum[row]), lds.val, uniform(lds.off[row]),
@@ -740,8 +799,7 @@ __device__ __forceinline__ double reduce_row_tile(int r0, int nr, const E& e,
 #pragma unroll
       for (int q = 0; q < kRowsPerThread; q++) {
         const int i = tid + q * NB;
-        if (i < nr && lds.off[i + 1] - lds.off[i] > wave_row_min<E>::value)
-          sum[q] = lds.longsum[i];
+        if (i < nr && lds.off[i + 1] - lds.off[i] > wave_from) sum[q] = lds.longsum[i];
       }
     }
   }
@@ -774,7 +832,7 @@ __device__ __forceinline__ double reduce_row_tile(int r0, int nr, const E& e,
 #pragma unroll
     for (int q = 0; q < kRowsPerThread; q++) {
       const int i = tid + q * NB;
-      if (i < nr && lds.off[i + 1] - lds.off[i] > kSeqRow) sum[q] = e.init(pre[q]) + lds.longsum[i];
+      if (i < nr && lds.off[i + 1] - lds.off[i] > kSeqRow) sum[q] += lds.longsum[i];
     }
   }
   double acc = 0.0;
@@ -791,14 +849,19 @@ template <int IPT, bool SORTED, class Pre, int NB = kBlock>
 __device__ __forceinline__ void stage_row_tile(const Tile& t, const TileRegs<IPT, Pre, NB>& R,
                                                const float (&v)[IPT], RowTileLds<IPT, NB>& lds) {
   const int tid = threadIdx.x;
-  const int nr = t.y - t.x, ne = t.w - t.z;
+  const int ne = t.w - t.z;
   if (tid == 0) lds.n_long = 0;
+  // No branch per store: each was two jumps of instruction fetches (RMAT-16 10
+  // percent of its time).  Offsets past the tile's rows are off[nr] (clamped
+  // loads), values past its edges go to a spare place.
 #pragma unroll
   for (int q = 0; q < kOffLoads; q++)
-    if (tid + q * NB <= nr) lds.off[tid + q * NB] = R.offv[q] - t.z;
+    lds.off[min(tid + q * NB, kRowsPerThread * NB)] = R.offv[q] - t.z;
 #pragma unroll
-  for (int j = 0; j < IPT; j++)
-    if (tid + j * NB < ne) lds.val[SORTED ? R.pos[j] : tid + j * NB] = v[j];
+  for (int j = 0; j < IPT; j++) {
+    const int at = tid + j * NB;
+    lds.val[at < ne ? (SORTED ? R.pos[j] : at) : NB * IPT] = v[j];
+  }
 }
 
 // One row tile: rows [r0, r1) whose edges are [e0, e0+ne).  The epilogue E
@@ -814,11 +877,12 @@ __device__ __forceinline__ double row_tile(const int32_t* __restrict__ off,
                                            const int32_t* __restrict__ col,
                                            const uint16_t* __restrict__ pos, int e_max, int r0,
                                            int r1, int e0, int ne, const G& g, const E& e,
-                                           RowTileLds<IPT, NB>& lds) {
+                                           RowTileLds<IPT, NB>& lds,
+                                           int wave_from = kNoWaveRows) {
   const Tile t{r0, r1, e0, e0 + ne};
   TileRegs<IPT, typename E::Pre, NB> R;
   issue_tile_loads<IPT, NT, SORTED, E, NB>(t, off, col, pos, e_max, e, R);
-  float v[IPT];
+  float v[IPT] = {};
   if (ne > 0) gather_values<IPT, SORTED, G, NB>(g, e0, ne, R.idx, R.pos, v);
   if constexpr (SORTED && scaled_gather<G>::value) {
     float f[IPT];
@@ -829,7 +893,7 @@ __device__ __forceinline__ double row_tile(const int32_t* __restrict__ off,
     stage_row_tile<IPT, SORTED, typename E::Pre, NB>(t, R, v, lds);
   }
   __syncthreads();
-  return reduce_row_tile<IPT, E, SEQ_ALL, NB>(r0, r1 - r0, e, R.pre, lds);
+  return reduce_row_tile<IPT, E, SEQ_ALL, NB>(r0, r1 - r0, e, R.pre, lds, wave_from);
 }
 
 // ---------------------------------------------------------------------------

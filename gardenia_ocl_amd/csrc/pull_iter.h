@@ -70,6 +70,7 @@ struct IterArgs {
   // windowed plans: the values expanded by window_expand_kernel; `col` holds
   // each edge's slot in it (nullptr: `col` holds sources)
   const float* __restrict__ slots;
+  const int32_t* __restrict__ wave_from;  // per row tile: see wave_rows_kernel
 };
 
 // The gather of policy P: from the iteration's source vector, or from the
@@ -160,7 +161,8 @@ __device__ __forceinline__ void tile_body(const typename P::Args& a, const IterA
   if (t.y >= 0) {
     const auto e = P::template epilogue<NT>(a, odd);
     err = row_tile<IPT, (NT > 0), SORTED, decltype(g), decltype(e), P::kSeqAll, NB>(
-        it.off, it.col, it.pos, it.e_max, t.x, t.y, t.z, t.w - t.z, g, e, lds);
+        it.off, it.col, it.pos, it.e_max, t.x, t.y, t.z, t.w - t.z, g, e, lds,
+        wave_rows<decltype(e)>::value ? it.wave_from[b] : kNoWaveRows);
   } else if constexpr (!P::kExactHubs) {
     const float p = segment_sum<IPT, (NT > 0), SORTED>(it.col, it.pos, t.z, t.w - t.z, g, lds.val);
     if (threadIdx.x == 0) it.hub_part[-t.y - 1] = p;
@@ -213,7 +215,7 @@ __global__ __launch_bounds__(kBlock) void pull_persistent_kernel(const typename 
       const bool has_next = tn < it.n_tiles;
       const Tile nxt = it.tiles[has_next ? tn : t];
       const int ne = cur.w - cur.z;
-      float v[IPT];
+      float v[IPT] = {};
       if (ne > 0) gather_values<IPT, SORTED>(g, cur.z, ne, R.idx, R.pos, v);
       Regs Rn;
       // unconditional (clamped) so the compiler's wait counting stays exact
@@ -226,7 +228,8 @@ __global__ __launch_bounds__(kBlock) void pull_persistent_kernel(const typename 
           scale_tile<IPT>(lds.val, ne, f);
         }
         __syncthreads();
-        err += reduce_row_tile<IPT, decltype(e), P::kSeqAll>(cur.x, cur.y - cur.x, e, R.pre, lds);
+        err += reduce_row_tile<IPT, decltype(e), P::kSeqAll>(
+            cur.x, cur.y - cur.x, e, R.pre, lds, wave_rows<E>::value ? it.wave_from[t] : kNoWaveRows);
       } else if constexpr (!P::kExactHubs) {
         float sacc = 0.0f;
 #pragma unroll
