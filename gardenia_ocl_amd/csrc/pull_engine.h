@@ -367,13 +367,24 @@ template <int K>
 __device__ __forceinline__ float wave_exact_seg(float s, const float (&v)[K]) {
   const int lane = threadIdx.x & (kWave - 1);
   const bool negative = lane_negative<K>(v);
-  // terms of both signs: a lane at a time from the start
-  const bool mixed = __popcll(__ballot(negative)) > 4;
-  int from = 0;  // lanes before it are added
   s = uniform(s);
+  // Terms of both signs: a lane at a time from the start, nothing else in the
+  // loop (weighted PageRank, RMAT of 100,000 vertices, 2 percent of the weights
+  // negative, 20 iterations and the gradient: 1,473 us, 2,584 in the loop below).
+  if (__popcll(__ballot(negative)) > 4) {
+#pragma unroll 2
+    for (int f = 0; f < kWave; f++) {
+      float t = s;
+#pragma unroll
+      for (int k = 0; k < K; k++) t += v[k];
+      s = __uint_as_float(read_lane(__float_as_uint(t), f));
+    }
+    return s;
+  }
+  int from = 0;  // lanes before it are added
   for (;;) {
     int f = from;
-    if (in_binade(s) && !mixed) {
+    if (in_binade(s)) {
       const uint32_t base = binade(s), at = __float_as_uint(s) - base;
       bool stop;
       const Steps inc = wave_steps<K>(v, lane >= from, negative, base, stop);
