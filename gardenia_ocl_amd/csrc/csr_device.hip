@@ -197,18 +197,76 @@ __global__ __launch_bounds__(kB) void place_kernel(int64_t n, const int32_t* __r
   if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(&sc->bad, 1);
 }
 
-// Whether sorted record i is kept: not a self-loop (rm_self), and not equal
-// to the previous record that is no dropped self-loop (rm_dup).
-__device__ __forceinline__ bool record_kept(const uint64_t* __restrict__ key, int64_t i, uint64_t k,
-                                            const KeyFormat& kf, int rm_self, int rm_dup) {
-  if (rm_self && kf.row(k) == kf.col(k)) return false;
-  if (!rm_dup) return true;
-  for (int64_t j = i - 1; j >= 0; j--) {
-    const uint64_t p = key[j];
-    if (!rm_self || kf.row(p) != kf.col(p)) return p != k;
-    if (kf.row(p) != kf.row(k)) return true;  // the rows before hold no equal record
+// The record of one lane, the same for all.
+__device__ __forceinline__ uint64_t lane_record(uint64_t k, int lane) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)k, lane);
+  return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(k >> 32), lane) << 32) | lo;
+}
+
+// The last record before `i0` of row r that is no self-loop, by the wavefront:
+// 1024 records a step, since a row may hold any number of them.
+__device__ __forceinline__ bool last_no_loop(const uint64_t* __restrict__ key, int64_t i0, int32_t r,
+                                             const KeyFormat& kf, uint64_t* rec) {
+  const int lane = threadIdx.x & 63;
+  for (int64_t e = i0; e > 0; e -= kWaveRecs) {
+    uint64_t k[kWaveRecs / 64];
+#pragma unroll
+    for (int q = 0; q < kWaveRecs / 64; q++) k[q] = key[max(e - 1 - q * 64 - lane, (int64_t)0)];
+#pragma unroll
+    for (int q = 0; q < kWaveRecs / 64; q++) {
+      const bool ends = kf.row(k[q]) != r || kf.col(k[q]) != r || e - 1 - q * 64 - lane <= 0;
+      const uint64_t b = __ballot(ends);
+      if (b) {
+        *rec = lane_record(k[q], __builtin_ctzll(b));
+        return kf.row(*rec) == r && kf.col(*rec) != r;
+      }
+    }
   }
-  return true;
+  return false;
+}
+
+// The sorted records [1024 w, + 1024) in order, 64 at a time, by one wavefront:
+// f(index, in range, record, row of the record before it or -1, kept).  Kept: not
+// a self-loop (rm_self), and not equal to the last record before it that is no
+// dropped self-loop (rm_dup).  That record is one of the 64, or carried from
+// those before; only the wavefront's first record that is no loop may have to
+// look back over loops before the wavefront, and not in rows sorted by column,
+// where a row's records on the two sides of its loops differ.  (When every
+// record looked back by itself, 200,000 loops of one vertex ahead of 1 M edges
+// took 64 ms.)
+template <class F>
+__device__ __forceinline__ void for_records(int64_t n, int64_t w, const uint64_t* __restrict__ key,
+                                            const KeyFormat& kf, int rm_self, int rm_dup, F f) {
+  const int lane = threadIdx.x & 63;
+  const int64_t i0 = w * kWaveRecs;
+  auto loop = [&](uint64_t k) { return rm_self && kf.row(k) == kf.col(k); };
+  uint64_t last = key[max(i0 - 1, (int64_t)0)];  // the last that is no loop, if there is one
+  bool have = i0 > 0 && !loop(last);
+  if (i0 > 0 && !have && rm_dup && !kf.sorted) {
+    uint64_t b = 0;
+    for (int64_t i = i0 + lane; !b && i - lane < min(i0 + kWaveRecs, n); i += 64) {
+      const uint64_t k = key[min(i, n - 1)];
+      b = __ballot(i < n && !loop(k));
+      if (b) have = last_no_loop(key, i0, kf.row(lane_record(k, __builtin_ctzll(b))), kf, &last);
+    }
+  }
+#pragma unroll 4
+  for (int q = 0; q < kWaveRecs / 64; q++) {
+    const int64_t i = i0 + q * 64 + lane;
+    const uint64_t k = key[min(i, n - 1)], prev = key[max(min(i, n) - 1, (int64_t)0)];
+    const bool in = i < n, real = in && !loop(k);
+    const uint64_t b = __ballot(real);
+    const uint64_t lower = b & ((1ull << lane) - 1);
+    uint64_t near = prev;
+    if (b != __ballot(in))  // a loop among the 64
+      near = (uint64_t)__shfl((long long)k, lower ? 63 - __builtin_clzll(lower) : 0, 64);
+    const bool twin = lower ? near == k : have && last == k;
+    f(i, in, k, i > 0 ? kf.row(prev) : -1, real && !(rm_dup && twin));
+    if (b) {
+      last = lane_record(k, 63 - __builtin_clzll(b));
+      have = true;
+    }
+  }
 }
 
 // cnt[w] = records kept among sorted records [1024 w, + 1024), one wavefront each.
@@ -216,17 +274,12 @@ __global__ __launch_bounds__(kB) void kept_count_kernel(int64_t n, int64_t waves
                                                         const uint64_t* __restrict__ key,
                                                         KeyFormat kf, int rm_self, int rm_dup,
                                                         int64_t* __restrict__ cnt) {
-  const int lane = threadIdx.x & 63;
   const int64_t w = (int64_t)blockIdx.x * (kB / 64) + threadIdx.x / 64;
   if (w >= waves) return;
   int c = 0;
-#pragma unroll 4
-  for (int q = 0; q < kWaveRecs / 64; q++) {
-    const int64_t i = w * kWaveRecs + q * 64 + lane;
-    c += i < n && record_kept(key, i, key[i], kf, rm_self, rm_dup);
-  }
-  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
-  if (lane == 0) cnt[w] = c;
+  for_records(n, w, key, kf, rm_self, rm_dup,
+              [&](int64_t, bool, uint64_t, int32_t, bool keep) { c += __popcll(__ballot(keep)); });
+  if ((threadIdx.x & 63) == 0) cnt[w] = c;
 }
 
 // Writes the kept records (columns, weights) at their place, base[w] kept
@@ -242,26 +295,22 @@ __global__ __launch_bounds__(kB) void kept_write_kernel(
   const int64_t w = (int64_t)blockIdx.x * (kB / 64) + threadIdx.x / 64;
   if (w >= waves) return;
   int64_t at = base[w];
-#pragma unroll 4
-  for (int q = 0; q < kWaveRecs / 64; q++) {
-    const int64_t i = w * kWaveRecs + q * 64 + lane;
-    const uint64_t k = key[min(i, n - 1)];
-    const bool keep = i < n && record_kept(key, i, k, kf, rm_self, rm_dup);
-    const uint64_t b = __ballot(keep);
-    const int64_t p = at + __popcll(b & ((1ull << lane) - 1));
-    at += __popcll(b);
-    if (keep) {
-      col[p] = kf.col(k);
-      if (wout) wout[p] = rw ? rw[i] : 1.0f;
-    }
-    if (i < n) {
-      const int32_t r = kf.row(k);
-      const int32_t prev = i ? kf.row(key[i - 1]) : -1;
-      for (int32_t t = prev + 1; t <= r; t++) off[t] = (int32_t)p;
-      if (i == n - 1)
-        for (int32_t t = r + 1; t <= m; t++) off[t] = (int32_t)(p + keep);
-    }
-  }
+  for_records(n, w, key, kf, rm_self, rm_dup,
+              [&](int64_t i, bool in, uint64_t k, int32_t prev, bool keep) {
+                const uint64_t b = __ballot(keep);
+                const int64_t p = at + __popcll(b & ((1ull << lane) - 1));
+                at += __popcll(b);
+                if (keep) {
+                  col[p] = kf.col(k);
+                  if (wout) wout[p] = rw ? rw[i] : 1.0f;
+                }
+                if (in) {
+                  const int32_t r = kf.row(k);
+                  for (int32_t t = prev + 1; t <= r; t++) off[t] = (int32_t)p;
+                  if (i == n - 1)
+                    for (int32_t t = r + 1; t <= m; t++) off[t] = (int32_t)(p + keep);
+                }
+              });
 }
 
 __global__ void fill_kernel(int64_t n, int32_t v, int32_t* __restrict__ a) { GRID_LOOP(i, n) a[i] = v; }
