@@ -14,7 +14,7 @@
 //
 // Layout in HBM (built once per plan).  Every color is a contiguous range of
 // plan rows, its rows of at most kSeqRow (64) off-diagonal entries first, by
-// falling length, then its longer rows.
+// falling length (in chunks, kSortRows), then its longer rows.
 //
 // Short rows: slices of up to 64 rows (one wavefront, one lane a row), the
 // entries of a slice stored in 16-byte groups across its rows (group k of lane
@@ -48,6 +48,18 @@ namespace gd {
 namespace {
 
 constexpr int kSgXcds = 8;
+
+// Rows sorted by length together.  A slice of rows far apart gathers from as many
+// lines of x as rows, so rows of many lengths are sorted in chunks: 200,000 rows
+// of 1 .. 64 entries within 2000 columns, one sweep, all together / in chunks of
+// 64 / 256 / 1024: 203 / 115 / 113 / 129 us (LDS row tiles over a CSR 129); 1 M of
+// 1 .. 40 540 / 257 / 204 / 261 (267); 1 M of 18 .. 27 310 / 166 / 173 / 210 (265).
+// Where nearly all of a color's rows are of one length (large stencils), they
+// stay neighbours in either order, and all together leave fewer slices with two
+// lengths.  27-point stencils, two sweeps, all together / in chunks of 256: 126^3
+// (95 % of the rows inside) 355 / 422 us, 97^3 (94 %) 212 / 189, 80^3 (93 %) 170 /
+// 161, 40^3 (86 %) 121 / 115; 1 M rows, three quarters of one length 309 / 173.
+constexpr int kSortRows = 256;
 constexpr int64_t kSgDeltaMax = (1ll << 31) - 128;  // distances a plan stores at most
 
 // Up to 64 rows of one color.  A general slice (delta < 0) has `n` pairs of
@@ -101,16 +113,19 @@ __device__ __forceinline__ void row_update(const SymgsArgs& a, const RowRec& r, 
   if (r.diag != 0.0f) a.x[r.orig] = (bv - rsum) / r.diag;
 }
 
-// One general slice on one wavefront, two pairs (four entries) a step, the next
-// step's in flight.  More a step is slower (8 pairs: 261 us where 2 take 234,
-// a 27-point stencil of 97^3): neighbouring entries of a row often share a line
-// of x, which the first load of it must have brought in before the next asks.
+// One general slice on one wavefront, kP pairs of entries a step, the next
+// step's in flight.  Two pairs for rows of up to 12 entries, four for longer ones
+// (200,000 rows of 1 .. 64, one sweep: 167 us with two, 113 with four; 50,000 of
+// 1 .. 64 121 / 93).  Eight are faster for few rows (92) and slower for many (1 M
+// of 1 .. 40 204 us with four, 228 with eight): neighbouring entries of a row
+// often share a line of x, which the first load of it must have brought in before
+// the next asks.
 // The entries a lane reads past its row are the slice's padding or, past the
 // slice's end, its last pair again: their terms are replaced by -0.0, which
 // changes no sum.
+template <int kP>
 __device__ __forceinline__ float general_sum(const SymgsArgs& a, const Slice& sl,
                                              const RowRec& r, int lane) {
-  constexpr int kP = 2;
   const int4* __restrict__ e = a.ent + sl.off + lane;
   const int last = sl.n - 1;
   float sum = 0.0f;
@@ -173,7 +188,10 @@ __device__ __forceinline__ void slice_rows(const SymgsArgs& a, const Slice& sl, 
   if (lane >= sl.n_rows) return;
   const RowRec r = a.rows[sl.row0 + lane];
   const float bv = a.b[r.orig];
-  row_update(a, r, bv, sl.delta >= 0 ? uniform_sum(a, sl, r, lane) : general_sum(a, sl, r, lane));
+  row_update(a, r, bv,
+             sl.delta >= 0 ? uniform_sum(a, sl, r, lane)
+             : sl.len > 12 ? general_sum<4>(a, sl, r, lane)
+                           : general_sum<2>(a, sl, r, lane));
 }
 
 // The slice of workgroup b: the slices in 8 equal runs, one an XCD, since
@@ -445,9 +463,9 @@ int plan_build(gd_symgs_plan* p, int m, int64_t nnz, const int32_t* d_Ap, const 
     GD_HIP_TRY(hipMemcpyAsync(h_len.data(), len.ptr, 4 * (size_t)n_p, hipMemcpyDeviceToHost, s));
     GD_HIP_TRY(hipStreamSynchronize(s));
   }
-  // Per color: short rows by falling length (stable, so neighbours of one
-  // length stay neighbours), cut into slices; long rows, the longest first
-  // (the color lasts as long as its longest row).
+  // Per color: short rows by falling length, in chunks of kSortRows or all at
+  // once (stable, so neighbours of one length stay neighbours), cut into slices;
+  // long rows, the longest first (the color lasts as long as its longest row).
   std::vector<int32_t> h_order(n_p);
   std::vector<Slice> slices;
   std::vector<Tile> hubs;
@@ -457,24 +475,37 @@ int plan_build(gd_symgs_plan* p, int m, int64_t nnz, const int32_t* d_Ap, const 
   int64_t deltas = 0, hub_nnz = 0;
   for (int c = 0; c < C; c++) {
     const int r0 = co[c] - co[0], r1 = co[c + 1] - co[0];
-    int start[kSeqRow + 1] = {};  // rows of length l, then where they go
     longs.clear();
+    int rows_of[kSeqRow + 1] = {}, n_short = 0;
     for (int i = r0; i < r1; i++) {
       p->nnz_p += h_len[i];
       p->max_row_len = std::max(p->max_row_len, (int)h_len[i]);
-      if (h_len[i] <= kSeqRow)
-        start[h_len[i]]++;
-      else
+      if (h_len[i] <= kSeqRow) {
+        rows_of[h_len[i]]++;
+        n_short++;
+      } else {
         longs.push_back(i);
+      }
     }
+    const int most = *std::max_element(rows_of, rows_of + kSeqRow + 1);
+    const int chunk = 15 * (int64_t)most >= 14 * (int64_t)n_short ? std::max(n_short, 1) : kSortRows;
     int at = r0;
-    for (int l = kSeqRow; l >= 0; l--) {
-      const int n = start[l];
-      start[l] = at;
-      at += n;
+    for (int i0 = r0, i1; i0 < r1; i0 = i1) {
+      int start[kSeqRow + 1] = {};  // rows of length l, then where they go
+      int n = 0;
+      for (i1 = i0; i1 < r1 && n < chunk; i1++)
+        if (h_len[i1] <= kSeqRow) {
+          start[h_len[i1]]++;
+          n++;
+        }
+      for (int l = kSeqRow; l >= 0; l--) {
+        const int rows = start[l];
+        start[l] = at;
+        at += rows;
+      }
+      for (int i = i0; i < i1; i++)
+        if (h_len[i] <= kSeqRow) h_order[start[h_len[i]]++] = i;
     }
-    for (int i = r0; i < r1; i++)
-      if (h_len[i] <= kSeqRow) h_order[start[h_len[i]]++] = i;
     for (int q = r0; q < at; q += kWave) {
       const int n = std::min(kWave, at - q);
       const int len = h_len[h_order[q]];
