@@ -691,6 +691,12 @@ int gd_spmv_bwd_plan_create(int rows, int cols, int64_t nnz, const int32_t* d_Ap
       rc = build_tile_sort(p->sched, kBwdTile, d_Aj, p->slot.as<int32_t>(), p->pos.as<uint16_t>(),
                            p->stream, false, 0, &segs);
     if (!rc) rc = build_window_gather(cols, nnz, segs, p->slot.as<int32_t>(), p->stream, &p->win);
+    if (rc == GD_ERR_ALLOC) {  // no room for windows: x itself
+      p->win.release();
+      p->slot.release();
+      p->pos.release();
+      rc = GD_OK;
+    }
     if (rc) return fail(rc);
   }
   *out = owner.release();

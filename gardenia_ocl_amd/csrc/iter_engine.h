@@ -64,6 +64,7 @@ struct IterEngine {
   bool windows = false;
   int window_min = kWindowMin;
   WindowGather win;
+  bool hubs_sorted = false;  // exact hub rows lie sorted in staging blocks: always staged
   int32_t* col_owned = nullptr;  // the caller's private copy of col: sorted in place
   int pull_grid = 0;
   const int32_t* off = nullptr;
@@ -169,7 +170,14 @@ struct IterEngine {
       std::vector<int2> seg;
       rc = build_tile_sort(sched, block * ipt, col, dst, pos.as<uint16_t>(), stream,
                            exact_len > 0, win_on ? kScanChunk : 0, &seg);
-      if (!rc && win_on) rc = build_window_gather(m, nnz, seg, dst, stream, &win);
+      if (!rc && win_on) {
+        hubs_sorted = true;
+        rc = build_window_gather(m, nnz, seg, dst, stream, &win);
+        if (rc == GD_ERR_ALLOC) {  // no room for windows: the sources themselves
+          win.release();
+          rc = GD_OK;
+        }
+      }
       if (rc) return rc;
       col = dst;
     }
@@ -190,7 +198,7 @@ struct IterEngine {
       int64_t hub_edges = 0;
       for (const Tile& t : hubs) hub_edges += t.w - t.z;
       const int64_t longest = hubs[0].w - hubs[0].z;
-      const bool want = stage_hubs == 1 || win.on() ||
+      const bool want = stage_hubs == 1 || hubs_sorted ||
                         (stage_hubs < 0 && longest * 500 > (int64_t)nnz - hub_edges);
       std::vector<int32_t> soff(n_hub_tiles, -1);
       std::vector<int4> blocks;
@@ -266,8 +274,8 @@ struct IterEngine {
     // small iterations end in their last pull workgroup (fused_finish): no hub
     // segments to close, one finalize workgroup's worth of partials
     const int parts = (n_tiles > 0 ? pull_grid : 0) + n_hub_tiles;
-    fused = !persistent && block == kBlock && (exact_len > 0 || n_hubs == 0) && parts > 0 &&
-            parts < 2 * kBlock;
+    fused = !persistent && block == kBlock && !hubs_sorted && (exact_len > 0 || n_hubs == 0) &&
+            parts > 0 && parts < 2 * kBlock;
     if (fused && n_stage_blocks) {  // one-launch iterations gather their hubs themselves
       stage.release();
       stage_blocks.release();
@@ -316,7 +324,7 @@ struct IterEngine {
                          a, it, win.n_src, win.pieces.as<int4>(), win.sid.as<uint16_t>(),
                          win.stage.as<float>());
     // staged hubs: their values are gathered first, by the whole GPU
-    if (staged && win.on())
+    if (staged && hubs_sorted)
       hipLaunchKernelGGL((hub_stage_kernel<P, NT, true>), dim3(n_stage_blocks), dim3(kBlock), 0,
                          stream, a, it, stage_blocks.as<int4>(), stage.as<float>());
     else if (staged)

@@ -18,6 +18,7 @@ int DeviceBuffer::alloc(size_t n) {
   if (n == 0) n = 256;
   hipError_t e = hipMalloc(&ptr, n);
   if (e != hipSuccess) {
+    (void)hipGetLastError();  // reported here, not by the next launch's check
     ptr = nullptr;
     set_error(std::string("hipMalloc(") + std::to_string(n) + "): " + hipGetErrorString(e));
     return e == hipErrorOutOfMemory ? GD_ERR_ALLOC : GD_ERR_DEVICE;

@@ -295,6 +295,12 @@ int gd_spmv_plan_create_ex(int rows, int cols, int64_t nnz, const int32_t* d_Ap,
       bool want = false;
       rc = wants_windows(p, &want);
       if (!rc && want) rc = build_windows(p);
+      if (rc == GD_ERR_ALLOC) {  // no room for windows: x itself
+        p->win.release();
+        p->slot.release();
+        p->pos.release();
+        rc = GD_OK;
+      }
     }
     if (!rc && nnz == 0) {
       rc = p->dummy_col.alloc(4);

@@ -44,6 +44,12 @@ struct WindowGather {
   DeviceBuffer stage;   // float[slots]: the expanded values
   DeviceBuffer pieces;  // int4[n_pieces]: window's first source, first slot, end slot
   bool on() const { return n_pieces > 0; }
+  void release() {
+    sid.release();
+    stage.release();
+    pieces.release();
+    n_pieces = 0;
+  }
 };
 
 // Whether a layout of `segs` segments over n_src sources stays in bounds
@@ -65,7 +71,8 @@ int gathered_lines(int64_t nnz, int run, const int32_t* d_col, hipStream_t strea
 
 // Slots for the edges of the segments (x: first edge, y: edges; each
 // segment's sources ascending in `col`).  col[e] is replaced by the edge's
-// slot.  Without segments the gather stays off.  Synchronises `stream`.
+// slot.  Without segments the gather stays off; GD_ERR_ALLOC leaves `col` as it
+// is (a plan then gathers plainly).  Synchronises `stream`.
 int build_window_gather(int n_src, int64_t nnz, const std::vector<int2>& segs, int32_t* d_col,
                         hipStream_t stream, WindowGather* g);
 
