@@ -219,108 +219,102 @@ constexpr int kBwdTile = kBlock * 8;  // edges of a tile of the SpMV backward's 
 // Row tiles of at most this many edges label their edges' rows in LDS first.
 constexpr int kMapEdges = 4096;
 
-// Per-edge map over a CSR tile schedule: f(e, row, col) for every edge.  A row
-// tile's edge belongs to the unique row i with s_off[i] <= e < s_off[i + 1]
-// (s_off = the tile's offsets in LDS).  Up to kMapEdges edges, thread t finds
-// it for edges [t * per, + per) by one binary search and a forward walk and
-// stores it in a row table, so each edge then costs one LDS read; larger
-// tiles binary-search every edge.  A launch with gridDim.y > 1 splits each
-// one-row (hub) tile's edges over gridDim.y workgroups; row tiles need
-// gridDim.y == 1.
-//
-// WIN (windowed gather of the operand that the column selects): col holds
-// slots, sorted within each tile, with their offsets there in pos.  The
-// tile's values (f.slots) go to their CSR positions in LDS first, and f is
-// called with the value instead of the column.
-template <class F, bool WIN = false>
+// Rows of a row tile's edges, as a table in LDS: s_row[e - t.z] = the row i of
+// the tile with s_off[i] <= e < s_off[i + 1], for at most kMapEdges edges.
+// Thread i finds it for its edges [i * per, + per) by one binary search and a
+// forward walk.
+__device__ __forceinline__ void label_rows(const Tile& t, const int* s_off, uint16_t* s_row) {
+  const int nr = t.y - t.x, per = (t.w - t.z + kBlock - 1) / kBlock;
+  const int e0 = t.z + threadIdx.x * per, e1 = min(e0 + per, t.w);
+  if (e0 >= e1) return;
+  int lo = 0, hi = nr;  // s_off[0] = t.z <= e0 < t.w = s_off[nr]
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (s_off[mid] <= e0) lo = mid; else hi = mid;
+  }
+  int next = s_off[lo + 1];
+  for (int e = e0; e < e1; e++) {
+    while (next <= e) next = s_off[++lo + 1];  // stops below nr: s_off[nr] > e
+    s_row[e - t.z] = (uint16_t)lo;
+  }
+}
+
+// Per-edge map over a CSR tile schedule: f(e, row, col) for every edge.  Row
+// tiles of up to kMapEdges edges label their edges' rows first (label_rows), so
+// each edge then costs one LDS read; larger tiles binary-search every edge.  A
+// launch with gridDim.y > 1 splits each one-row (hub) tile's edges over
+// gridDim.y workgroups; row tiles need gridDim.y == 1.
+template <class F>
 __global__ __launch_bounds__(kBlock) void edge_map_kernel(const Tile* __restrict__ tiles,
                                                           const int32_t* __restrict__ off,
-                                                          const int32_t* __restrict__ col, F f,
-                                                          const uint16_t* __restrict__ pos = nullptr) {
-  constexpr int kEdges = WIN ? kBwdTile : kMapEdges;
+                                                          const int32_t* __restrict__ col, F f) {
   __shared__ int s_off[kTileRows + 1];
-  __shared__ uint16_t s_row[kEdges];
+  __shared__ uint16_t s_row[kMapEdges];
   static_assert(kTileRows <= 65536, "row table holds 16-bit tile rows");
-  const Tile t = tiles[WIN ? xcd_run_block(blockIdx.x, gridDim.x) : (int)blockIdx.x];
-  if constexpr (WIN) {  // tiles of at most kBwdTile edges, hub segments too
-    __shared__ float s_val[kBwdTile];
-    constexpr int kU = kBwdTile / kBlock;
-    const int n = t.w - t.z;
-    int slot[kU], p[kU];
-    float v[kU];
-#pragma unroll
-    for (int j = 0; j < kU; j++) {
-      const int e = t.z + min((int)threadIdx.x + j * kBlock, max(n - 1, 0));
-      slot[j] = n > 0 ? col[e] : 0;
-      p[j] = n > 0 ? pos[e] : 0;
-    }
-#pragma unroll
-    for (int j = 0; j < kU; j++) v[j] = f.slots[slot[j]];
-#pragma unroll
-    for (int j = 0; j < kU; j++)
-      if ((int)threadIdx.x + j * kBlock < n) s_val[p[j]] = v[j];
-    const int nr = t.y >= 0 ? t.y - t.x : 0;
-    for (int i = threadIdx.x; i <= nr; i += kBlock) s_off[i] = off[t.x + i];
-    __syncthreads();
-    if (t.y >= 0) {
-      const int per = (n + kBlock - 1) / kBlock;
-      const int e0 = t.z + threadIdx.x * per, e1 = min(e0 + per, t.w);
-      if (e0 < e1) {
-        int lo = 0, hi = nr;
-        while (hi - lo > 1) {
-          const int mid = (lo + hi) >> 1;
-          if (s_off[mid] <= e0) lo = mid; else hi = mid;
-        }
-        int next = s_off[lo + 1];
-        for (int e = e0; e < e1; e++) {
-          while (next <= e) next = s_off[++lo + 1];
-          s_row[e - t.z] = (uint16_t)lo;
-        }
-      }
-      __syncthreads();
-    }
-    for (int i = threadIdx.x; i < n; i += kBlock)
-      f(t.z + i, t.y >= 0 ? t.x + s_row[i] : t.x, s_val[i]);
-    return;
-  }
-  if constexpr (!WIN) {
-  if (t.y >= 0) {
-    const int nr = t.y - t.x;
-    for (int i = threadIdx.x; i <= nr; i += kBlock) s_off[i] = off[t.x + i];
-    __syncthreads();
-    const int n = t.w - t.z;
-    if (n <= kMapEdges) {
-      const int per = (n + kBlock - 1) / kBlock;
-      const int e0 = t.z + threadIdx.x * per, e1 = min(e0 + per, t.w);
-      if (e0 < e1) {
-        int lo = 0, hi = nr;  // s_off[0] = t.z <= e0 < t.w = s_off[nr]
-        while (hi - lo > 1) {
-          const int mid = (lo + hi) >> 1;
-          if (s_off[mid] <= e0) lo = mid; else hi = mid;
-        }
-        int next = s_off[lo + 1];
-        for (int e = e0; e < e1; e++) {
-          while (next <= e) next = s_off[++lo + 1];  // stops below nr: s_off[nr] > e
-          s_row[e - t.z] = (uint16_t)lo;
-        }
-      }
-      __syncthreads();
-      for (int e = t.z + threadIdx.x; e < t.w; e += kBlock) f(e, t.x + s_row[e - t.z], col[e]);
-      return;
-    }
-    for (int e = t.z + threadIdx.x; e < t.w; e += kBlock) {
-      int lo = 0, hi = nr;  // largest i with s_off[i] <= e
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (s_off[mid] <= e) lo = mid; else hi = mid;
-      }
-      f(e, t.x + lo, col[e]);
-    }
-  } else {
+  const Tile t = tiles[blockIdx.x];
+  if (t.y < 0) {
     for (int e = t.z + blockIdx.y * kBlock + threadIdx.x; e < t.w; e += kBlock * gridDim.y)
       f(e, t.x, col[e]);
+    return;
   }
+  const int nr = t.y - t.x;
+  for (int i = threadIdx.x; i <= nr; i += kBlock) s_off[i] = off[t.x + i];
+  __syncthreads();
+  if (t.w - t.z <= kMapEdges) {
+    label_rows(t, s_off, s_row);
+    __syncthreads();
+    for (int e = t.z + threadIdx.x; e < t.w; e += kBlock) f(e, t.x + s_row[e - t.z], col[e]);
+    return;
   }
+  for (int e = t.z + threadIdx.x; e < t.w; e += kBlock) {
+    int lo = 0, hi = nr;  // largest i with s_off[i] <= e
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (s_off[mid] <= e) lo = mid; else hi = mid;
+    }
+    f(e, t.x + lo, col[e]);
+  }
+}
+
+// The same over tiles (row tiles and hub segments) of at most kBwdTile edges
+// whose col holds slots of the operand that the column selects (a windowed
+// gather), sorted within each tile, with their offsets there in pos: the tile's
+// values (f.slots) go to their CSR positions in LDS first, and f is called with
+// the value instead of the column.
+template <class F>
+__global__ __launch_bounds__(kBlock) void slot_map_kernel(const Tile* __restrict__ tiles,
+                                                          const int32_t* __restrict__ off,
+                                                          const int32_t* __restrict__ col, F f,
+                                                          const uint16_t* __restrict__ pos) {
+  constexpr int kU = kBwdTile / kBlock;
+  static_assert(kBwdTile <= kMapEdges, "label_rows takes the whole tile");
+  __shared__ int s_off[kTileRows + 1];
+  __shared__ uint16_t s_row[kBwdTile];
+  __shared__ float s_val[kBwdTile];
+  const Tile t = tiles[xcd_run_block(blockIdx.x, gridDim.x)];
+  const int n = t.w - t.z;
+  int slot[kU], p[kU];
+  float v[kU];
+#pragma unroll
+  for (int j = 0; j < kU; j++) {
+    const int e = t.z + min((int)threadIdx.x + j * kBlock, max(n - 1, 0));
+    slot[j] = n > 0 ? col[e] : 0;
+    p[j] = n > 0 ? pos[e] : 0;
+  }
+#pragma unroll
+  for (int j = 0; j < kU; j++) v[j] = f.slots[slot[j]];
+#pragma unroll
+  for (int j = 0; j < kU; j++)
+    if ((int)threadIdx.x + j * kBlock < n) s_val[p[j]] = v[j];
+  if (t.y >= 0)
+    for (int i = threadIdx.x; i <= t.y - t.x; i += kBlock) s_off[i] = off[t.x + i];
+  __syncthreads();
+  if (t.y >= 0) {
+    label_rows(t, s_off, s_row);
+    __syncthreads();
+  }
+  for (int i = threadIdx.x; i < n; i += kBlock)
+    f(t.z + i, t.y >= 0 ? t.x + s_row[i] : t.x, s_val[i]);
 }
 
 struct WprGradOp {
@@ -531,7 +525,7 @@ int gd_wpr_backward(gd_wpr_plan* p, const float* d_x, const float* d_w, float* d
     // every edge once: the forward's row tiles, then its whole-row hub tiles
     if (p->fwd.n_tiles)
       hipLaunchKernelGGL(edge_map_kernel<WprGradOp>, dim3(p->fwd.n_tiles), dim3(kBlock), 0,
-                         p->stream, p->fwd.tiles.as<Tile>(), p->off, p->col, op, nullptr);
+                         p->stream, p->fwd.tiles.as<Tile>(), p->off, p->col, op);
     if (p->fwd.n_hub_tiles) {
       // one workgroup per 8 edges per thread of the longest hub
       const int split = std::min<int64_t>(
@@ -539,7 +533,7 @@ int gd_wpr_backward(gd_wpr_plan* p, const float* d_x, const float* d_w, float* d
                                        (kBlock * 8)));
       hipLaunchKernelGGL(edge_map_kernel<WprGradOp>, dim3(p->fwd.n_hub_tiles, split),
                          dim3(kBlock), 0, p->stream, p->fwd.hub_tiles.as<Tile>(), p->off, p->col,
-                         op, nullptr);
+                         op);
     }
     GD_HIP_TRY(hipGetLastError());
   }
@@ -726,7 +720,7 @@ int gd_spmv_bwd_run(gd_spmv_bwd_plan* p, const float* d_Ax, const float* d_x, co
                          p->stream, d_x, p->cols, p->win.pieces.as<int4>(),
                          p->win.sid.as<uint16_t>(), p->win.stage.as<float>());
       const SpmvDaSlotOp op{p->win.stage.as<float>(), d_g, d_dA};
-      hipLaunchKernelGGL((edge_map_kernel<SpmvDaSlotOp, true>), dim3(p->n_tiles), dim3(kBlock), 0,
+      hipLaunchKernelGGL(slot_map_kernel<SpmvDaSlotOp>, dim3(p->n_tiles), dim3(kBlock), 0,
                          p->stream, p->tiles.as<Tile>(), p->Ap, p->slot.as<int32_t>(), op,
                          p->pos.as<uint16_t>());
     } else {

@@ -85,7 +85,8 @@ struct IterEngine {
       errors;
   int errors_cap = 0;
   std::vector<hipEvent_t> ev;
-  // exact hubs run on a second stream, forked from / joined to `stream`
+  // beside exact hubs on `stream`, the row tiles of wider workgroups or a
+  // persistent grid run on a second stream, forked from / joined to it
   hipStream_t side = nullptr;
   hipEvent_t fork_ev = nullptr, join_ev = nullptr;
   // A chunk of iterations (identical launches) captured into a hipGraph when it
@@ -224,9 +225,11 @@ struct IterEngine {
                                   hipMemcpyHostToDevice, stream));
       }
       GD_HIP_TRY(hipStreamSynchronize(stream));  // host vectors go out of scope
-      GD_HIP_TRY(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
-      GD_HIP_TRY(hipEventCreateWithFlags(&fork_ev, hipEventDisableTiming));
-      GD_HIP_TRY(hipEventCreateWithFlags(&join_ev, hipEventDisableTiming));
+      if (persistent || block != kBlock) {  // else one launch takes hubs and row tiles
+        GD_HIP_TRY(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
+        GD_HIP_TRY(hipEventCreateWithFlags(&fork_ev, hipEventDisableTiming));
+        GD_HIP_TRY(hipEventCreateWithFlags(&join_ev, hipEventDisableTiming));
+      }
     }
     rc = tiles.alloc(sizeof(Tile) * std::max(1, n_tiles));
     if (!rc) rc = hub_row.alloc(4 * (size_t)std::max(1, n_hubs));
