@@ -560,8 +560,8 @@ struct gd_spmv_bwd_plan {
   DeviceBuffer tiles;
   int n_tiles = 0;
   gd_spmv_plan* tplan = nullptr;  // SpMV over the CSC: dx = A^T g
-  // g larger than one XCD's L2: A's values go into CSC order through buckets
-  // (vperm), in two passes whose scattered accesses stay in L2
+  // A's values go into CSC order through buckets (vperm), in two passes whose
+  // scattered accesses stay in L2 (wants_buckets), or by one gather
   bool bucketed = false;
   BucketedPermutation vperm;
   // x larger than one XCD's L2: dA reads x through windows (window_gather.h)
@@ -582,6 +582,23 @@ __global__ void bucket_keys_kernel(int64_t nnz, const int32_t* __restrict__ col,
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < nnz;
        e += (int64_t)gridDim.x * blockDim.x)
     keys[e] = col[e] >> cshift;
+}
+
+// Buckets pay where g exceeds one XCD's L2 and the values of a run of CSC entries
+// are spread: those of a band lie close together.  dx, us, one gather / buckets,
+// by lines per entry of runs of kValueRun: 2 M rows x 16 within 250 columns 0.04,
+// 201 / 307, within 4,000 0.09, 326 / 420, within 30,000 0.42, 413 / 458, within
+// 200,000 0.86, 690 / 453; 4 M x 16 in runs of 8 columns 0.13, 503 / 671; 2 M x 16
+// of 2 0.49, 574 / 466; RMAT 1.2 M x 4 0.54, 104 / 105, 2.5 M x 16 0.67, 740 / 699.
+constexpr int kValueRun = 1 << 16;
+
+int wants_buckets(const gd_spmv_bwd_plan* p, bool* want) {
+  *want = p->nnz > 0 && (int64_t)p->rows * 4 > (4 << 20);
+  if (!*want) return GD_OK;
+  double lines = 0.0;
+  const int rc = gathered_lines(p->nnz, kValueRun, p->tr.perm.as<int32_t>(), p->stream, &lines);
+  *want = lines >= 0.45;
+  return rc;
 }
 
 // dA reads x through windows as the forward does (spmv.hip), but each value is
@@ -648,7 +665,10 @@ int gd_spmv_bwd_plan_create(int rows, int cols, int64_t nnz, const int32_t* d_Ap
   if (rc) return fail(rc);
   GD_HIP_TRY(hipMemsetAsync(p->at.ptr, 0, 4 * (size_t)std::max<int64_t>(nnz, 1), p->stream));
   if (cols > 0) {
-    if (nnz > 0 && (int64_t)rows * 4 > (4 << 20)) {
+    bool buckets = false;
+    rc = wants_buckets(p, &buckets);
+    if (rc) return fail(rc);
+    if (buckets) {
       // buckets of about 2^18 entries: a range of A's columns, contiguous in
       // CSC order, so the second pass reads the buckets one after another
       p->bucketed = true;

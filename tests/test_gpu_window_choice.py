@@ -163,7 +163,19 @@ def test_sources_near_their_rows_stay_out_of_windows(device):
     plan.run(_t(device, x), y)
     np.testing.assert_array_equal(y.cpu().numpy(),
                                   oracle.spmv(m, off, col, val, x, np.zeros(m, np.float32)))
-    assert not SpmvBackwardPlan(_t(device, off), _t(device, col), m).windowed
+    bwd = SpmvBackwardPlan(_t(device, off), _t(device, col), m)
+    assert not bwd.windowed
+    g = rng.random(m, dtype=np.float32) - np.float32(0.5)
+    row = np.repeat(np.arange(m), k)
+    dx, dA = torch.empty(m, device=device), torch.empty(m * k, device=device)
+    bwd.run(_t(device, val), _t(device, x), _t(device, g), dx, dA)
+    np.testing.assert_array_equal(dA.cpu().numpy(), g[row] * x[col])
+    order = np.argsort(col, kind="stable")
+    toff = np.zeros(m + 1, np.int32)
+    np.cumsum(np.bincount(col, minlength=m), out=toff[1:])
+    np.testing.assert_array_equal(
+        dx.cpu().numpy(), oracle.spmv(m, toff, row[order].astype(np.int32), val[order], g,
+                                      np.zeros(m, np.float32)))
 
 
 @pytest.mark.parametrize("rows,cols,k,on", [
