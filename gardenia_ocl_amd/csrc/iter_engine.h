@@ -70,7 +70,7 @@ struct IterEngine {
   const int32_t* off = nullptr;
   const int32_t* col = nullptr;
   int e_max = 0;
-  DeviceBuffer dummy_col, col_sorted, pos, wave_from;
+  DeviceBuffer dummy_col, col_sorted, pos;
   Schedule sched;
   int n_tiles = 0, n_hubs = 0, n_hub_tiles = 0, fin_blocks = 1;
   bool fused = false;  // the pull launches finish each iteration (no finalize launch)
@@ -231,7 +231,7 @@ struct IterEngine {
         GD_HIP_TRY(hipEventCreateWithFlags(&join_ev, hipEventDisableTiming));
       }
     }
-    rc = tiles.alloc(sizeof(Tile) * std::max(1, n_tiles));
+    rc = tiles.alloc((sizeof(Tile) + 4) * std::max(1, n_tiles));  // and wave_from()
     if (!rc) rc = hub_row.alloc(4 * (size_t)std::max(1, n_hubs));
     if (!rc) rc = hub_slot.alloc(4 * (size_t)std::max(1, n_hubs));
     if (!rc) rc = hub_nseg.alloc(4 * (size_t)std::max(1, n_hubs));
@@ -244,11 +244,9 @@ struct IterEngine {
       return n ? hipMemcpyAsync(b.ptr, src, n, hipMemcpyHostToDevice, stream) : hipSuccess;
     };
     GD_HIP_TRY(up(tiles, sched.tiles.data(), sizeof(Tile) * n_tiles));
-    rc = wave_from.alloc(4 * (size_t)std::max(1, n_tiles));
-    if (rc) return rc;
     if (n_tiles) {
       hipLaunchKernelGGL(wave_rows_kernel, dim3((n_tiles + kWaves - 1) / kWaves), dim3(kBlock), 0,
-                         stream, tiles.as<Tile>(), n_tiles, off, wave_from.as<int32_t>());
+                         stream, tiles.as<Tile>(), n_tiles, off, wave_from());
       GD_HIP_TRY(hipGetLastError());
     }
     GD_HIP_TRY(up(hub_row, sched.hub_row.data(), 4 * (size_t)n_hubs));
@@ -288,6 +286,9 @@ struct IterEngine {
     return GD_OK;
   }
 
+  // Per row tile, behind the tiles: see wave_rows_kernel.
+  int32_t* wave_from() const { return reinterpret_cast<int32_t*>(tiles.as<Tile>() + n_tiles); }
+
   IterArgs iter_args() {
     const int parts = (n_tiles > 0 ? pull_grid : 0) + n_hub_tiles;
     const bool staged = n_stage_blocks > 0 && !fused;
@@ -296,7 +297,7 @@ struct IterEngine {
                     hub_part.as<float>(), err_part.as<double>(), state.as<IterState>(),
                     fused ? parts : 0, errors.as<double>(),
                     staged ? hub_soff.as<int32_t>() : nullptr, stage.as<float>(),
-                    win.on() ? win.stage.as<float>() : nullptr, wave_from.as<int32_t>()};
+                    win.on() ? win.stage.as<float>() : nullptr, wave_from()};
   }
 
   // exact hubs finish their rows in the pull launch: no hub epilogues here

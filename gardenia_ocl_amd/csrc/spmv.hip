@@ -201,6 +201,11 @@ bool long_rows_beside(const gd_spmv_plan* p) {
 // 0.49, 68 / 77, x 8 within 16,000 0.43, 42.5 / 45.5, within 64,000 0.78, 47.8 /
 // 45.3.
 int wants_windows(const gd_spmv_plan* p, bool* want) {
+  const int64_t cols = p->cols;
+  const bool large = cols > 2 << 20;
+  *want = cols > 1 << 20 && (p->sched.hub_row.empty() || long_rows_beside(p)) &&
+          window_gather_fits(p->cols, p->nnz, (int64_t)p->sched.tiles.size());
+  if (!*want) return GD_OK;
   int64_t in_tiles = 0;
   std::vector<int2> runs;
   for (const Tile& t : p->sched.tiles) {
@@ -208,11 +213,7 @@ int wants_windows(const gd_spmv_plan* p, bool* want) {
     runs.push_back(make_int2(t.z, t.w - t.z));
     in_tiles += t.w - t.z;
   }
-  const int64_t cols = p->cols;
-  const bool large = cols > 2 << 20;
-  *want = cols > 1 << 20 && in_tiles >= (large ? cols / 2 : 2 * cols) &&
-          (p->sched.hub_row.empty() || long_rows_beside(p)) &&
-          window_gather_fits(p->cols, p->nnz, (int64_t)p->sched.tiles.size());
+  *want = in_tiles >= (large ? cols / 2 : 2 * cols);
   if (!*want) return GD_OK;
   double lines = 0.0;
   const int rc = gathered_lines(runs, p->Aj, p->stream, &lines);
