@@ -779,15 +779,28 @@ def bench_adjoint(scale, spmv_log2, seed):
     return out
 
 
-def traffic_from_profile(scale):
+def pull_kernel_name(info):
+    """The kernel that takes the plan's row tiles."""
+    p = f"PrPolicy, {info['items_per_thread']}, {info['nontemporal']}, "
+    p += "true" if info["sort_tiles"] else "false"
+    if info["persistent"]:
+        return f"pull_persistent_kernel<{p}>"
+    if info["block"] != 256:
+        return f"pull_tile_kernel<{p}, {info['block']}>"
+    return f"pull_kernel<{p}, {'true' if info['staged_hubs'] else 'false'}>"
+
+
+def traffic_from_profile(scale, kernel):
     """The pull phase's counters measured with rocprofv3 (HBM bytes from
     FETCH_SIZE / WRITE_SIZE scaled by a 1 GiB copy, L2 requests and hits from
-    TCC_REQ / TCC_HIT) for this workload, or {} when none is committed."""
+    TCC_REQ / TCC_HIT) for this workload and this kernel, or {} when none is
+    committed."""
     path = os.path.join(ROOT, "profiles", f"pr_pull_rmat{scale}_traffic.json")
     if not os.path.exists(path):
         return {}
     with open(path) as f:
-        return json.load(f)
+        prof = json.load(f)
+    return prof if prof.get("kernel") == kernel else {}
 
 
 def main():
@@ -948,17 +961,15 @@ def main():
     avg_pull_ms = pull_ms / max(1, pull_n)
     bytes_iter = 4 * E + 24 * V + 4
     achieved = bytes_iter / (avg_pull_ms * 1e-3) / 1e9
-    prof = traffic_from_profile(args.scale)
+    kernel = pull_kernel_name(info)
+    prof = traffic_from_profile(args.scale, kernel)
     roof = {
         "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
         "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": prof.get("hbm_bytes_per_launch"),
         "traffic_kernels": prof.get("phase_kernels"),
         "l2_requests_per_edge": prof.get("l2_requests_per_edge"),
         "l2_hit_rate": prof.get("l2_hit_rate"),
-        "kernel": (f"{'pull_persistent_kernel' if info['persistent'] else 'pull_tile_kernel'}"
-                   f"<PrPolicy, {info['items_per_thread']}, {info['nontemporal']}, "
-                   f"{'true' if info['sort_tiles'] else 'false'}"
-                   f"{', ' + str(info['block']) if info['block'] != 256 else ''}>"),
+        "kernel": kernel,
         "avg_launch_ms": round(avg_pull_ms, 5),
         "algorithmic_bytes_per_launch": bytes_iter,
     }
