@@ -48,8 +48,8 @@ struct Tile {
 // than exact_len is instead one whole-row hub tile (summed in edge order by one
 // workgroup); the longest of them come first, the rest are spread evenly
 // among the row tiles.
-// Whole-row exact hubs of PageRank-like plans are summed by the workgroup's
-// binade scan (exact_row_sum); long rows of the SpMV / SymGS / many-graph /
+// Whole-row exact hubs of PageRank-like plans and of many graphs are summed by a
+// workgroup in parallel (exact_row_sum); long rows of the SpMV / SymGS /
 // no-allocation paths by one lane from LDS chunks of kHubChunk edges
 // (hub_chain_sum).
 constexpr int kHubChunk = 1536;    // 192 gathering lanes x 8 edges

@@ -15,8 +15,8 @@
 //
 // What bounds it: the L2 requests of the gathers.  Every graph's contrib fits
 // an XCD's L2, so a tile's edges are gathered in source order (tile_sort.h;
-// lanes share lines) and the kernel holds 94 registers and 24.6 KB of LDS:
-// 64 RMAT graphs of 2^12 to 2^18 vertices, 62 M edges, tol 1e-4: 4.00 ms; in
+// lanes share lines) and the kernel holds 96 registers and 24.7 KB of LDS:
+// 64 RMAT graphs of 2^12 to 2^18 vertices, 62 M edges, tol 1e-4: 3.75 ms; in
 // edge order and with one lane's chain for the hub rows 5.23 ms.
 
 #include <hip/hip_runtime.h>

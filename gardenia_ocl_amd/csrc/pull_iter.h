@@ -14,7 +14,7 @@
 //   struct P::Args                      kernel arguments (pointers, scalars)
 //   static constexpr bool kExactHubs    hub rows (whole-row tiles) summed in
 //                                       edge order with sequential FP32
-//                                       rounding (exact_hub_kernel), else hub
+//                                       rounding (hub_body), else hub
 //                                       segments tree-summed + finalize
 //   static constexpr bool kSeqAll       every row of a row tile summed by its
 //                                       owner thread in edge order (else rows
@@ -249,12 +249,12 @@ __global__ __launch_bounds__(kBlock) void pull_persistent_kernel(const typename 
 }
 
 // Whole-row hubs of an exact-hub policy: one workgroup per hub row adds the
-// row in edge order with the reference's sequential rounding (exact_row_sum:
-// the workgroup's binade scan, the next chunk's gathers in flight during the
-// scan), then runs the row's epilogue.  A kernel of its own, launched before
-// and beside the row-tile launch, longest row first.  Hub rows are stored in
-// edge order.  hub_body: exact hub h of the iteration (the caller checked
-// st->done).
+// row in edge order with the reference's sequential rounding (exact_row_sum,
+// the next chunk's gathers in flight during a chunk's prefix), then runs the
+// row's epilogue.  The first workgroups of the row tiles' launch (pull_kernel) or
+// a launch of their own beside it (exact_hub_kernel), longest row first.  Hub rows
+// are stored in edge order, or in sorted staging blocks (IterEngine::hubs_sorted).
+// hub_body: exact hub h of the iteration (the caller checked st->done).
 struct HubLds {
   alignas(16) float buf[kScanChunk];  // one chunk of the row
   ExactLds xs;
@@ -293,8 +293,8 @@ __device__ __forceinline__ void hub_body(const typename P::Args& a, const IterAr
 // coalesced from L2 instead of waiting on each chunk's random gathers, so a
 // long row's workgroup is bound by its scan.  Workgroup b gathers block b:
 // x = first edge, y = edges (<= kScanChunk), z = offset in stage.  PERM
-// (windowed plans): a block's edges are sorted by source; the values go back
-// to edge order through LDS.
+// (IterEngine::hubs_sorted): a block's edges are sorted by source; the values go
+// back to edge order through LDS.
 template <class P, int NT, bool PERM>
 __global__ __launch_bounds__(kBlock) void hub_stage_kernel(const typename P::Args a,
                                                            const IterArgs it,
@@ -355,7 +355,7 @@ __global__ __launch_bounds__(kBlock) void exact_hub_kernel(const typename P::Arg
 // workgroups [0, n_hub_tiles) take the exact hubs (longest first), so they
 // are placed before the tiles fill the CUs, the rest the row tiles.  The two
 // bodies share one LDS allocation, and the hub body needs fewer registers
-// than the tile's (72 and 94), so it costs the tiles nothing; two launches on
+// than the tile's (72 and 96), so it costs the tiles nothing; two launches on
 // two streams cost about 20 us of fork and join per iteration (1 M vertices:
 // 78 to 60 us).  In small iterations (it.fuse_parts > 0) the last workgroup
 // to finish closes the iteration (fused_finish): no finalize launch either.

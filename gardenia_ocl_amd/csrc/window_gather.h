@@ -13,9 +13,9 @@
 //      sorted by source, lie in one run of consecutive slots per window, so
 //      64 lanes read a few whole lines.
 // The values, and the order in which a row adds them, stay the same.  Both
-// passes are bound by HBM: 6 bytes per edge in the first (5.1 TB/s), 10 in the
-// second.  RMAT-24, per iteration: 1.36 ms with plain gathers; expand 0.32,
-// hub staging 0.11, row tiles 0.73.  The order of the tiles matters: a tile's
+// passes are bound by HBM: 6 bytes per edge in the first (5.2 TB/s), 10 in the
+// second (5.1).  RMAT-24, per iteration: 1.34 ms with plain gathers; expand 0.32,
+// hub staging 0.11, row tiles and hubs 0.56.  The order of the tiles matters: a tile's
 // run shares its first and last line with the neighbouring tiles', so with
 // neighbours on different XCDs the tiles fetched 3.3 GB instead of 2.5.
 #ifndef GD_WINDOW_GATHER_H_

@@ -50,8 +50,10 @@ class SpmvPlan:
     def __init__(self, Ap, Aj, Ax, num_cols=None, stream=None, mode="tiles"):
         """mode: "tiles" (any column order), "sliced" (sorted rows only), "auto"
         (sliced when x exceeds one XCD's L2 and rows are short and sorted).
-        All give the same results; where x exceeds one XCD's L2 it is gathered
-        through windows, in a buffer that the plan's runs share."""
+        All give the same results; where x exceeds one XCD's L2 and a tile's columns
+        are spread it is gathered through windows (``windowed``), in a buffer that
+        the plan's runs share: threads may run one plan, graphs captured from its
+        runs must not be replayed beside one another."""
         import torch
 
         for t, dt in ((Ap, torch.int32), (Aj, torch.int32), (Ax, torch.float32)):

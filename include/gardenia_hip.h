@@ -92,8 +92,8 @@ typedef struct gd_pr_plan_config {
                            workgroups per CU); 0: auto (256); the persistent grid always
                            uses 256 */
   int hub_threshold;    /* rows with more in-edges than this are whole-row hubs summed by a
-                           workgroup of their own (exact_hub_kernel), the rest by their
-                           owner thread inside a row tile; 64 .. 256*items_per_thread;
+                           workgroup of their own, the rest by their owner thread or a
+                           wavefront inside a row tile; 64 .. 256*items_per_thread;
                            0: auto (256*items_per_thread, the longest row a 256-thread
                            tile holds) */
   int stage_hubs;       /* 1: the hub rows are gathered by a kernel of their own, spread
@@ -101,8 +101,10 @@ typedef struct gd_pr_plan_config {
                            workgroups sum them (each hub workgroup is then bound by its scan
                            instead of its gathers); same results; 0: never; -1: auto (when
                            the longest hub row * 500 exceeds the edges in row tiles: the
-                           longest row's chain would outlast the row tiles).  Iterations
-                           small enough to run as one launch never stage */
+                           longest row's chain would outlast the row tiles; always in
+                           plans that gather through windows, gd_pr_plan_windowed, which 0
+                           turns off).  Iterations small enough to run as one launch never
+                           stage */
 } gd_pr_plan_config;
 
 void gd_pr_default_plan_config(gd_pr_plan_config *cfg);
@@ -110,9 +112,8 @@ void gd_pr_default_plan_config(gd_pr_plan_config *cfg);
 typedef struct gd_pr_plan_info_t {
   int64_t n_tiles;        /* workgroups per iteration: row tiles + whole-row hub tiles */
   int64_t n_hubs;         /* rows summed as hubs: longer than hub_threshold edges
-                             (whole-row tiles in the reference's summation order:
-                             one lane's chain over the first 4096 edges, the
-                             workgroup's exact scan beyond) */
+                             (whole-row tiles in the reference's summation order, a
+                             workgroup each) */
   int64_t n_hub_segments; /* tiles spent on hub rows */
   int32_t max_row_len;
   int32_t relabel;        /* 1 if the plan relabelled the vertices */
